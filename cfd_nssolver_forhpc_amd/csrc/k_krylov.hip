@@ -17,6 +17,7 @@
 // batch instead of once per dot product.  FP64 dots are kept for every
 // scalar, also when the vectors are FP32.
 #include <algorithm>
+#include <atomic>
 #include <cstdio>
 #include <mutex>
 #include <string>
@@ -24,6 +25,7 @@
 #include <cmath>
 
 #include "dev_common.h"
+#include "dev_resident.h"
 #include "dev_spmv.h"
 
 namespace cfd {
@@ -462,6 +464,79 @@ hipError_t launch_iters(Ctx &c, const OpArgs &a, const Vecs<T> &v, KrylovScalars
   return hipGetLastError();
 }
 
+// Workgroups of resident solves in flight on each device.  They hold a CU
+// each, so a solve that would not find its CUs free takes the launch path.
+constexpr int MAX_DEVICES = 64;
+std::atomic<int> g_resident[MAX_DEVICES];
+
+struct ResidentSlots {
+  std::atomic<int> *n = nullptr;
+  int blocks = 0;
+  bool take(int device, int want) {
+    if (device < 0 || device >= MAX_DEVICES) return false;
+    int cus = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) return false;
+    n = &g_resident[device];
+    if (n->fetch_add(want) + want > cus) {
+      n->fetch_sub(want);
+      return false;
+    }
+    blocks = want;
+    return true;
+  }
+  ~ResidentSlots() {
+    if (blocks) n->fetch_sub(blocks);
+  }
+};
+
+// The iterations of an FP64 solve on the ELL operator in one launch
+// (dev_resident.h) where its rows fit the chip's registers; the state after
+// init_kernel is the launch path's and so is every result, bit for bit.
+// *solved is false when the launch path has to go on from where the state is:
+// the system is too large, its matrix is no stencil, or the CUs are taken.
+// The limit is what the registers of 256 one-workgroup CUs hold (RES_MAX_N,
+// 524288 rows); it is the faster path over that whole range (at the limit
+// 23.5 us an iteration against 53.6, at one workgroup 4.5 against 26.7).
+int solve_resident(Ctx &c, const OpArgs &a, const Vecs<double> &v, KrylovScalars *ks, bool *solved) {
+  *solved = false;
+  if (a.op != CFD_OP_ELL || a.N > RES_MAX_N) return CFD_OK;
+  ResArgs r;
+  r.N = a.N;
+  r.nbx = blocks_for(a.N, 4 * 256, RED_MAX_BLOCKS);
+  r.S = (int64_t)r.nbx * 256;
+  r.nblk = (int)((r.S + RES_THREADS - 1) / RES_THREADS);
+  r.sliced = a.sliced;
+  r.col = a.col;
+  r.val = a.val;
+  r.x = v.x;
+  r.r0 = v.r0;
+  r.r1 = v.r1;
+  r.p1 = v.p1;
+  // the launch path's s and A p are its only users of these two vectors
+  r.ll0 = reinterpret_cast<uint64_t *>(v.s1);
+  r.ll1 = reinterpret_cast<uint64_t *>(v.ap);
+  static_assert(2 * RES_RED_WORDS <= 3 * RED_MAX_BLOCKS, "an exchanged sum fits its site's partials");
+  const int sites[3] = {RS_SPMV_DOT, RS_SPMV_DOT2, RS_XR};
+  for (int q = 0; q < 3; ++q) r.red[q] = reinterpret_cast<uint64_t *>(red_part_host(c, sites[q]));
+  r.ks = ks;
+  r.chunk = 4096;  // bounds one launch to some tens of milliseconds
+  ResidentSlots slots;
+  if (!slots.take(c.device, r.nblk)) return CFD_OK;
+  const int nbc = blocks_for(std::max<int64_t>(a.N, 2 * RES_RED_WORDS), 256, 1 << 30);
+  for (;;) {
+    resident_clear_kernel<<<nbc, 256, 0, c.stream>>>(r);
+    bicg_resident_kernel<<<r.nblk, RES_THREADS, 0, c.stream>>>(r);
+    CFD_HIP(hipGetLastError());
+    CFD_HIP(hipMemcpyAsync(c.hks, ks, sizeof(KrylovScalars), hipMemcpyDeviceToHost, c.stream));
+    CFD_HIP(hipStreamSynchronize(c.stream));
+    if (c.hks->pad1 == RES_STUCK) return fail(CFD_ERR_RUNTIME, "resident BiCGSTAB: a workgroup stopped answering");
+    if (c.hks->pad1 != RES_GO) return CFD_OK;
+    if (c.hks->done) break;
+  }
+  *solved = true;
+  return CFD_OK;
+}
+
 // Generic driver: set up scalars, r0 = b - A x, then batches of iterations
 // with one host read of the scalars per batch.  The batch length follows
 // the observed convergence rate so that few no-op launches follow the
@@ -476,10 +551,14 @@ int solve_bicg(Ctx &c, const OpArgs &a, const Vecs<T> &v, KrylovScalars *ks, int
                                                       red_part_host(c, RS_INIT));
   init_finalize<<<1, FIN_THREADS, 0, c.stream>>>(red_part_host(c, RS_INIT), nb, ks);
   CFD_HIP(hipGetLastError());
+  bool solved = false;
+  if constexpr (std::is_same<T, double>::value) {
+    if (int rc = solve_resident(c, a, v, ks, &solved)) return rc;
+  }
   int batch = 2;
   double prev_rel = -1.0;
   int prev_it = 0;
-  for (;;) {
+  while (!solved) {
     CFD_HIP(launch_iters<T>(c, a, v, ks, batch));
     CFD_HIP(hipMemcpyAsync(c.hks, ks, sizeof(KrylovScalars), hipMemcpyDeviceToHost, c.stream));
     CFD_HIP(hipStreamSynchronize(c.stream));
