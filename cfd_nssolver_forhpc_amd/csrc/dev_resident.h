@@ -27,9 +27,9 @@
 //
 // What bounds it is the latency of the five exchanges, about 2 us each, and,
 // past 10^5 rows, the halo words.  Measured on one MI355X, us an iteration,
-// launch path -> here: 512 rows 26.7 -> 4.5 (one workgroup: sums through
-// LDS), 4096 32.7 -> 11.6, 32768 33.1 -> 13.0, 65536 34.6 -> 16.0, 303750
-// 48.7 -> 30.0, 524288 53.6 -> 23.5.
+// launch path -> here: 512 rows 26.4 -> 4.7 (one workgroup: sums through
+// LDS), 4096 33.0 -> 10.9, 32768 33.3 -> 11.8, 65536 34.4 -> 14.4, 303750
+// 47.7 -> 22.4, 524288 53.1 -> 19.5.
 #pragma once
 
 #include "dev_common.h"
@@ -95,7 +95,11 @@ __device__ inline double ll_value(uint64_t w0, uint64_t w1) {
 }
 
 // Once every workgroup is known to be resident, each wait ends when the
-// others reach the same point, microseconds later; the bound (some seconds of
+// others reach the same point, microseconds later.  No wave polls before
+// every wave of its workgroup has issued the words others wait for (a barrier
+// stands between): the memory pipeline takes older waves first, and waves
+// that poll scattered words keep it full, so a younger wave's stores could
+// wait for ever behind polls that wait for them.  The bound (some seconds of
 // polling, counted in polls so that a preempted kernel does not run into it)
 // is there so that the kernel ends whatever happens, with RES_STUCK for the
 // host to report.
@@ -110,7 +114,7 @@ struct ResLds {
   double wsum[2][RES_ROWS][RES_THREADS / 64];
   double fin[2][FIN_THREADS / 64];
   double one[2][4][2];                     // block sums of a lone workgroup (at most 4 slots)
-  int nhalo, irregular, state, stuck;
+  int nhalo, state, stuck;
 };
 
 // Loads U pairs of words at a time until each carries the epoch: get(u) is
@@ -181,7 +185,7 @@ __device__ inline void resident_put(const ResArgs &a, ResLds &L, uint64_t *red, 
 // goes to the workgroup that holds the second, which adds its four waves to
 // it: one more hop, in every second slab of an odd nbx.  (Leaving the five
 // parts for every reader to add instead took 58 us an iteration at 303750
-// rows against 27: each workgroup reads every slot.)
+// rows against 30: each workgroup reads every slot.)
 template <int NV>
 __device__ inline void resident_put_rows(const ResArgs &a, ResLds &L, uint64_t *red, unsigned epoch) {
   const int t = threadIdx.x;
@@ -240,8 +244,8 @@ template <int NV>
 __device__ inline void resident_total(const ResArgs &a, ResLds &L, const uint64_t *red, int nslot, unsigned epoch,
                                       double (&tot)[NV]) {
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  __syncthreads();  // this workgroup's sums are left (L.one, or issued: RES_SPIN)
   if (a.nblk == 1) {
-    __syncthreads();  // the sums in L.one
     if (wid < NV) {  // at most 4 slots: the first finalize wave's lanes
       double v = 0.0;
       if (lane < nslot) v = L.one[wid][lane][0];
@@ -286,9 +290,7 @@ __device__ inline void resident_total(const ResArgs &a, ResLds &L, const uint64_
 // Every workgroup resident, or none goes on: arrivals are counted, the last
 // one sets RES_GO, and a workgroup that waits too long (other kernels hold the
 // CUs) sets RES_ABORT instead; the first of the two to be set stands for all.
-// A matrix that is no stencil aborts the same way: its halo does not fit, or is
-// scattered (a quarter of it off its wave's diagonals), where polling word by
-// word from everywhere was seen to be slower than the launches it saves.
+// A halo that does not fit (a matrix that is no stencil) aborts the same way.
 __device__ inline int resident_arrive(const ResArgs &a, ResLds &L, bool fits) {
   if (threadIdx.x == 0) {
     unsigned *const st = reinterpret_cast<unsigned *>(&a.ks->pad1);
@@ -352,7 +354,6 @@ __global__ void __launch_bounds__(RES_THREADS) bicg_resident_kernel(ResArgs a) {
   if (t == 0) {
     L.nhalo = a.nblk > 1 ? 1 : 0;  // entry 0: column N - 1, where every padding slot points
     L.hcol[0] = (int32_t)(N - 1);
-    L.irregular = 0;
     L.stuck = 0;
   }
   __syncthreads();
@@ -378,9 +379,6 @@ __global__ void __launch_bounds__(RES_THREADS) bicg_resident_kernel(ResArgs a) {
         } else if (c == N - 1) {
           at = RES_OWN;
         } else {
-          // a stencil's wave reads one diagonal per slot, the grid's edges aside
-          const int d = (int)(c - row);
-          if (d != __builtin_amdgcn_readfirstlane(d)) atomicAdd(&L.irregular, 1);
           const int e = atomicAdd(&L.nhalo, 1);
           if (e < RES_HALO) {
             L.hcol[e] = (int32_t)c;
@@ -396,8 +394,7 @@ __global__ void __launch_bounds__(RES_THREADS) bicg_resident_kernel(ResArgs a) {
     r[m] = own(m) ? *at32(a.r1, row) : 0.0;
     p[m] = own(m) ? *at32(a.p1, row) : 0.0;
   }
-  __syncthreads();
-  fits = __syncthreads_and(fits && 4 * L.irregular <= L.nhalo);
+  fits = __syncthreads_and(fits);
   if (resident_arrive(a, L, fits) != RES_GO) return;
   const int nslot = (int)((a.N + 511) / 512);
   double alpha = 0.0, omega = 0.0, beta = 0.0, pre_rho = 0.0, rnorm = 0.0, relres = 0.0;
@@ -413,6 +410,7 @@ __global__ void __launch_bounds__(RES_THREADS) bicg_resident_kernel(ResArgs a) {
       if (own(m) && a.nblk > 1) ll_store(at32(a.ll0, v + m * S), at32(a.ll1, v + m * S), p[m], 2 * epoch - 1);
       r0[m] = own(m) ? *at32(a.r0, v + m * S) : 0.0;
     }
+    __syncthreads();  // every wave has issued its words (RES_SPIN)
     resident_halo(L, a, 2 * epoch - 1);
     __syncthreads();
     resident_rows(L, val, pos, ap);
@@ -435,6 +433,7 @@ __global__ void __launch_bounds__(RES_THREADS) bicg_resident_kernel(ResArgs a) {
       L.vec[m * RES_THREADS + t] = s[m];
       if (own(m) && a.nblk > 1) ll_store(at32(a.ll0, v + m * S), at32(a.ll1, v + m * S), s[m], 2 * epoch);
     }
+    __syncthreads();
     resident_halo(L, a, 2 * epoch);
     __syncthreads();
     resident_rows(L, val, pos, as);

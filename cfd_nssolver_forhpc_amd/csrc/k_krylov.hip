@@ -15,7 +15,8 @@
 // memory; every kernel returns at once when the device-side `done` flag is
 // set, so the host launches iterations in batches and reads the flag once per
 // batch instead of once per dot product.  FP64 dots are kept for every
-// scalar, also when the vectors are FP32.
+// scalar, also when the vectors are FP32.  FP64 systems of up to half a million
+// ELL rows run their iterations in one kernel instead (dev_resident.h).
 #include <algorithm>
 #include <atomic>
 #include <cstdio>
@@ -496,7 +497,7 @@ struct ResidentSlots {
 // the system is too large, its matrix is no stencil, or the CUs are taken.
 // The limit is what the registers of 256 one-workgroup CUs hold (RES_MAX_N,
 // 524288 rows); it is the faster path over that whole range (at the limit
-// 23.5 us an iteration against 53.6, at one workgroup 4.5 against 26.7).
+// 19.5 us an iteration against 53.1, at one workgroup 4.7 against 26.4).
 int solve_resident(Ctx &c, const OpArgs &a, const Vecs<double> &v, KrylovScalars *ks, bool *solved) {
   *solved = false;
   if (a.op != CFD_OP_ELL || a.N > RES_MAX_N) return CFD_OK;

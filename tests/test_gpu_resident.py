@@ -6,8 +6,8 @@ what cfd_bicgstab(tol = 0, maxit = K) must return, bit for bit: both sum in the
 same order.  Sizes: one workgroup (N <= 2048), an odd and an even number of
 1024-row groups (their sums cross workgroups differently), a ragged end, the
 largest halo (lines longer than a workgroup's 512 rows), the largest resident
-system and the next, and a solve that takes more than one launch.  A matrix
-that is no stencil must take the launch path.
+system and the next, and a solve that takes more than one launch; random
+columns, whose halo fits the workgroup or does not (the launch path).
 """
 from __future__ import annotations
 
@@ -66,7 +66,7 @@ def test_more_iterations_than_a_launch(require_gpu):
         assert np.array_equal(sim.download(capi.X), want)
 
 
-@pytest.mark.parametrize("ncal", [(24, 25, 10), (32, 32, 16)])  # the halo of random columns would fit; would not
+@pytest.mark.parametrize("ncal", [(24, 25, 10), (32, 32, 16)])  # the halo of random columns fits; does not
 def test_matrix_that_is_no_stencil(require_gpu, ncal):
     with make_sim(ncal) as sim:
         sim.init_state()
