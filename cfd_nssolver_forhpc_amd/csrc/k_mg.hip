@@ -24,17 +24,17 @@
 // workgroup (one launch for the whole bottom of the cycle); the coarsest is
 // solved by its dense inverse or smoothed MG_COARSE_SWEEPS times.
 //
-// The finest level, two thirds of a cycle's bytes, keeps x and b
-// colour-split (ColourSplit) and has kernels of its own: colour sweeps whose
-// threads walk MG_PLANES planes and load each other-colour entry once for
-// its three uses, the post-smoothing's first sweep with the prolongation
-// folded in and its last one writing the result, and a restriction that
-// reads the children as colour pairs.  The next levels run the same kernels
-// in the same layout while the level above halves every axis and they are
-// not part of the one-workgroup bottom, up to MG_SPLIT_MAX levels
-// (split_levels).  Each does the arithmetic of the generic per-cell
-// functions term for term, so the cycle's result is the same bit for bit in
-// either layout.
+// The finest level keeps x and b colour-split (ColourSplit), and so does every
+// next level while the level above halves every axis and it is not part of
+// the one-workgroup bottom (split_levels).  Their sweeps run up to four
+// half-sweeps in one pass over the level (mg_fused_kernel), the first pass
+// after the coarse correction with the prolongation folded in, the last one
+// writing the result; the restriction reads the children as colour pairs.
+// What a pass cannot take (one sweep, the odd sweep of an odd count, lines
+// too long for its tiles) runs as single colour sweeps whose threads walk
+// MG_PLANES planes and load each other-colour entry once for its three uses.
+// Each does the arithmetic of the generic per-cell functions term for term,
+// so the cycle's result is the same bit for bit in either layout.
 //
 // Every kernel returns at once when the Krylov solver's `done` flag is set,
 // so preconditioned iterations can be launched in batches like the plain
@@ -47,19 +47,13 @@
 #include <vector>
 
 #include "dev_common.h"
+#include "pred_tiled.h"
 
 namespace cfd {
 
 constexpr int MG_MAX_LEVELS = 16;
 constexpr int64_t MG_SMALL = 4096;
 constexpr int MG_COARSE_SWEEPS = 48;
-// colour-split levels at most (the finest one and the next ones).  At
-// 512x256x64, two (512x256x64, 256x128x32) ran the multigrid steps 1-2%
-// faster than the finest alone; a third level (128x64x16) gave that back
-// and a fourth cost 2% more: the small levels' sweeps are bound by their
-// launches, and fewer threads walking planes hide less latency.
-constexpr int MG_SPLIT_MAX = 2;
-
 // per-level device view: ax = cm[nx] cp[nx] dd[nx] w[nx] (and ay, az)
 struct MGView {
   int nx, ny, nz, fx, fy, fz;
@@ -77,6 +71,9 @@ struct MGLevel {
   // by its last post-smoothing half-sweep for the prolongation above it
   double *xn64 = nullptr;
   float *xn32 = nullptr;
+  // a colour-split level's second x: mg_fused_kernel reads one and writes the other
+  double *xb64 = nullptr;
+  float *xb32 = nullptr;
 };
 
 struct MGState {
@@ -315,7 +312,7 @@ __global__ void __launch_bounds__(256) mg_rb_kernel(MGView L, int colour, const 
   rb_at<T, Lay>(L, i, j, k2, colour, b, x);
 }
 
-// planes of the colour-split finest level that one thread of a sweep walks:
+// planes of a colour-split level that one thread of a single sweep walks:
 // at 4 the FP64 sweeps hold 72-112 VGPRs (4-7 waves a SIMD; 8 planes: 112-182,
 // 2-4 waves), and the 512x256x64 multigrid steps ran 1-1.5% faster than at 8
 // (2 planes: 5% slower)
@@ -426,6 +423,271 @@ __global__ void __launch_bounds__(256) mg_split_sweep_kernel(MGView L, MGView C,
       out[idx3(L, i, j, k)] = (V)v;
     else
       own[i * sx + col] = v;
+  }
+}
+
+// ---- several half-sweeps of a colour-split level in one pass ---------------
+//
+// A half-sweep alone streams 12 B a cell (FP64) and, on the small levels, is
+// a launch of 3-6 us whatever its size.  mg_fused_kernel runs NS of them in
+// one pass: a workgroup owns a tile of rows (all of z) and a run of planes,
+// marches along i, and at step t applies half-sweep 1 to plane t, half-sweep
+// 2 to plane t - 1, ... NS to plane t - NS + 1.  Thread (row, k2) holds the
+// column's entries of both colours; its x- and same-k2 neighbours are its
+// own registers, the other three come from LDS, where every stage leaves its
+// half-plane for the next step (two buffers, one barrier a step).  Tiles
+// overlap by NS rows and planes: the overlap is computed twice instead of
+// exchanged, so x is read from one buffer and written to another.  Loads run
+// two (FP64: registers) or three planes ahead; the loop is unrolled by the length of the register
+// rings, so their positions are fixed.  The arithmetic is rb_at's, term for
+// term (an absent neighbour's coefficient is 0).
+//
+// What bounds a pass is latency on the small levels (8-14 us for 4
+// half-sweeps, 4 launches of 3.5-6 us before) and, on the finest, the stages'
+// chain of LDS reads and divisions: four half-sweeps of 512x256x64 take
+// 41-51 us FP64 and 28 us FP32 (4 x 21 and 4 x 15 as single sweeps), at 30 B
+// a cell 6.1 TB/s of FP64 traffic.  With a branch per stage the compiler
+// drained every load before its use and an FP64 pass took 59-68 us.  One
+// workgroup a CU: tiles of 24 rows and 23 planes at that size, each computing
+// 1.5 times its cells, are what 256 CUs leave.  Three timesteps
+// there went from 73.9 to 57.2 ms (FP64; mixed 65.5 to 50.8), the 256x128x32
+// adjoint from 110 to 83 ms.
+constexpr int FUSED_THREADS = 1024;
+constexpr int FUSED_RING = 6;     // planes of x and b a thread holds
+constexpr int FUSED_CHUNK = 512;  // planes of a run at most (its coefficients sit in LDS)
+
+struct FusedShape {
+  int hz, R, TJ, njt, chunk, nci, halo;  // halo: rows beside a tile (0: one tile spans y)
+};
+
+// n / d as the compiler's division does it, split so that the reciprocal of
+// d is shared by the two divisions a cell of a pass makes: the same
+// operations on the same operands while neither needs rescaling (quotients
+// and divisors far from the exponent range's ends)
+__device__ inline double div_recip(double d) {
+  double y = __builtin_amdgcn_rcp(d);
+  double e = fma(-d, y, 1.0);
+  y = fma(y, e, y);
+  e = fma(-d, y, 1.0);
+  return fma(y, e, y);
+}
+__device__ inline double div_by(double n, double d, double y) {
+  const double q = n * y;
+  const double r = fma(-d, q, n);
+  return __builtin_amdgcn_div_fixup(fma(r, y, q), d, n);
+}
+__device__ inline float div_recip(float d) {
+  const float y = __builtin_amdgcn_rcpf(d);
+  const float e = fmaf(-d, y, 1.0f);
+  return fmaf(e, y, y);
+}
+__device__ inline float div_by(float n, float d, float y) {
+  const float q = n * y;
+  const float r = fmaf(-d, q, n);
+  const float q1 = fmaf(r, y, q);
+  const float r1 = fmaf(-d, q1, n);
+  return __builtin_amdgcn_div_fixupf(fmaf(r1, y, q1), d, n);
+}
+
+// the column a thread of mg_fused_kernel owns and what it carries
+template <typename T, int NS>
+struct FusedCol {
+  T in[FUSED_RING], bA[FUSED_RING], bB[FUSED_RING];  // other colour before the pass; right-hand sides
+  T st[NS][3];                                       // stage results of the last three planes
+  T yA[3], yB[3], dA[3], dB[3];                      // 1 / diagonal and diagonal of both colours
+  T cym, cyp, czm[2], czp[2];
+  double dy, dz[2];
+  int side[2];  // LDS position of the k neighbour beside k2, by plane parity
+  bool up[2];   // that neighbour is the +z one
+};
+
+template <typename T>
+struct alignas(2 * sizeof(T)) CoefX {
+  T m, p;  // to the -x and +x neighbour
+};
+
+template <typename T, typename V, int NS, int START, bool PRO, bool OUT>
+__global__ void __launch_bounds__(FUSED_THREADS) mg_fused_kernel(MGView L, MGView C, FusedShape S,
+                                                                 const T *__restrict__ b, const T *__restrict__ xin,
+                                                                 T *__restrict__ xout, const T *__restrict__ xc,
+                                                                 V *__restrict__ out, const KrylovScalars *ks) {
+  if (ks && ks->done) return;
+  constexpr int PD = sizeof(T) == 8 ? 2 : 3;
+  constexpr bool KEEP_D = sizeof(T) == 4;  // FP64 adds the diagonal again instead of holding it
+  __shared__ T half[2][NS][FUSED_THREADS];
+  __shared__ CoefX<T> cxl[FUSED_CHUNK + 2 * NS];
+  __shared__ double dxl[FUSED_CHUNK + 2 * NS];
+  const int tid = threadIdx.x, hz = S.hz;
+  const int blk = pt_xcd_order((int)blockIdx.x, S.njt * S.nci);
+  const int jt = blk % S.njt, ci = blk / S.njt;
+  const int row = tid / hz, k2 = tid - row * hz;
+  const int j = jt * S.TJ - S.halo + row;
+  const int jc = min(max(j, 0), L.ny - 1);
+  const bool store = row < S.R && j >= jt * S.TJ && j < min((jt + 1) * S.TJ, L.ny);
+  const int i0 = ci * S.chunk, i1 = min(i0 + S.chunk, L.nx);
+  const int ta = max(i0 - (NS - 1), 0), te = i1 - 1 + (NS - 1);
+  const int64_t ns = (int64_t)L.nx * L.ny * hz;
+  const int sx = L.ny * hz, at = jc * hz + k2;
+  const T *__restrict__ xo = xin + (START ? 0 : ns);  // the colour the first half-sweep reads
+  const T *__restrict__ bA = b + (START ? ns : 0), *__restrict__ bB = b + (START ? 0 : ns);
+  // a plane's base is uniform, a thread's place in it 32 bits
+  const unsigned atb = (unsigned)at * (unsigned)sizeof(T);
+  auto in_plane = [&](const T *p, int plane) {
+    return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(p + (int64_t)plane * sx) + atb);
+  };
+  // per-plane coefficients ta .. min(te, nx - 1)
+  const int npl = min(te, L.nx - 1) - ta + 1;
+  for (int q = tid; q < npl; q += (int)blockDim.x) {
+    cxl[q] = CoefX<T>{(T)L.ax[ta + q], (T)L.ax[L.nx + ta + q]};
+    dxl[q] = L.ax[2 * L.nx + ta + q];
+  }
+  FusedCol<T, NS> c;
+  c.cym = (T)L.ay[jc];
+  c.cyp = (T)L.ay[L.ny + jc];
+  c.dy = L.ay[2 * L.ny + jc];
+  // the START colour at plane ta + n has k = 2 k2 + e, e = (ta + n + j + START) & 1;
+  // index q of the parity arrays: n & 1 for that colour, the other for the other
+  bool pad[2];  // k is past an odd nz (never read: the entry is 0 and its result unused)
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const int e = (ta + q + jc + START) & 1;
+    const int k = min(2 * k2 + e, L.nz - 1);
+    pad[q] = 2 * k2 + e >= L.nz;
+    c.czm[q] = (T)L.az[k];
+    c.czp[q] = (T)L.az[L.nz + k];
+    c.dz[q] = L.az[2 * L.nz + k];
+    c.up[q] = e;
+    const int ks2 = e ? (k2 + 1 < hz ? k2 + 1 : (L.wz ? 0 : k2)) : (k2 > 0 ? k2 - 1 : (L.wz ? hz - 1 : k2));
+    c.side[q] = tid + (ks2 - k2);
+  }
+  if (row >= S.R) c.side[0] = c.side[1] = tid;
+  const int im = row > 0 ? tid - hz : tid, ip = row + 1 < S.R ? tid + hz : tid;
+  auto load_in = [&](int plane, int q) -> T {  // q: parity index of the other colour at that plane
+    plane = min(max(plane, 0), L.nx - 1);
+    T v = in_plane(xo, plane);
+    if (PRO) {
+      const int k = min(2 * k2 + (c.up[q] ? 1 : 0), L.nz - 1);
+      const unsigned pb = (unsigned)((L.fy == 2 ? jc >> 1 : jc) * C.nz + (L.fz == 2 ? k >> 1 : k)) * (unsigned)sizeof(T);
+      const T *pl = xc + (int64_t)(L.fx == 2 ? plane >> 1 : plane) * C.ny * C.nz;
+      v += *reinterpret_cast<const T *>(reinterpret_cast<const char *>(pl) + pb);
+    }
+    return pad[q] ? (T)0 : v;
+  };
+  auto load_b = [&](const T *__restrict__ p, int plane, int q) -> T {
+    const T v = in_plane(p, min(max(plane, 0), L.nx - 1));
+    return pad[q] ? (T)0 : v;
+  };
+  // ring positions: plane ta + m of x at (m + 1) mod 6, of b at m mod 6
+#pragma unroll
+  for (int m = -1; m <= PD; ++m) c.in[m + 1] = load_in(ta + m, (m + 1) & 1);
+#pragma unroll
+  for (int m = 0; m < PD; ++m) c.bA[m] = load_b(bA, ta + m, m & 1);
+#pragma unroll
+  for (int m = 0; m < PD - 1; ++m) c.bB[m] = load_b(bB, ta + m, (m + 1) & 1);
+#pragma unroll
+  for (int m = PD; m < FUSED_RING; ++m) {
+    if (m > PD + 1) c.in[m] = (T)0;
+    c.bA[m] = c.bB[m] = (T)0;
+  }
+  c.bB[PD - 1] = (T)0;
+#pragma unroll
+  for (int q = 0; q < 3; ++q) {
+    c.yA[q] = c.yB[q] = c.dA[q] = c.dB[q] = (T)1;
+#pragma unroll
+    for (int s = 0; s < NS; ++s) c.st[s][q] = (T)0;
+  }
+  half[1][0][tid] = c.in[1];  // plane ta, as if left by the step before the first
+#pragma unroll
+  for (int s = 1; s < NS; ++s) half[1][s][tid] = (T)0;  // planes before ta: read, never needed
+  __syncthreads();
+
+  // A step has no branches: every stage runs, on planes it need not do as
+  // well (they feed only such planes, and values finite but unused: a
+  // coefficient across the grid's end is 0), and every load is issued with
+  // its plane clamped, so that the waits count loads instead of draining
+  // them and the stages' LDS reads overlap.
+  const int ilast = npl - 1;
+  const unsigned outb = (unsigned)(jc * L.nz + 2 * k2) * (unsigned)sizeof(V);
+  auto step = [&](auto uc, int n) {
+    constexpr int u = decltype(uc)::value;  // n mod 6
+    constexpr int q = u & 1;                // parity index of every stage's colour at its plane
+    const T(*prev)[FUSED_THREADS] = half[(u + 1) & 1];
+    T(*cur)[FUSED_THREADS] = half[u & 1];
+    // loads of the planes PD ahead of their first use
+    c.in[(u + 2 + PD) % 6] = load_in(min(ta + n + 1 + PD, te + 1), (u + PD) & 1);
+    c.bA[(u + PD) % 6] = load_b(bA, min(ta + n + PD, te), (u + PD) & 1);
+    c.bB[(u + PD - 1) % 6] = load_b(bB, min(ta + n + PD - 1, te), (u + PD) & 1);
+    // a stage's LDS reads are issued before the stage ahead of it is computed,
+    // and not earlier (all at once they take registers that FP64 lacks)
+    T vym[NS], vyp[NS], vs[NS];
+    CoefX<T> cx[NS];
+    auto fetch = [&](int s) {  // stage s works on plane ta + n - s
+      vym[s] = prev[s][im];
+      vyp[s] = prev[s][ip];
+      vs[s] = prev[s][c.side[q]];
+      cx[s] = cxl[min(max(n - s, 0), ilast)];
+    };
+    fetch(0);
+    const double dx0 = dxl[min(n, ilast)], dx1 = dxl[min(max(n - 1, 0), ilast)];
+    double dx2 = 0.0, dx3 = 0.0;
+    if (!KEEP_D) {
+      dx2 = dxl[min(max(n - 2, 0), ilast)];
+      if (NS > 3) dx3 = dxl[min(max(n - 3, 0), ilast)];
+    }
+    c.dA[u % 3] = (T)(dx0 + c.dy + c.dz[q]);
+    c.yA[u % 3] = div_recip(c.dA[u % 3]);
+    c.dB[(u + 2) % 3] = (T)(dx1 + c.dy + c.dz[q]);
+    c.yB[(u + 2) % 3] = div_recip(c.dB[(u + 2) % 3]);
+#pragma unroll
+    for (int s = 0; s < NS; ++s) {
+      if (s + 1 < NS) fetch(s + 1 < NS ? s + 1 : 0);
+      if (sizeof(T) == 8) __builtin_amdgcn_sched_barrier(0);
+      // ring positions mod 3 of the planes ta + n - s - 1, ta + n - s, ta + n - s + 1
+      const int r0 = (u + 6 - s) % 3, rm = (u + 5 - s) % 3, rp = (u + 7 - s) % 3;
+      const T xm = s == 0 ? c.in[u % 6] : c.st[s > 0 ? s - 1 : 0][rm];
+      const T x0 = s == 0 ? c.in[(u + 1) % 6] : c.st[s > 0 ? s - 1 : 0][r0];
+      const T xp = s == 0 ? c.in[(u + 2) % 6] : c.st[s > 0 ? s - 1 : 0][rp];
+      const T bv = (s & 1) ? c.bB[(u + 6 - s) % 6] : c.bA[(u + 6 - s) % 6];
+      const T d = KEEP_D ? ((s & 1) ? c.dB[r0] : c.dA[r0])
+                         : (T)((s == 0 ? dx0 : s == 1 ? dx1 : s == 2 ? dx2 : dx3) + c.dy + c.dz[q]);
+      const T y = (s & 1) ? c.yB[r0] : c.yA[r0];
+      T v = fma(cx[s].m, xm, (T)0);
+      v = fma(cx[s].p, xp, v);
+      v = fma(c.cym, vym[s], v);
+      v = fma(c.cyp, vyp[s], v);
+      const T v1 = c.up[q] ? x0 : vs[s], v2 = c.up[q] ? vs[s] : x0;  // -z, +z
+      v = fma(c.czm[q], v1, v);
+      v = fma(c.czp[q], v2, v);
+      c.st[s][r0] = div_by(bv + v, d, y);
+      if (s + 1 < NS) cur[s + 1 < NS ? s + 1 : 0][tid] = c.st[s][r0];
+    }
+    cur[0][tid] = c.in[(u + 2) % 6];
+    // the pass's result of plane ta + n - NS + 1: the last half-sweep's colour and the other
+    const int p = ta + n - (NS - 1);
+    if (p >= i0 && p < i1 && store) {
+      constexpr int rf = (u + 6 - (NS - 1)) % 3;
+      const T last = c.st[NS - 1][rf], other = c.st[NS - 2][rf];
+      if (OUT) {
+        char *o = reinterpret_cast<char *>(out + (int64_t)p * L.ny * L.nz) + outb;
+        reinterpret_cast<V *>(o)[0] = (V)(c.up[q] ? other : last);
+        if (2 * k2 + 1 < L.nz) reinterpret_cast<V *>(o)[1] = (V)(c.up[q] ? last : other);
+      } else {
+        constexpr int lastc = (NS & 1) ? START : 1 - START;
+        char *o = reinterpret_cast<char *>(xout + (int64_t)p * sx);
+        *reinterpret_cast<T *>(o + (lastc ? ns * (int64_t)sizeof(T) : 0) + atb) = last;
+        *reinterpret_cast<T *>(o + (lastc ? 0 : ns * (int64_t)sizeof(T)) + atb) = other;
+      }
+    }
+    __syncthreads();
+  };
+  const int nst = te - ta + 1;
+  for (int n = 0; n < nst; n += 6) {
+    step(std::integral_constant<int, 0>{}, n);
+    if (n + 1 < nst) step(std::integral_constant<int, 1>{}, n + 1);
+    if (n + 2 < nst) step(std::integral_constant<int, 2>{}, n + 2);
+    if (n + 3 < nst) step(std::integral_constant<int, 3>{}, n + 3);
+    if (n + 4 < nst) step(std::integral_constant<int, 4>{}, n + 4);
+    if (n + 5 < nst) step(std::integral_constant<int, 5>{}, n + 5);
   }
 }
 
@@ -706,6 +968,40 @@ Shape3 shape3(int nk, int ny, int nx) {
   return s;
 }
 
+// tiles of mg_fused_kernel on a level; R = 0 where a line is too long for a
+// workgroup to hold rows beside each other (nz > 128)
+FusedShape fused_shape(const MGView &v, int ns) {
+  FusedShape s{};
+  s.hz = (v.nz + 1) / 2;
+  const int rmax = FUSED_THREADS / s.hz;
+  if (rmax < 4 * ns) return s;
+  if (v.ny <= rmax) {
+    s.R = s.TJ = v.ny;
+    s.njt = 1;
+    s.halo = 0;
+  } else {
+    s.halo = ns;
+    const int tj = rmax - 2 * ns;
+    s.njt = (v.ny + tj - 1) / tj;
+    s.TJ = (v.ny + s.njt - 1) / s.njt;
+    s.R = s.TJ + 2 * ns;
+  }
+  // one workgroup a CU: as many runs of planes as keep the tiles within 256
+  const int runs = std::max(1, 256 / s.njt);
+  s.chunk = std::min((v.nx + runs - 1) / runs, FUSED_CHUNK);
+  s.nci = (v.nx + s.chunk - 1) / s.chunk;
+  return s;
+}
+
+template <typename T, typename V, int NS, int START, bool PRO, bool OUT>
+void launch_fused(const MGView &v, const MGView &C, const T *b, const T *xin, T *xout, const T *xc, V *out,
+                  const KrylovScalars *ks, hipStream_t st) {
+  const FusedShape s = fused_shape(v, NS);
+  const int threads = (s.R * s.hz + 63) / 64 * 64;
+  mg_fused_kernel<T, V, NS, START, PRO, OUT>
+      <<<s.njt * s.nci, threads, 0, st>>>(v, C, s, b, xin, xout, xc, out, ks);
+}
+
 int nblk(int64_t n) { return blocks_for(n, 256, 1 << 30); }
 
 template <typename T>
@@ -720,6 +1016,12 @@ template <>
 double *lxn<double>(MGLevel &L) { return L.xn64; }
 template <>
 float *lxn<float>(MGLevel &L) { return L.xn32; }
+template <typename T>
+T *lxb(MGLevel &L);
+template <>
+double *lxb<double>(MGLevel &L) { return L.xb64; }
+template <>
+float *lxb<float>(MGLevel &L) { return L.xb32; }
 template <typename T>
 T *lb(MGLevel &L);
 template <>
@@ -775,35 +1077,87 @@ int mg_apply(Ctx &c, const V *r, V *out, const KrylovScalars *ks) {
     LevelOps<T, Natural>::scale_from(M.lv[0].v, r, c.f[CFD_JP], b0, x0, ks, c.stream);
   // nu sweeps of level l: pre-smoothing skips the red half-sweep its
   // right-hand side's producer did; post-smoothing folds the prolongation
-  // into its first red half-sweep, and on the finest level ends in the
-  // half-sweep that writes out
+  // into its first red half-sweep, and on a colour-split level ends in the
+  // half-sweep that writes out (or the level's natural copy)
+  T *xs[MG_MAX_LEVELS] = {};  // the buffer that holds a colour-split level's x
+  for (int l = 0; l < M.split_levels; ++l) xs[l] = X(l);
+  auto correction = [&](int l) { return l + 1 < M.split_levels ? lxn<T>(M.lv[l + 1]) : X(l + 1); };
+  auto single = [&](int l, int colour, int mode) {
+    const MGView &v = M.lv[l].v, &C = M.lv[l + 1].v;
+    Shape3 sh = shape3((v.nz + 1) / 2, v.ny, v.nx);
+    sh.grid.z = (v.nx + MG_PLANES - 1) / MG_PLANES;
+    T *bl = l == 0 ? b0 : lb<T>(M.lv[l]);
+    if (mode == SWEEP_PROLONG)
+      mg_split_sweep_kernel<T, T, SWEEP_PROLONG><<<sh.grid, sh.block, 0, c.stream>>>(v, C, 0, bl, xs[l], correction(l),
+                                                                                    nullptr, ks);
+    else if (mode == SWEEP_OUT && l > 0)  // the natural copy the level above reads
+      mg_split_sweep_kernel<T, T, SWEEP_OUT><<<sh.grid, sh.block, 0, c.stream>>>(v, C, 1, bl, xs[l], nullptr,
+                                                                                lxn<T>(M.lv[l]), ks);
+    else if (mode == SWEEP_OUT)
+      mg_split_sweep_kernel<T, V, SWEEP_OUT><<<sh.grid, sh.block, 0, c.stream>>>(v, C, 1, bl, xs[l], nullptr, out, ks);
+    else
+      mg_split_sweep_kernel<T, T, SWEEP_PLAIN><<<sh.grid, sh.block, 0, c.stream>>>(v, C, colour, bl, xs[l], nullptr,
+                                                                                  nullptr, ks);
+  };
+  // passes of up to four half-sweeps (mg_fused_kernel); what is left over
+  // (one before, two after for an odd nu) runs as single half-sweeps
+  auto smooth_fused = [&](int l, bool pre) {
+    const MGView &v = M.lv[l].v, &C = M.lv[l + 1].v;
+    const T *bl = l == 0 ? b0 : lb<T>(M.lv[l]);
+    T *other = xs[l] == X(l) ? lxb<T>(M.lv[l]) : X(l);
+    auto swap = [&] { std::swap(xs[l], other); };
+    T *const none = nullptr;
+    if (pre) {
+      int left = 2 * M.nu - 1;  // black first
+      for (; left >= 4; left -= 4) {
+        launch_fused<T, T, 4, 1, false, false>(v, C, bl, xs[l], other, none, none, ks, c.stream);
+        swap();
+      }
+      if (left == 3) {
+        launch_fused<T, T, 3, 1, false, false>(v, C, bl, xs[l], other, none, none, ks, c.stream);
+        swap();
+      } else if (left == 1) {
+        single(l, 1, SWEEP_PLAIN);
+      }
+      return;
+    }
+    const T *xc = correction(l);
+    int left = 2 * M.nu - 4;
+    if (left == 0) {  // nu = 2: prolongation to result in one pass
+      if (l > 0)
+        launch_fused<T, T, 4, 0, true, true>(v, C, bl, xs[l], other, xc, lxn<T>(M.lv[l]), ks, c.stream);
+      else
+        launch_fused<T, V, 4, 0, true, true>(v, C, bl, xs[l], other, xc, out, ks, c.stream);
+      return;
+    }
+    launch_fused<T, T, 4, 0, true, false>(v, C, bl, xs[l], other, xc, none, ks, c.stream);
+    swap();
+    for (; left > 4; left -= 4) {
+      launch_fused<T, T, 4, 0, false, false>(v, C, bl, xs[l], other, none, none, ks, c.stream);
+      swap();
+    }
+    if (left == 4) {
+      if (l > 0)
+        launch_fused<T, T, 4, 0, false, true>(v, C, bl, xs[l], other, none, lxn<T>(M.lv[l]), ks, c.stream);
+      else
+        launch_fused<T, V, 4, 0, false, true>(v, C, bl, xs[l], other, none, out, ks, c.stream);
+    } else {
+      single(l, 0, SWEEP_PLAIN);
+      single(l, 1, SWEEP_OUT);
+    }
+  };
   auto smooth = [&](int l, bool pre) {
     const MGView &v = M.lv[l].v;
+    if (l < M.split_levels && M.nu >= 2 && fused_shape(v, 4).R > 0) {
+      smooth_fused(l, pre);
+      return;
+    }
     for (int s = 0; s < M.nu; ++s)
       for (int colour = 0; colour < 2; ++colour) {
         const bool first = s == 0 && colour == 0, last = s == M.nu - 1 && colour == 1;
         if (first && pre) continue;
         if (l < M.split_levels) {
-          Shape3 sh = shape3((v.nz + 1) / 2, v.ny, v.nx);
-          sh.grid.z = (v.nx + MG_PLANES - 1) / MG_PLANES;
-          const MGView &C = M.lv[l + 1].v;
-          T *bl = l == 0 ? b0 : lb<T>(M.lv[l]), *xl = X(l);
-          if (first && l + 1 < M.split_levels)  // the correction from a split level's natural copy
-            mg_split_sweep_kernel<T, T, SWEEP_PROLONG><<<sh.grid, sh.block, 0, c.stream>>>(v, C, 0, bl, xl,
-                                                                                          lxn<T>(M.lv[l + 1]),
-                                                                                          nullptr, ks);
-          else if (last && !pre && l > 0)  // a split level's last half-sweep writes its natural copy
-            mg_split_sweep_kernel<T, T, SWEEP_OUT><<<sh.grid, sh.block, 0, c.stream>>>(v, C, 1, bl, xl, nullptr,
-                                                                                      lxn<T>(M.lv[l]), ks);
-          else if (first)
-            mg_split_sweep_kernel<T, T, SWEEP_PROLONG><<<sh.grid, sh.block, 0, c.stream>>>(v, C, 0, bl, xl, X(l + 1),
-                                                                                          nullptr, ks);
-          else if (last && !pre && l == 0)
-            mg_split_sweep_kernel<T, V, SWEEP_OUT><<<sh.grid, sh.block, 0, c.stream>>>(v, C, 1, bl, xl, nullptr, out,
-                                                                                      ks);
-          else
-            mg_split_sweep_kernel<T, T, SWEEP_PLAIN><<<sh.grid, sh.block, 0, c.stream>>>(v, C, colour, bl, xl,
-                                                                                        nullptr, nullptr, ks);
+          single(l, colour, first ? SWEEP_PROLONG : last && !pre ? SWEEP_OUT : SWEEP_PLAIN);
         } else {
           using Ops = LevelOps<T, Natural>;
           if (first)
@@ -823,12 +1177,12 @@ int mg_apply(Ctx &c, const V *r, V *out, const KrylovScalars *ks) {
       const Shape3 sh = shape3(C.nz, C.ny, C.nx);
       if (l + 1 < M.split_levels)  // the coarse right-hand side in its colour-split layout
         mg_restrict_split_kernel<T, ColourSplit><<<sh.grid, sh.block, 0, c.stream>>>(
-            F, C, bf, X(l), lb<T>(M.lv[l + 1]), X(l + 1), ks);
+            F, C, bf, xs[l], lb<T>(M.lv[l + 1]), X(l + 1), ks);
       else
-        mg_restrict_split_kernel<T><<<sh.grid, sh.block, 0, c.stream>>>(F, C, bf, X(l), lb<T>(M.lv[l + 1]),
+        mg_restrict_split_kernel<T><<<sh.grid, sh.block, 0, c.stream>>>(F, C, bf, xs[l], lb<T>(M.lv[l + 1]),
                                                                         X(l + 1), ks);
     } else if (fsplit)  // a colour-split level into a natural one, cell by cell
-      LevelOps<T, ColourSplit>::restrict_to(F, M.lv[l + 1].v, bf, X(l), lb<T>(M.lv[l + 1]), X(l + 1), ks, c.stream);
+      LevelOps<T, ColourSplit>::restrict_to(F, M.lv[l + 1].v, bf, xs[l], lb<T>(M.lv[l + 1]), X(l + 1), ks, c.stream);
     else
       LevelOps<T, Natural>::restrict_to(M.lv[l].v, M.lv[l + 1].v, lb<T>(M.lv[l]), X(l), lb<T>(M.lv[l + 1]),
                                         X(l + 1), ks, c.stream);
@@ -886,6 +1240,8 @@ void mg_release(Ctx &c) {
     mg_free(L.b32);
     mg_free(L.xn64);
     mg_free(L.xn32);
+    mg_free(L.xb64);
+    mg_free(L.xb32);
   }
   mg_free(c.mg->cinv64);
   mg_free(c.mg->cinv32);
@@ -970,7 +1326,7 @@ int mg_ensure(Ctx &c, bool fp32) {
     // next one is too while the level above halves every axis (its split
     // restriction then writes the coarse right-hand side in that layout)
     M->split_levels = M->small_from > 0 ? 1 : 0;
-    while (M->split_levels < M->small_from && M->split_levels < MG_SPLIT_MAX) {
+    while (M->split_levels < M->small_from) {
       const MGView &P = M->lv[M->split_levels - 1].v;
       if (!(P.fx == 2 && P.fy == 2 && P.fz == 2)) break;
       M->split_levels++;
@@ -1053,10 +1409,12 @@ int mg_ensure(Ctx &c, bool fp32) {
       if (!L.b32 && (rc = mg_alloc(&L.b32, n))) return rc;
       if (!L.x32 && (rc = mg_alloc(&L.x32, n))) return rc;
       if (nat && !L.xn32 && (rc = mg_alloc(&L.xn32, (size_t)L.v.n))) return rc;
+      if (sp && !L.xb32 && (rc = mg_alloc(&L.xb32, n))) return rc;
     } else {
       if (!L.b64 && (rc = mg_alloc(&L.b64, n))) return rc;
       if (!L.x64 && (rc = mg_alloc(&L.x64, n))) return rc;
       if (nat && !L.xn64 && (rc = mg_alloc(&L.xn64, (size_t)L.v.n))) return rc;
+      if (sp && !L.xb64 && (rc = mg_alloc(&L.xb64, n))) return rc;
     }
   }
   const size_t N = (size_t)c.g.N;

@@ -1,0 +1,195 @@
+"""The multigrid V-cycle's kernels against a numpy restatement.
+
+Two iterations of the V-cycle-preconditioned BiCGSTAB from x = 0 (four cycles)
+are compared with the same two iterations in numpy, whose cycle is written
+with whole-array red-black sweeps: levels, coefficients, volume-weighted
+restriction, piecewise-constant prolongation, the coarsest level's exact solve
+or 48 sweeps.  Grids: tiles of the fused half-sweeps that end inside, at and
+past a workgroup's rows, lines longer than a tile holds, odd and unhalved
+axes, periodic z, stretched axes, a hierarchy that is all bottom kernel, and a
+bottom without a dense solve.
+
+Tolerance: a cycle is a few hundred roundings deep and the problem is scaled
+to O(1), so FP64 agrees to ~1e-12 and the FP32 cycle to ~1e-4 of the solution;
+a wrong coefficient, neighbour or tile edge shows at 1e-2 or more.
+"""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from cfd_nssolver_forhpc_amd import capi, configs
+from cfd_nssolver_forhpc_amd.capi import GridArrays
+from cfd_nssolver_forhpc_amd.solver import Simulation, axis_tanh, axis_uniform, uniform_grid
+
+pytestmark = pytest.mark.gpu
+
+
+class Level:
+    def __init__(self, w, lo, hi, dir_lo, dir_hi, pz):
+        self.shape = tuple(len(q) for q in w)
+        self.wz = pz
+        self.cm, self.cp, self.dd = [], [], []
+        for a in range(3):
+            per = a == 2 and pz
+            xm, xp = 1.0 / w[a] / lo[a], 1.0 / w[a] / hi[a]
+            cm, cp = xm.copy(), xp.copy()
+            dm, dp = xm.copy(), xp.copy()
+            if not per:
+                cm[0] = cp[-1] = 0.0
+                if not dir_lo[a]:
+                    dm[0] = 0.0
+                if not dir_hi[a]:
+                    dp[-1] = 0.0
+            self.cm.append(self.along(cm, a))
+            self.cp.append(self.along(cp, a))
+            self.dd.append(self.along(dm + dp, a))
+        self.diag = self.dd[0] + self.dd[1] + self.dd[2]
+        self.vol = self.along(w[0], 0) * self.along(w[1], 1) * self.along(w[2], 2)
+        i, j, k = np.indices(self.shape)
+        self.mask = [((i + j + k) & 1) == c for c in (0, 1)]
+
+    @staticmethod
+    def along(v, a):
+        s = [1, 1, 1]
+        s[a] = -1
+        return np.asarray(v).reshape(s)
+
+    def off(self, x):
+        s = np.zeros_like(x)
+        for a in range(3):
+            s = s + self.cm[a].astype(x.dtype) * np.roll(x, 1, a) + self.cp[a].astype(x.dtype) * np.roll(x, -1, a)
+        return s
+
+    def sweep(self, x, b):
+        for c in (0, 1):
+            x = np.where(self.mask[c], (b + self.off(x)) / self.diag.astype(x.dtype), x)
+        return x
+
+
+def hierarchy(grid, p):
+    pz = bool(p.periodic_z)
+    sl = [slice(2, n + 2) for n in grid.ncal]
+    D, Ds = (grid.Dx, grid.Dy, grid.Dz), (grid.Dxs, grid.Dys, grid.Dzs)
+    w = [D[a][sl[a]].copy() for a in range(3)]
+    lo = [Ds[a][1:grid.ncal[a] + 1].copy() for a in range(3)]
+    hi = [Ds[a][sl[a]].copy() for a in range(3)]
+    dl = [bool(p.p_dirichlet[0]), bool(p.p_dirichlet[2]), not pz and bool(p.p_dirichlet[4])]
+    dh = [bool(p.p_dirichlet[1]), bool(p.p_dirichlet[3]), not pz and bool(p.p_dirichlet[5])]
+    levels, factors = [], []
+    while True:
+        L = Level(w, lo, hi, dl, dh, pz)
+        levels.append(L)
+        f = [2 if len(q) % 2 == 0 and len(q) >= 4 else 1 for q in w]
+        if pz and (len(w[2]) // 2) % 2 != 0:
+            f[2] = 1
+        if max(f) == 1 or np.prod(L.shape) <= 64:
+            break
+        factors.append(f)
+        for a in range(3):
+            if f[a] == 1:
+                continue
+            wc = w[a][0::2] + w[a][1::2]
+            mid = 0.5 * (wc[:-1] + wc[1:])
+            seam = 0.5 * (wc[-1] + wc[0])
+            first, last = (seam, seam) if a == 2 and pz else (wc[0], wc[-1])
+            w[a], lo[a], hi[a] = wc, np.concatenate([[first], mid]), np.concatenate([mid, [last]])
+    return levels, factors, any(dl + dh)
+
+
+def coarsest(L, b, exact):
+    if not exact:
+        x = np.zeros_like(b)
+        for _ in range(48):
+            x = L.sweep(x, b)
+        return x
+    n = b.size
+    A = np.empty((n, n))
+    for c in range(n):
+        e = np.zeros(n)
+        e[c] = 1.0
+        e = e.reshape(L.shape)
+        A[:, c] = (L.diag * e - L.off(e)).ravel()
+    return np.linalg.solve(A, b.ravel().astype(np.float64)).reshape(L.shape).astype(b.dtype)
+
+
+def cycle(levels, factors, dirichlet, nu, b, l=0):
+    L = levels[l]
+    if l == len(levels) - 1:
+        return coarsest(L, b, dirichlet and b.size <= 512)
+    x = np.zeros_like(b)
+    for _ in range(nu):
+        x = L.sweep(x, b)
+    r = L.vol * (b - (L.diag.astype(b.dtype) * x - L.off(x))).astype(np.float64)
+    f, s = factors[l], L.shape
+    rc = r.reshape(s[0] // f[0], f[0], s[1] // f[1], f[1], s[2] // f[2], f[2]).sum(axis=(1, 3, 5))
+    xc = cycle(levels, factors, dirichlet, nu, (rc / levels[l + 1].vol).astype(b.dtype), l + 1)
+    for a in range(3):
+        xc = np.repeat(xc, f[a], axis=a)
+    x = x + xc
+    for _ in range(nu):
+        x = L.sweep(x, b)
+    return x
+
+
+def grids(name):
+    if name == "stretched":
+        ax, ay = axis_tanh(96, 12.0, 4.0, 0.05, 1.0, 1.08), axis_tanh(80, 10.0, 5.0, 0.05, 1.0, 1.08)
+        az = axis_uniform(24, 2.4)
+        return GridArrays((96, 80, 24), ax[0], ay[0], az[0], ax[1], ay[1], az[1], ax[2], ay[2], az[2], 12.0, 10.0, 2.4)
+    return uniform_grid(name, tuple(0.1 * n for n in name))
+
+
+@pytest.mark.parametrize("ncal,nu,periodic,mixed", [
+    ((64, 32, 16), 4, False, False), ((64, 32, 16), 2, True, False), ((64, 32, 16), 3, True, False),
+    ((64, 32, 16), 1, False, False), ((48, 48, 64), 4, True, False), ((40, 96, 64), 4, False, True),
+    ((44, 100, 40), 5, False, False), ((24, 20, 132), 4, True, False), ((24, 16, 260), 2, False, False),
+    ((34, 50, 21), 4, False, False), ((20, 36, 27), 6, False, True), ((16, 12, 8), 4, False, False),
+    ((50, 26, 10), 4, False, False), ("stretched", 4, True, False), ((8, 64, 64), 4, False, True)])
+def test_two_iterations_against_numpy(require_gpu, ncal, nu, periodic, mixed):
+    print(f"multigrid cycle ncal={ncal} nu={nu} periodic={periodic} mixed={mixed}", flush=True)
+    grid = grids(ncal)
+    p = configs.cylinder_params(100.0, 0.002, 1.0, 1.0, 1.0, 1e-30)
+    p.precond, p.mg_nu, p.maxit = capi.CFD_PRECOND_MG, nu, 1
+    p.periodic_z = int(periodic)
+    if mixed:
+        p.precision, p.mixed_mode = capi.CFD_MIXED, capi.CFD_MIXED_PC32
+    with Simulation(grid, p) as sim:
+        sim.init_state()
+        sim.createPressureMatrix()
+        b = np.random.default_rng(11).standard_normal(sim.N)
+        b -= b.mean()
+        sim.upload(capi.RHS, b)
+        sim.upload(capi.X, np.zeros(sim.N))
+        it, _ = sim.solve()
+        assert it == 1  # stopped at the cap, after the second iteration
+        got = sim.download(capi.X)
+        col, val = (q.reshape(7, -1) for q in sim.ell())
+        jp = sim.download(capi.JP)
+    levels, factors, dirichlet = hierarchy(grid, p)
+    dt = np.float32 if mixed else np.float64
+
+    def M(r):
+        c = cycle(levels, factors, dirichlet, nu, (r / jp).astype(dt).reshape(grid.ncal))
+        return c.astype(np.float64).ravel()
+
+    def A(x):
+        return (val * x[col]).sum(axis=0)
+
+    x, r = np.zeros_like(b), b.copy()
+    r0, q, rho = r.copy(), r.copy(), r @ r
+    for _ in range(2):
+        ph = M(q)
+        v = A(ph)
+        alpha = rho / (v @ r0)
+        s = r - alpha * v
+        sh = M(s)
+        t = A(sh)
+        omega = (t @ s) / (t @ t)
+        x += alpha * ph + omega * sh
+        r = s - omega * t
+        rho_new = r @ r0
+        q = r + (alpha / omega) * (rho_new / rho) * (q - omega * v)
+        rho = rho_new
+    err = np.linalg.norm(got - x) / np.linalg.norm(x)
+    assert err < (1e-4 if mixed else 1e-11), err
