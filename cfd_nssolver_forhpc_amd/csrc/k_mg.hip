@@ -778,116 +778,284 @@ __global__ void __launch_bounds__(256) mg_restrict_kernel(MGView F, MGView C, co
   restrict_at<T, Lay>(F, C, I, J, K, bf, xf, bc, xc);
 }
 
-constexpr int MG_SMALL_THREADS = 512;
-
-// dense-inverse entries a thread of the bottom kernel prefetches: with the
-// levels in LDS and an inverse of at most DENSE_PF * MG_SMALL_THREADS
-// entries (64 cells), the whole inverse is loaded with the first level's x and
-// b and staged through the LDS left over, instead of 16+ dependent round
-// trips to memory at the coarsest solve
-constexpr int DENSE_PF = 8;
+// ---- the bottom of the V-cycle (levels of at most MG_SMALL cells) ----------
+//
+// One workgroup, one launch; __syncthreads separates the half-sweeps.  What
+// bounds it is the length of a half-sweep's chain: about 35 of them follow
+// each other whatever the levels' sizes.  So a thread keeps what a half-sweep
+// needs of its cells (at most BOTTOM_CELLS of each colour: neighbour
+// positions, coefficients, diagonal and its reciprocal, right-hand side) in
+// registers for as long as the workgroup works on a level; the levels' x, the
+// right-hand sides handed down, the residuals and the axis arrays are in LDS.
+// A half-sweep is then six LDS reads, their sum, a division and a barrier.
+// 512x256x64's bottom (2048, 256 and 64 cells, 30 half-sweeps and a dense
+// solve) takes 21.9 us FP64 against 48.8 for the cell-by-cell form that
+// read coefficients from memory and split indices by division in every
+// half-sweep; 96 half-sweeps of a 1625-cell coarsest level 26.3 against 110.
+constexpr int BOTTOM_THREADS = 1024;
+constexpr int BOTTOM_CELLS = (int)(MG_SMALL / 2 / BOTTOM_THREADS);
+static_assert(BOTTOM_CELLS * 2 * BOTTOM_THREADS == MG_SMALL, "a thread's cells");
+constexpr size_t BOTTOM_LDS = 156 * 1024;  // of a CU's 160 KB
+constexpr int DENSE_PF = 4;  // dense-inverse entries a thread prefetches: a 64-cell inverse
 
 template <typename T>
 struct SmallArgs {
   int nlev, nu, coarse_sweeps, dense;
-  int stage_off, stage_cols;   // dense-inverse staging in LDS: element offset, columns a chunk (0: none)
-  int lds_off[MG_MAX_LEVELS];  // with the levels in LDS: element offset of level l's x (its b follows)
+  // the bottom kernel's LDS: doubles, then elements of T
+  int coef_off[MG_MAX_LEVELS];  // level l's axis arrays
+  int x_off[MG_MAX_LEVELS];     // its x, its b behind it
+  int t_base, res_off, stage_off, staged;
   MGView v[MG_MAX_LEVELS];
   T *x[MG_MAX_LEVELS];
   T *b[MG_MAX_LEVELS];
   const T *cinv;  // dense inverse of the coarsest operator, column-major, when dense
 };
 
-// fills lds_off and, when the dense inverse is prefetched, stage_off /
-// stage_cols; the LDS bytes to launch with (0: the levels do not fit in a
-// workgroup's default 64 KiB and stay in global memory)
+// fills the LDS positions; the bytes to launch the bottom kernel with (0: the
+// levels do not fit a workgroup)
 template <typename T>
-size_t small_lds_layout(SmallArgs<T> &S) {
-  size_t elems = 0;
+size_t bottom_layout(SmallArgs<T> &S) {
+  if (S.v[0].n > MG_SMALL) return 0;
+  size_t dbl = 0, elems = 0;
   for (int l = 0; l < S.nlev; ++l) {
-    S.lds_off[l] = (int)elems;
+    S.coef_off[l] = (int)dbl;
+    dbl += 4 * (size_t)(S.v[l].nx + S.v[l].ny + S.v[l].nz);
+    S.x_off[l] = (int)elems;
     elems += 2 * (size_t)S.v[l].n;
+    // an odd nz leaves threads without a cell: more of them than there are
+    if ((int64_t)S.v[l].nx * S.v[l].ny * ((S.v[l].nz + 1) / 2) > BOTTOM_CELLS * BOTTOM_THREADS) return 0;
   }
-  S.stage_off = 0;
-  S.stage_cols = 0;
-  if (elems * sizeof(T) > 65536) return 0;
-  const int64_t n = S.v[S.nlev - 1].n;
-  if (S.dense && n * n <= (int64_t)DENSE_PF * MG_SMALL_THREADS) {
-    const int64_t cols = std::min<int64_t>(n, (65536 / (int64_t)sizeof(T) - (int64_t)elems) / n);
-    if (cols >= 1) {
-      S.stage_off = (int)elems;
-      S.stage_cols = (int)cols;
-      elems += (size_t)(cols * n);
-    }
+  S.t_base = (int)dbl;
+  S.res_off = (int)elems;
+  if (S.nlev > 1) elems += (size_t)S.v[0].n;
+  S.stage_off = (int)elems;
+  S.staged = 0;
+  if (dbl * sizeof(double) + elems * sizeof(T) > BOTTOM_LDS) return 0;
+  const size_t nn = (size_t)(S.v[S.nlev - 1].n * S.v[S.nlev - 1].n);
+  if (S.dense && nn <= (size_t)DENSE_PF * BOTTOM_THREADS &&
+      dbl * sizeof(double) + (elems + nn) * sizeof(T) <= BOTTOM_LDS) {
+    S.staged = 1;
+    elems += nn;
   }
-  return elems * sizeof(T);
+  return dbl * sizeof(double) + elems * sizeof(T);
 }
 
-// the bottom of the V-cycle (levels of at most MG_SMALL cells) in one
-// workgroup; __syncthreads separates the phases.  When they fit, every
-// level's x and b live in LDS for the whole launch: the first level's
-// right-hand side and first red half-sweep (written by the launch before)
-// are read in at the start and its x is written back at the end, the only
-// values the rest of the cycle uses.  Otherwise they stay in global memory
-// (L2-resident).  The coarsest level is solved by its dense inverse when it
-// is nonsingular, else smoothed coarse_sweeps times.
-template <typename T, bool LDS>
-__global__ void __launch_bounds__(MG_SMALL_THREADS) mg_small_kernel(SmallArgs<T> S, const KrylovScalars *ks) {
+// a level as the bottom kernel sees it: axis arrays in LDS
+struct BottomLevel {
+  int nx, ny, nz, n, wz;
+  const double *ax, *ay, *az;
+  __device__ double diag(int i, int j, int k) const { return ax[2 * nx + i] + ay[2 * ny + j] + az[2 * nz + k]; }
+  __device__ double vol(int i, int j, int k) const { return ax[3 * nx + i] * ay[3 * ny + j] * az[3 * nz + k]; }
+};
+
+// one cell of a thread: LDS positions (two to a register), coefficients in
+// rb_at's order (an absent neighbour is the cell itself with coefficient 0)
+template <typename T>
+struct BottomCell {
+  unsigned cn, x, y, z;  // own position | parent's; -x | +x; -y | +y; -z | +z
+  T a[6], d, r, b;       // coefficients, diagonal and its reciprocal, right-hand side
+  bool on;
+
+  __device__ T off(const T *xl) const {
+    const T vxm = xl[x & 0xffff], vxp = xl[x >> 16], vym = xl[y & 0xffff], vyp = xl[y >> 16], vzm = xl[z & 0xffff],
+            vzp = xl[z >> 16];
+    T s = fma(a[0], vxm, (T)0);
+    s = fma(a[1], vxp, s);
+    s = fma(a[2], vym, s);
+    s = fma(a[3], vyp, s);
+    s = fma(a[4], vzm, s);
+    return fma(a[5], vzp, s);
+  }
+};
+
+template <typename T>
+__global__ void __launch_bounds__(BOTTOM_THREADS) mg_bottom_kernel(SmallArgs<T> S, const KrylovScalars *ks) {
   if (ks && ks->done) return;
-  const int nt = MG_SMALL_THREADS;
-  extern __shared__ __align__(16) unsigned char small_lds[];
-  T *const lds = reinterpret_cast<T *>(small_lds);
-  // compile-time choice, so that the LDS accesses compile to LDS instructions
-  auto X = [&](int l) -> T * {
-    if constexpr (LDS) return lds + S.lds_off[l];
-    else return S.x[l];
+  extern __shared__ __align__(16) double bottom_lds[];
+  const int tid = threadIdx.x;
+  T *const lds = reinterpret_cast<T *>(bottom_lds + S.t_base);
+  T *const res = lds + S.res_off;
+  auto X = [&](int l) { return lds + S.x_off[l]; };
+  auto B = [&](int l) { return lds + S.x_off[l] + (int)S.v[l].n; };
+  auto level = [&](int l) {
+    const MGView &v = S.v[l];
+    const double *c = bottom_lds + S.coef_off[l];
+    return BottomLevel{v.nx, v.ny, v.nz, (int)v.n, v.wz, c, c + 4 * v.nx, c + 4 * (v.nx + v.ny)};
   };
-  auto B = [&](int l) -> T * {
-    if constexpr (LDS) return lds + S.lds_off[l] + S.v[l].n;
-    else return S.b[l];
-  };
-  // with the levels in LDS: the first level's x and b (at most MG_SMALL
-  // cells, 8 a thread) and, with staging, the dense inverse are loaded
-  // before the first LDS store, one round trip to memory for all of them
-  T pf[DENSE_PF];
-  const int nn = S.stage_cols > 0 ? (int)(S.v[S.nlev - 1].n * S.v[S.nlev - 1].n) : 0;
-  if (LDS) {
-    constexpr int CP = (int)(MG_SMALL / MG_SMALL_THREADS);
-    const int n0 = (int)S.v[0].n;
-    T xv[CP], bv[CP];
+  // the first level's x and b, the axis arrays and a small dense inverse: one
+  // round trip to memory for all of them
+  constexpr int CP = (int)(MG_SMALL / BOTTOM_THREADS);
+  const int n0 = (int)S.v[0].n, last = S.nlev - 1;
+  T xv[CP], bv[CP], pf[DENSE_PF];
 #pragma unroll
-    for (int u = 0; u < CP; ++u) {
-      const int t = threadIdx.x + u * nt;
-      xv[u] = t < n0 ? S.x[0][t] : (T)0;
-      bv[u] = t < n0 ? S.b[0][t] : (T)0;
+  for (int u = 0; u < CP; ++u) {
+    const int t = tid + u * BOTTOM_THREADS;
+    xv[u] = t < n0 ? S.x[0][t] : (T)0;
+    bv[u] = t < n0 ? S.b[0][t] : (T)0;
+  }
+  const int nn = S.staged ? (int)(S.v[last].n * S.v[last].n) : 0;
+#pragma unroll
+  for (int u = 0; u < DENSE_PF; ++u) {
+    const int e = tid + u * BOTTOM_THREADS;
+    pf[u] = e < nn ? S.cinv[e] : (T)0;
+  }
+  for (int l = 0; l < S.nlev; ++l) {
+    const int nc = 4 * (S.v[l].nx + S.v[l].ny + S.v[l].nz);
+    for (int q = tid; q < nc; q += BOTTOM_THREADS) bottom_lds[S.coef_off[l] + q] = S.v[l].ax[q];
+  }
+#pragma unroll
+  for (int u = 0; u < CP; ++u) {
+    const int t = tid + u * BOTTOM_THREADS;
+    if (t < n0) {
+      X(0)[t] = xv[u];
+      B(0)[t] = bv[u];
     }
+  }
 #pragma unroll
-    for (int u = 0; u < DENSE_PF; ++u) {
-      const int e = threadIdx.x + u * nt;
-      pf[u] = e < nn ? S.cinv[e] : (T)0;
-    }
+  for (int u = 0; u < DENSE_PF; ++u) {
+    const int e = tid + u * BOTTOM_THREADS;
+    if (e < nn) lds[S.stage_off + e] = pf[u];
+  }
+  __syncthreads();
+
+  // nsw sweeps of level l.  skip_red0: the first red half-sweep is done;
+  // correct: level l + 1's correction goes into the black cells first (the red
+  // ones are overwritten); restrict_to: the residual into res at the end.
+  // C: cells of a colour a thread owns.
+  auto visit = [&](auto cc, int l, int nsw, bool skip_red0, bool correct, bool residual)
+                   __attribute__((always_inline)) {
+    constexpr int C = decltype(cc)::value;
+    const BottomLevel L = level(l);
+    T *const xl = X(l);
+    const T *const bl = B(l);
+    const int hz = (L.nz + 1) / 2, sx = L.ny * L.nz, cnt = L.nx * L.ny * hz;
+    const MGView &F = S.v[l];
+    BottomCell<T> cell[2][C];
 #pragma unroll
-    for (int u = 0; u < CP; ++u) {
-      const int t = threadIdx.x + u * nt;
-      if (t < n0) {
-        X(0)[t] = xv[u];
-        B(0)[t] = bv[u];
+    for (int m = 0; m < C; ++m) {
+      const int t = tid + m * BOTTOM_THREADS;
+      const int q = min(t, cnt - 1) / hz, k2 = min(t, cnt - 1) - q * hz, i = q / L.ny, j = q - i * L.ny;
+#pragma unroll
+      for (int colour = 0; colour < 2; ++colour) {
+        BottomCell<T> &e = cell[colour][m];
+        const int kk = 2 * k2 + ((i + j + colour) & 1), k = min(kk, L.nz - 1);
+        e.on = t < cnt && kk < L.nz;
+        const int o = (i * L.ny + j) * L.nz + k;
+        const int zm = k > 0 ? o - 1 : L.wz ? o + (L.nz - 1) : o, zp = k < L.nz - 1 ? o + 1 : L.wz ? o - (L.nz - 1) : o;
+        int par = 0;
+        if (correct)
+          par = ((F.fx == 2 ? i >> 1 : i) * S.v[l + 1].ny + (F.fy == 2 ? j >> 1 : j)) * S.v[l + 1].nz +
+                (F.fz == 2 ? k >> 1 : k);
+        e.cn = (unsigned)o | (unsigned)par << 16;
+        e.x = (unsigned)(i > 0 ? o - sx : o) | (unsigned)(i < L.nx - 1 ? o + sx : o) << 16;
+        e.y = (unsigned)(j > 0 ? o - L.nz : o) | (unsigned)(j < L.ny - 1 ? o + L.nz : o) << 16;
+        e.z = (unsigned)zm | (unsigned)zp << 16;
+        e.a[0] = (T)L.ax[i];
+        e.a[1] = (T)L.ax[L.nx + i];
+        e.a[2] = (T)L.ay[j];
+        e.a[3] = (T)L.ay[L.ny + j];
+        e.a[4] = (T)L.az[k];
+        e.a[5] = (T)L.az[L.nz + k];
+        e.d = (T)L.diag(i, j, k);
+        e.r = div_recip(e.d);
+        e.b = bl[o];
       }
     }
-    for (int t = threadIdx.x + CP * nt; t < n0; t += nt) {  // not taken: the levels hold at most MG_SMALL cells
-      X(0)[t] = S.x[0][t];
-      B(0)[t] = S.b[0][t];
+    if (correct) {
+#pragma unroll
+      for (int m = 0; m < C; ++m)
+        if (cell[1][m].on) xl[cell[1][m].cn & 0xffff] += X(l + 1)[cell[1][m].cn >> 16];
+      __syncthreads();
+    }
+    for (int s = 0; s < nsw; ++s) {
+#pragma unroll
+      for (int colour = 0; colour < 2; ++colour) {
+        if (s == 0 && colour == 0 && skip_red0) continue;
+#pragma unroll
+        for (int m = 0; m < C; ++m) {
+          const BottomCell<T> &e = cell[colour][m];
+          const T v = div_by(e.b + e.off(xl), e.d, e.r);
+          if (e.on) xl[e.cn & 0xffff] = v;
+        }
+        __syncthreads();
+      }
+    }
+    if (residual) {
+#pragma unroll
+      for (int colour = 0; colour < 2; ++colour)
+#pragma unroll
+        for (int m = 0; m < C; ++m) {
+          const BottomCell<T> &e = cell[colour][m];
+          const T r = e.b - fma(e.d, xl[e.cn & 0xffff], -e.off(xl));
+          if (e.on) res[e.cn & 0xffff] = r;
+        }
+      __syncthreads();
+    }
+  };
+  // down to the coarsest level and up again
+#pragma unroll 1
+  for (int ph = 0; ph <= 2 * last; ++ph) {
+    const bool down = ph < last, up = ph > last;
+    const int l = up ? 2 * last - ph : ph;
+    if (ph == last && S.dense) {
+      // x = A^-1 b, a row a thread, summed over the columns in order
+      const int n = (int)S.v[last].n;
+      const T *const bl = B(last);
+      T *const xl = X(last);
+      if (tid < n) {
+        double acc = 0.0;
+        if (S.staged) {
+          const T *const inv = lds + S.stage_off + tid;
+          for (int q = 0; q < n; ++q) acc += (double)inv[q * n] * (double)bl[q];
+        } else {
+          for (int q = 0; q < n; ++q) acc += (double)S.cinv[(int64_t)q * n + tid] * (double)bl[q];
+        }
+        xl[tid] = (T)acc;
+      }
+      __syncthreads();
+      continue;
+    }
+    const int nsw = ph == last ? S.coarse_sweeps : S.nu;
+    if (S.v[l].nx * S.v[l].ny * ((S.v[l].nz + 1) / 2) <= BOTTOM_THREADS)
+      visit(std::integral_constant<int, 1>{}, l, nsw, !up, up, down);
+    else
+      visit(std::integral_constant<int, BOTTOM_CELLS>{}, l, nsw, !up, up, down);
+    if (!down) continue;
+    // the children's residuals, volume-weighted, and the first red half-sweep (set_rhs)
+    const BottomLevel F = level(l), C = level(l + 1);
+    const int fx = S.v[l].fx, fy = S.v[l].fy, fz = S.v[l].fz;
+    for (int t = tid; t < C.n; t += BOTTOM_THREADS) {
+      const int K = t % C.nz, q = t / C.nz, J = q % C.ny, I = q / C.ny;
+      double acc = 0.0;
+      for (int di = 0; di < fx; ++di)
+        for (int dj = 0; dj < fy; ++dj)
+          for (int dk = 0; dk < fz; ++dk) {
+            const int i = I * fx + di, j = J * fy + dj, k = K * fz + dk;
+            acc = fma(F.vol(i, j, k), (double)res[(i * F.ny + j) * F.nz + k], acc);
+          }
+      const T bc = (T)(acc / C.vol(I, J, K));
+      B(l + 1)[t] = bc;
+      X(l + 1)[t] = ((I + J + K) & 1) == 0 ? bc / (T)C.diag(I, J, K) : (T)0;
     }
     __syncthreads();
   }
+  for (int t = tid; t < n0; t += BOTTOM_THREADS) S.x[0][t] = X(0)[t];
+}
+
+// The same on levels that a workgroup's LDS does not hold (a coarsest level
+// that never halves below MG_SMALL cells): cell by cell, x and b in memory.
+constexpr int MG_SMALL_THREADS = 512;
+
+template <typename T>
+__global__ void __launch_bounds__(MG_SMALL_THREADS) mg_small_kernel(SmallArgs<T> S, const KrylovScalars *ks) {
+  if (ks && ks->done) return;
+  const int nt = MG_SMALL_THREADS;
   // nsw sweeps of level l; skip_red0: the first red half-sweep is done;
   // prolong_from >= 0: the first red half-sweep folds in that level's correction
   auto sweep = [&](int l, int nsw, bool skip_red0, int prolong_from) {
     const MGView &L = S.v[l];
     const int half = (L.nz + 1) / 2;
     const int cnt = L.nx * L.ny * half;
-    T *xl = X(l);
-    const T *bl = B(l);
     for (int s = 0; s < nsw; ++s)
       for (int colour = 0; colour < 2; ++colour) {
         if (s == 0 && colour == 0 && skip_red0) continue;
@@ -895,9 +1063,9 @@ __global__ void __launch_bounds__(MG_SMALL_THREADS) mg_small_kernel(SmallArgs<T>
         for (int t = threadIdx.x; t < cnt; t += nt) {
           const int k2 = t % half, r = t / half;
           if (fold)
-            rb_prolong_at<T, Natural>(L, S.v[prolong_from], r / L.ny, r % L.ny, k2, bl, xl, X(prolong_from));
+            rb_prolong_at<T, Natural>(L, S.v[prolong_from], r / L.ny, r % L.ny, k2, S.b[l], S.x[l], S.x[prolong_from]);
           else
-            rb_at<T, Natural>(L, r / L.ny, r % L.ny, k2, colour, bl, xl);
+            rb_at<T, Natural>(L, r / L.ny, r % L.ny, k2, colour, S.b[l], S.x[l]);
         }
         __syncthreads();
       }
@@ -908,50 +1076,23 @@ __global__ void __launch_bounds__(MG_SMALL_THREADS) mg_small_kernel(SmallArgs<T>
     const MGView &C = S.v[l + 1];
     for (int t = threadIdx.x; t < (int)C.n; t += nt) {
       const int K = t % C.nz, r = t / C.nz;
-      restrict_at<T, Natural>(S.v[l], C, r / C.ny, r % C.ny, K, B(l), X(l), B(l + 1), X(l + 1));
+      restrict_at<T, Natural>(S.v[l], C, r / C.ny, r % C.ny, K, S.b[l], S.x[l], S.b[l + 1], S.x[l + 1]);
     }
     __syncthreads();
   }
-  if (S.dense && LDS && S.stage_cols > 0) {
-    // the prefetched inverse (entry e = q n + t in thread e % nt) through
-    // the LDS stage, stage_cols columns at a time; thread t < n sums its row
-    // over q = 0 .. n - 1 in order, as below
-    const int n = (int)S.v[last].n, sc = S.stage_cols;
-    const T *bl = B(last);
-    T *xl = X(last);
-    T *stage = lds + S.stage_off;
-    double acc = 0.0;
-    for (int q0 = 0; q0 < n; q0 += sc) {
-      const int q1 = min(n, q0 + sc);
-#pragma unroll
-      for (int u = 0; u < DENSE_PF; ++u) {
-        const int e = threadIdx.x + u * nt;
-        if (e >= q0 * n && e < q1 * n) stage[e - q0 * n] = pf[u];
-      }
-      __syncthreads();
-      if ((int)threadIdx.x < n)
-        for (int q = q0; q < q1; ++q) acc += (double)stage[(q - q0) * n + threadIdx.x] * (double)bl[q];
-      __syncthreads();
-    }
-    if ((int)threadIdx.x < n) xl[threadIdx.x] = (T)acc;
-    __syncthreads();
-  } else if (S.dense) {
+  if (S.dense) {
     // consecutive threads read consecutive entries of a column
     const int n = (int)S.v[last].n;
-    const T *bl = B(last);
-    T *xl = X(last);
     for (int t = threadIdx.x; t < n; t += nt) {
       double acc = 0.0;
-      for (int q = 0; q < n; ++q) acc += (double)S.cinv[(int64_t)q * n + t] * (double)bl[q];
-      xl[t] = (T)acc;
+      for (int q = 0; q < n; ++q) acc += (double)S.cinv[(int64_t)q * n + t] * (double)S.b[last][q];
+      S.x[last][t] = (T)acc;
     }
     __syncthreads();
   } else {
     sweep(last, S.coarse_sweeps, true, -1);
   }
   for (int l = last - 1; l >= 0; --l) sweep(l, S.nu, false, l + 1);
-  if (LDS)
-    for (int t = threadIdx.x; t < (int)S.v[0].n; t += nt) S.x[0][t] = X(0)[t];
 }
 
 // launch shape of a 3-D kernel over (nk, ny, nx) with 256-thread blocks
@@ -1199,11 +1340,14 @@ int mg_apply(Ctx &c, const V *r, V *out, const KrylovScalars *ks) {
     S.x[l - ls] = X(l);
     S.b[l - ls] = lb<T>(M.lv[l]);
   }
-  const size_t lds_bytes = small_lds_layout(S);
-  if (lds_bytes)
-    mg_small_kernel<T, true><<<1, MG_SMALL_THREADS, lds_bytes, c.stream>>>(S, ks);
-  else
-    mg_small_kernel<T, false><<<1, MG_SMALL_THREADS, 0, c.stream>>>(S, ks);
+  const size_t lds_bytes = bottom_layout(S);
+  if (lds_bytes) {
+    CFD_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(mg_bottom_kernel<T>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)BOTTOM_LDS));
+    mg_bottom_kernel<T><<<1, BOTTOM_THREADS, lds_bytes, c.stream>>>(S, ks);
+  } else {
+    mg_small_kernel<T><<<1, MG_SMALL_THREADS, 0, c.stream>>>(S, ks);
+  }
   for (int l = ls - 1; l >= 0; --l) smooth(l, false);
   if (!same && !split) mg_widen_kernel<T, V><<<nblk(c.g.N), 256, 0, c.stream>>>(c.g.N, x0, out, ks);
   CFD_HIP(hipGetLastError());
