@@ -46,19 +46,22 @@ try:  # the host cores this process may use, before an OpenMP runtime binds its 
     HOST_CPUS = os.sched_getaffinity(0)
 except (AttributeError, OSError):
     HOST_CPUS = None
-# algorithmic bytes per row: ELL SpMV 7 x (val + col) + x + y; SPE x + jp + y;
-# BiCGSTAB iteration (5 fused kernels) 320; RB-SOR sweep 84 + x + b + x(w) + x(nbr)
-# SpMV-dot (K1 of the iteration): the SpMV's 100 plus r0 8
-BYTES = {"spmv_fp64": 100, "spmv_fp32": 64, "spe_fp64": 24, "bicg_iter": 320, "sor_sweep": 116,
-         "copy": 16, "predictor": 48, "spmv_dot": 108}
+# algorithmic bytes per row.  The assembled ELL operator's FP64 products form its
+# entries again from the axis coefficients: SpMV x + y; with the dot of the
+# iteration's K1 r0 too; BiCGSTAB iteration K1 24, s 24, K3 16, x/r 56, p 32.
+# An uploaded matrix is read (..._stored): 7 x (val + col) more.  SPE x + jp + y;
+# RB-SOR sweep 84 + x + b + x(w) + x(nbr)
+BYTES = {"spmv_fp64": 16, "spmv_fp32": 64, "spe_fp64": 24, "bicg_iter": 152, "sor_sweep": 116,
+         "copy": 16, "predictor": 48, "spmv_dot": 24, "spmv_stored": 100, "spmv_dot_stored": 108,
+         "bicg_iter_stored": 320}
 
 
 def log(msg):
     print(msg, file=sys.stderr, flush=True)
 
 
-def profiled_traffic(key="spmv_dot_kernel<double, 512> traffic_bytes_per_launch:"):
-    """HBM bytes per launch of a kernel from the committed rocprofv3 counter
+def profiled_traffic(key="BiCGSTAB iteration traffic_bytes:"):
+    """HBM bytes of an iteration's kernels from the committed rocprofv3 counter
     summary (FETCH_SIZE and WRITE_SIZE scaled by the copy-kernel calibration)."""
     path = ROOT / "profiles" / "kernels_512x256x64.md"
     try:
@@ -302,10 +305,13 @@ def kernel_table(sim, reps):
     except Exception as e:  # CSR operator not assembled for this context
         log(f"[bench] kernel spmv_csr: {e}")
     for what, name in ((8, "spmv_dot"), (0, "spmv_fp64"), (1, "spmv_fp32"), (2, "spe_fp64"), (7, "spmv_csr"),
-                       (6, "copy"), (5, "predictor"), (4, "bicg_iter"), (3, "sor_sweep")):
+                       (6, "copy"), (5, "predictor"), (4, "bicg_iter"), (3, "sor_sweep"),
+                       (0, "spmv_stored"), (8, "spmv_dot_stored"), (4, "bicg_iter_stored")):
         if name not in nbytes:
             continue
         try:
+            if name == "spmv_stored":  # the same matrix as an uploaded one
+                sim.set_ell(*sim.ell())
             ms = sim.time_kernel(what, reps if what != 4 else max(10, reps // 4))
         except Exception as e:  # an operator not assembled for this context
             log(f"[bench] kernel {name}: {e}")
@@ -508,7 +514,7 @@ def main():
     iters64 = per_step(st64, "iters")
     solves = passes_report(st64, w64.params.maxit)
     counters = sim64.solver_counters()
-    # kernel table; the timed step spends most in the iteration's SpMV-dot kernels
+    # kernel table; the timed step spends most in the solve's iterations
     sim64.setupPressure()
     sim64.createPressureMatrixCSR()
     kt = kernel_table(sim64, args.reps)
@@ -543,7 +549,7 @@ def main():
         cpu = cpu_baseline(w64, iters64, threads, args.cpu_iters, args.cpu_ref_iters)
         cpu["gpu_speedup"] = tps64 / cpu["value"]  # the same algorithm on both sides
 
-    kd = kt["spmv_dot"]
+    kd = kt["bicg_iter"]
     pressure = (f"bicgstabRe2 (the reference's BiCGSTAB) on the Jacobi-scaled ELL operator, FP64, tol 1e-10, iters_max "
                 f"{w64.params.maxit} as the reference: {solves['passes_at_iteration_cap']} of {solves['passes']} "
                 f"timed passes stopped at iters_max, worst final relative residual {solves['max_final_relres']:.1e} "
@@ -566,8 +572,8 @@ def main():
                    "pressure": pressure, "passes_per_step": 4, "bicgstab_iters_per_step": iters64},
         "roofline": {"bound": "hbm", "achieved": kd["gbs"], "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": kd["gbs"] / HBM_PEAK_GBS, "traffic": profiled_traffic(),
-                     "kernel": "spmv_dot_kernel<double, 512>: K1 of the BiCGSTAB iteration, ap = A p (ELL) with the partial "
-                               "ap . r0; 108 B/row x 8388608 rows per launch",
+                     "kernel": "one BiCGSTAB iteration of the timed step's solve (ap = A p with ap . r0, s, as = A s with "
+                               "its dots, x/r with theirs, p; three reductions): 152 B/row x 8388608 rows",
                      "avg_us": kd["avg_us"]},
         "fp64_solves": solves,
         "solver_counters": counters,

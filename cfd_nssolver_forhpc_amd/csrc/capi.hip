@@ -123,7 +123,8 @@ void free_ctx(Ctx *c) {
   dfree(c->viseff);
   for (auto &q : c->pred) dfree(q);
   for (auto &p : c->f) dfree(p);
-  dfree(c->col); dfree(c->val); dfree(c->val32); dfree(c->colP); dfree(c->valP); dfree(c->valP32); dfree(c->perm);
+  dfree(c->col); dfree(c->val); dfree(c->val32); dfree(c->ell_coef);
+  dfree(c->colP); dfree(c->valP); dfree(c->valP32); dfree(c->perm);
   dfree(c->spe_coef); dfree(c->spe_jp);
   dfree(c->csr_ptr); dfree(c->csr_col); dfree(c->csr_val); dfree(c->csr_jp);
   dfree(c->r0); dfree(c->r1); dfree(c->p1); dfree(c->s1); dfree(c->ap); dfree(c->as); dfree(c->px1); dfree(c->px2);
@@ -512,7 +513,9 @@ int cfd_create(const cfd_grid_desc *grid, const cfd_params *params, int device, 
     if ((rc = dmalloc(&c->f[fid], len))) return bail(rc);
     if (hipMemset(c->f[fid], 0, len * sizeof(double)) != hipSuccess) return bail(fail(CFD_ERR_HIP, "memset"));
   }
-  if ((rc = dmalloc(&c->col, ell_len(N))) || (rc = dmalloc(&c->val, ell_len(N)))) return bail(rc);
+  if ((rc = dmalloc(&c->col, ell_len(N))) || (rc = dmalloc(&c->val, ell_len(N))) ||
+      (rc = dmalloc(&c->ell_coef, (size_t)2 * (c->g.nxc + c->g.nyc + c->g.nzc))))
+    return bail(rc);
   double **kv[8] = {&c->r0, &c->r1, &c->p1, &c->s1, &c->ap, &c->as, &c->px1, &c->px2};
   for (auto p : kv) {
     if ((rc = dmalloc(p, (size_t)N))) return bail(rc);
@@ -766,6 +769,7 @@ int cfd_ell_upload(cfd_ctx *ctx, const int32_t *col, const double *val, size_t n
       hv[(size_t)(b + s * st)] = val[(size_t)s * N + r];
     }
   }
+  c.ell_grid = false;  // from here on the stored entries are the operator
   CFD_HIP(hipMemcpyAsync(c.col, hc.data(), sizeof(int32_t) * hc.size(), hipMemcpyHostToDevice, c.stream));
   CFD_HIP(hipMemcpyAsync(c.val, hv.data(), sizeof(double) * hv.size(), hipMemcpyHostToDevice, c.stream));
   CFD_HIP(hipStreamSynchronize(c.stream));  // the staging vectors go out of scope

@@ -99,6 +99,13 @@ struct Ctx {
   int32_t *perm = nullptr;  // natural row -> permuted position
   int64_t ncolour[2] = {0, 0};
   bool ell_ready = false, spe_ready = false;
+  // the ELL operator is the one cfd_ell_assemble builds (not a caller's): its
+  // entries follow from these axis coefficients (xm, xp over nxc; ym, yp; zm,
+  // zp) and the boundary conditions it was assembled with
+  bool ell_grid = false;
+  double *ell_coef = nullptr;
+  int ell_pd[6] = {};
+  int ell_wrapz = 0;
   // SPE coefficients (xm, xp over nxc; ym, yp over nyc; zm, zp over nzc) and jp
   double *spe_coef = nullptr;
   double *spe_jp = nullptr;

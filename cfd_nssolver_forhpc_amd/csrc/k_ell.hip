@@ -1,5 +1,6 @@
 // k_ell.hip -- pressure-operator assembly and standalone SpMV kernels.
 #include "dev_common.h"
+#include "dev_ell_grid.h"
 #include "dev_spmv.h"
 
 namespace cfd {
@@ -72,6 +73,18 @@ __global__ void __launch_bounds__(256) ell_assemble_kernel(DevGrid g, PBC b, int
     val[eb + q * est] = vs[q];
     if (val32) val32[eb + q * est] = (float)vs[q];
   }
+}
+
+// the quotients of ell_assemble_kernel an axis at a time (ell_grid_value forms
+// the entries from them again)
+__global__ void __launch_bounds__(256) ell_coef_kernel(DevGrid g, double *__restrict__ coef) {
+  const int ax = blockIdx.y, m = (int)(blockIdx.x * blockDim.x + threadIdx.x);
+  const int n = ax == 0 ? g.nxc : ax == 1 ? g.nyc : g.nzc;
+  if (m >= n) return;
+  const double *D = ax == 0 ? g.Dx : ax == 1 ? g.Dy : g.Dz, *Ds = ax == 0 ? g.Dxs : ax == 1 ? g.Dys : g.Dzs;
+  double *q = coef + 2 * (ax == 0 ? 0 : ax == 1 ? g.nxc : g.nxc + g.nyc);
+  q[m] = 1.0 / D[m + GC] / Ds[m + GC - 1];
+  q[n + m] = 1.0 / D[m + GC] / Ds[m + GC];
 }
 
 // Colour-ordered copy of the ELL matrix for red-black SOR: row r moves to
@@ -225,6 +238,11 @@ PBC pbc_of(const Ctx &c) {
 int stream_blocks(int64_t n) { return blocks_for(n, 256, 1 << 30); }
 
 hipError_t launch_ell_assemble(Ctx &c) {
+  const int nax = std::max(c.g.nxc, std::max(c.g.nyc, c.g.nzc));
+  ell_coef_kernel<<<dim3((unsigned)blocks_for(nax, 256, 1 << 30), 3), 256, 0, c.stream>>>(c.g, c.ell_coef);
+  for (int f = 0; f < 6; ++f) c.ell_pd[f] = c.prm.p_dirichlet[f];
+  c.ell_wrapz = c.prm.periodic_z;
+  c.ell_grid = true;
   ell_assemble_kernel<<<blocks_for(c.g.N, 256, 1 << 30), 256, 0, c.stream>>>(c.g, pbc_of(c), c.ell_sliced, c.col,
                                                                              c.val, c.val32, c.f[CFD_JP]);
   return hipGetLastError();
@@ -260,6 +278,8 @@ hipError_t launch_spmv(Ctx &c, int op, int precision, const double *x, double *y
     spmv32_from64_kernel<<<stream_blocks(c.g.N), 256, 0, c.stream>>>(a, x, y);
   else if (op == CFD_OP_SPE && T.blocks <= (1 << 30))
     spe_spmv_kernel<<<(unsigned)T.blocks, 256, 0, c.stream>>>(a, T, x, y);
+  else if (const int pp = ell_grid_period(a, c.g.N / 256, 256, {x, y}))
+    launch_ell_grid<256, 0>(a, pp, nullptr, x, y, nullptr, nullptr, c.stream);
   else
     spmv_kernel<<<stream_blocks(c.g.N), 256, op_lds_bytes(a), c.stream>>>(a, x, y);
   return hipGetLastError();

@@ -28,6 +28,7 @@
 #include "dev_common.h"
 #include "dev_resident.h"
 #include "dev_spmv.h"
+#include "dev_ell_grid.h"
 
 namespace cfd {
 
@@ -439,8 +440,13 @@ hipError_t launch_iters(Ctx &c, const OpArgs &a, const Vecs<T> &v, KrylovScalars
   const SpeTiles tiles = spe_tiles(c.g.nxc, c.g.nyc, c.g.nzc);
   const bool spe = std::is_same<T, double>::value && a.op == CFD_OP_SPE && tiles.blocks <= RED_MAX_BLOCKS;
   const int nbs = spe ? (int)tiles.blocks : nb;
+  const int pp = std::is_same<T, double>::value ? ell_grid_period(a, nb, SPMV_DOT_THREADS, {v.p1, v.ap, v.r0, v.s1, v.as}) : 0;
   for (int it = 0; it < nit; ++it) {
-    if (spe)
+    if (pp)
+      launch_ell_grid<SPMV_DOT_THREADS, 1>(a, pp, ks, reinterpret_cast<const double *>(v.p1),
+                                               reinterpret_cast<double *>(v.ap),
+                                               reinterpret_cast<const double *>(v.r0), p1, c.stream);
+    else if (spe)
       spe_spmv_dot_kernel<<<nbs, 256, 0, c.stream>>>(a, tiles, ks, reinterpret_cast<const double *>(v.p1),
                                                      reinterpret_cast<double *>(v.ap),
                                                      reinterpret_cast<const double *>(v.r0), p1);
@@ -450,7 +456,10 @@ hipError_t launch_iters(Ctx &c, const OpArgs &a, const Vecs<T> &v, KrylovScalars
       spmv_dot_kernel<T><<<nb, 256, op_lds_bytes(a), c.stream>>>(a, ks, v.p1, v.ap, v.r0, p1);
     alpha_finalize<<<1, FIN_THREADS, 0, c.stream>>>(p1, nbs, ks);
     s_update_kernel<T><<<nbu, 256, 0, c.stream>>>(N, ks, v.r1, v.ap, v.s1);
-    if (spe)
+    if (pp)
+      launch_ell_grid<SPMV_DOT_THREADS, 2>(a, pp, ks, reinterpret_cast<const double *>(v.s1),
+                                               reinterpret_cast<double *>(v.as), nullptr, p2, c.stream);
+    else if (spe)
       spe_spmv_dot2_kernel<<<nbs, 256, 0, c.stream>>>(a, tiles, ks, reinterpret_cast<const double *>(v.s1),
                                                       reinterpret_cast<double *>(v.as), p2);
     else if (wide)
@@ -500,7 +509,7 @@ struct ResidentSlots {
 // 19.5 us an iteration against 53.1, at one workgroup 4.7 against 26.4).
 int solve_resident(Ctx &c, const OpArgs &a, const Vecs<double> &v, KrylovScalars *ks, bool *solved) {
   *solved = false;
-  if (a.op != CFD_OP_ELL || a.N > RES_MAX_N) return CFD_OK;
+  if ((a.op != CFD_OP_ELL && a.op != OP_ELL_GRID) || a.N > RES_MAX_N) return CFD_OK;
   ResArgs r;
   r.N = a.N;
   r.nbx = blocks_for(a.N, 4 * 256, RED_MAX_BLOCKS);
@@ -640,10 +649,14 @@ int launch_pc_iters(Ctx &c, const OpArgs &a, const PVecs<T> &v, KrylovScalars *k
   const SpeTiles tiles = spe_tiles(c.g.nxc, c.g.nyc, c.g.nzc);
   const bool spe = std::is_same<T, double>::value && a.op == CFD_OP_SPE && tiles.blocks <= RED_MAX_BLOCKS;
   const int nbs = spe ? (int)tiles.blocks : nb;
+  const int pp = std::is_same<T, double>::value ? ell_grid_period(a, nb, 256, {v.ph, v.v, v.r0, v.sh, v.t, v.s1}) : 0;
   for (int it = 0; it < nit; ++it) {
     int rc = precondition<T>(c, v.p1, v.ph, ks, pc32);
     if (rc) return rc;
-    if (spe)
+    if (pp)
+      launch_ell_grid<256, 1>(a, pp, ks, reinterpret_cast<const double *>(v.ph), reinterpret_cast<double *>(v.v),
+                                  reinterpret_cast<const double *>(v.r0), p1, c.stream);
+    else if (spe)
       spe_spmv_dot_kernel<<<nbs, 256, 0, c.stream>>>(a, tiles, ks, reinterpret_cast<const double *>(v.ph),
                                                      reinterpret_cast<double *>(v.v),
                                                      reinterpret_cast<const double *>(v.r0), p1);
@@ -652,7 +665,10 @@ int launch_pc_iters(Ctx &c, const OpArgs &a, const PVecs<T> &v, KrylovScalars *k
     alpha_finalize<<<1, FIN_THREADS, 0, c.stream>>>(p1, nbs, ks);
     s_update_kernel<T><<<nbu, 256, 0, c.stream>>>(N, ks, v.r1, v.v, v.s1);
     if ((rc = precondition<T>(c, v.s1, v.sh, ks, pc32))) return rc;
-    if (spe)
+    if (pp)
+      launch_ell_grid<256, 3>(a, pp, ks, reinterpret_cast<const double *>(v.sh), reinterpret_cast<double *>(v.t),
+                                  reinterpret_cast<const double *>(v.s1), p2, c.stream);
+    else if (spe)
       spe_spmv_dot2_pc_kernel<<<nbs, 256, 0, c.stream>>>(a, tiles, ks, reinterpret_cast<const double *>(v.sh),
                                                          reinterpret_cast<const double *>(v.s1),
                                                          reinterpret_cast<double *>(v.t), p2);
@@ -814,7 +830,10 @@ hipError_t launch_spmv_dot(Ctx &c) {
   const OpArgs a = op_args(c, c.prm.op);
   const SpeTiles tiles = spe_tiles(c.g.nxc, c.g.nyc, c.g.nzc);
   double *part = red_part_host(c, RS_SPMV_DOT);
-  if (a.op == CFD_OP_SPE && tiles.blocks <= RED_MAX_BLOCKS)
+  if (const int pp = ell_grid_period(a, blocks_for(c.g.N, SPMV_DOT_THREADS, RED_MAX_BLOCKS), SPMV_DOT_THREADS,
+                                      {c.p1, c.ap, c.r0}))
+    launch_ell_grid<SPMV_DOT_THREADS, 1>(a, pp, c.ks32, c.p1, c.ap, c.r0, part, c.stream);
+  else if (a.op == CFD_OP_SPE && tiles.blocks <= RED_MAX_BLOCKS)
     spe_spmv_dot_kernel<<<(int)tiles.blocks, 256, 0, c.stream>>>(a, tiles, c.ks32, c.p1, c.ap, c.r0, part);
   else if (a.op != CFD_OP_CSR)  // launch_iters' launch
     spmv_dot_kernel<double, SPMV_DOT_THREADS>
