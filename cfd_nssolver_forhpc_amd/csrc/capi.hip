@@ -523,9 +523,9 @@ int cfd_create(const cfd_grid_desc *grid, const cfd_params *params, int device, 
   }
   if ((rc = dmalloc(&c->spe_coef, (size_t)2 * (g.nxc + g.nyc + g.nzc))) || (rc = dmalloc(&c->spe_jp, (size_t)N)))
     return bail(rc);
-  if ((rc = dmalloc(&c->ks, 1)) || (rc = dmalloc(&c->ks32, 1))) return bail(rc);
-  (void)hipMemset(c->ks, 0, sizeof(KrylovScalars));
-  (void)hipMemset(c->ks32, 0, sizeof(KrylovScalars));
+  if ((rc = dmalloc(&c->ks, 2)) || (rc = dmalloc(&c->ks32, 2))) return bail(rc);
+  (void)hipMemset(c->ks, 0, 2 * sizeof(KrylovScalars));
+  (void)hipMemset(c->ks32, 0, 2 * sizeof(KrylovScalars));
   if ((rc = dmalloc(&c->red.partials, (size_t)RED_SITES * 3 * RED_MAX_BLOCKS)) ||
       (rc = dmalloc(&c->red.counters, (size_t)RED_SITES)) || (rc = dmalloc(&c->red.out, (size_t)RED_SITES * 4)) ||
       (rc = dmalloc(&c->stepbuf, (size_t)64)))

@@ -124,7 +124,7 @@ struct Ctx {
   double *xP = nullptr, *bP = nullptr, *rP = nullptr;
   float *xP32 = nullptr, *bP32 = nullptr;
   // device scalars and reduction workspace
-  KrylovScalars *ks = nullptr;   // FP64 outer / plain solve
+  KrylovScalars *ks = nullptr;   // FP64 outer / plain solve; [0] between iterations, [1] within one (k_krylov.hip)
   KrylovScalars *ks32 = nullptr; // FP32 inner solve
   KrylovScalars *hks = nullptr;  // pinned host mirror
   RedWork red{};

@@ -12,7 +12,7 @@
 //   K5  p  = r + beta (p - omega ap)   (or r0 = p = r on restart)
 // F1-F3 are one-block kernels combining the per-block partials in a fixed
 // order (deterministic results) and updating the solver's scalars in device
-// memory; every kernel returns at once when the device-side `done` flag is
+// memory, or parts of K2, K4 and K5 in small systems (fold_of); every kernel returns at once when the device-side `done` flag is
 // set, so the host launches iterations in batches and reads the flag once per
 // batch instead of once per dot product.  FP64 dots are kept for every
 // scalar, also when the vectors are FP32.  FP64 systems of up to half a million
@@ -174,15 +174,76 @@ __global__ void __launch_bounds__(256) spe_spmv_dot2_kernel(OpArgs a, SpeTiles T
   block_partials<2>(acc, part);
 }
 
+// combine_partials of nblk <= C FIN_THREADS partials by a block of BT threads:
+// thread t stands in for threads t, t + BT, .. of the finalize block, whose
+// sums over its slots, waves and block are formed in the same order.  (In the
+// finalize kernels too: with 2 of the 16 slots that combine_partials loads at a
+// time, 5.7 -> 3.7 us.)
+template <int BT, int C, int NV>
+__device__ inline void combine_folded(const double *part, int nblk, double (&tot)[NV]) {
+  constexpr int G = FIN_THREADS / BT;
+  static_assert(C == 1 || C == 2 || C == 4, "the tree below");
+  __shared__ double lds[NV][FIN_THREADS / 64];
+  double s[NV][G][C];
+#pragma unroll
+  for (int q = 0; q < NV; ++q)
+#pragma unroll
+    for (int g = 0; g < G; ++g)
+#pragma unroll
+      for (int u = 0; u < C; ++u) {
+        const int b = (int)threadIdx.x + g * BT + u * FIN_THREADS;
+        s[q][g][u] = part[q * RED_MAX_BLOCKS + min(b, nblk - 1)];
+      }
+#pragma unroll
+  for (int q = 0; q < NV; ++q)
+#pragma unroll
+    for (int g = 0; g < G; ++g) {
+#pragma unroll
+      for (int u = 0; u < C; ++u) {
+        const int b = (int)threadIdx.x + g * BT + u * FIN_THREADS;
+        s[q][g][u] = b < nblk ? s[q][g][u] : 0.0;
+      }
+      double v = s[q][g][0];
+      if (C > 1) v += s[q][g][C > 1 ? 1 : 0];
+      if (C > 2) v += s[q][g][C > 2 ? 2 : 0] + s[q][g][C > 2 ? 3 : 0];
+      v = wave_sum(v + 0.0);
+      if ((threadIdx.x & 63) == 0) lds[q][g * (BT / 64) + (threadIdx.x >> 6)] = v;
+    }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < NV; ++q) {
+    double v = lds[q][0];
+#pragma unroll
+    for (int w = 1; w < FIN_THREADS / 64; ++w) v += lds[q][w];
+    tot[q] = v;
+  }
+}
+
+// f(slots a finalize thread takes; 0: combine_partials' chunks of sixteen)
+template <typename F>
+void with_slots(int nblk, F f) {
+  if (nblk <= FIN_THREADS) f(std::integral_constant<int, 1>());
+  else if (nblk <= 2 * FIN_THREADS) f(std::integral_constant<int, 2>());
+  else if (nblk <= 4 * FIN_THREADS) f(std::integral_constant<int, 4>());
+  else f(std::integral_constant<int, 0>());
+}
+
+template <int C, int NV>
+__device__ inline void combine_slots(const double *part, int nblk, double (&tot)[NV]) {
+  if constexpr (C > 0) combine_folded<FIN_THREADS, C>(part, nblk, tot);
+  else combine_partials<NV>(part, nblk, tot);
+}
+
 // The finalize kernels read the scalars they use before the partials, so
 // that those reads share the partials' round trip to memory instead of
 // preceding it; with `done` set the totals are combined and dropped.
+template <int C>
 __global__ void __launch_bounds__(FIN_THREADS) alpha_finalize(const double *part, int nblk, KrylovScalars *ks) {
   const int done = ks->done;
   const double rho = ks->rho;
   asm volatile("" ::: "memory");  // issue both loads here, not after the combine
   double tot[1];
-  combine_partials<1>(part, nblk, tot);
+  combine_slots<C>(part, nblk, tot);
   if (done) return;
   if (threadIdx.x == 0) ks->alpha = rho / tot[0];
 }
@@ -215,11 +276,12 @@ __global__ void __launch_bounds__(BT) spmv_dot2_kernel(OpArgs a, const KrylovSca
   block_partials<2, false, BT>(acc, part);
 }
 
+template <int C>
 __global__ void __launch_bounds__(FIN_THREADS) omega_finalize(const double *part, int nblk, KrylovScalars *ks) {
   const int done = ks->done;
   asm volatile("" ::: "memory");
   double tot[2];
-  combine_partials<2>(part, nblk, tot);
+  combine_slots<C>(part, nblk, tot);
   if (done) return;
   if (threadIdx.x == 0) ks->omega = tot[0] / tot[1];
 }
@@ -235,7 +297,7 @@ __global__ void __launch_bounds__(256) xr_update_kernel(int64_t N, const KrylovS
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   for (int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; r < N; r += stride) {
     const double s = (double)s1[r];
-    ntstore((T)((double)x[r] + (alpha * (double)p1[r] + omega * s)), x + r);
+    ntstore((T)((double)x[r] + fma(omega, s, alpha * (double)p1[r])), x + r);
     const T rn = (T)(s - omega * (double)as[r]);
     ntstore(rn, r1 + r);
     acc[0] += (double)rn * (double)rn;
@@ -245,33 +307,48 @@ __global__ void __launch_bounds__(256) xr_update_kernel(int64_t N, const KrylovS
 }
 
 // stop test, beta and the restart rule (bicgstabRe2.hpp:137-183)
-__global__ void __launch_bounds__(FIN_THREADS) conv_finalize(const double *part, int nblk, KrylovScalars *ks) {
-  const KrylovScalars k = *ks;
+// the scalars after an iteration with (r . r) = rr, (r . r0) = rho
+__device__ inline KrylovScalars conv_next(KrylovScalars k, double rr, double rho) {
+  const double pre_rho = k.rho;
+  k.rnorm = sqrt(rr);
+  k.relres = k.rnorm / k.norm0;
+  if (k.relres < k.tol) {
+    k.done = 1;
+  } else if (k.iters >= k.maxit) {
+    k.done = 1;
+    k.hit_maxit = 1;
+  } else {
+    k.pre_rho = pre_rho;
+    k.rho = rho;
+    k.beta = (k.alpha / k.omega) * (rho / pre_rho);
+    k.restart = (k.timestep < 10 || fabs(pre_rho) > k.restart_tol) ? 0 : 1;
+    k.restarts += k.restart;
+    k.iters += 1;
+  }
+  return k;
+}
+
+template <int C>
+__global__ void __launch_bounds__(FIN_THREADS) conv_finalize(const double *part, int nblk, const KrylovScalars *in,
+                                                             KrylovScalars *out) {
+  const KrylovScalars k = *in;
   asm volatile("" ::: "memory");
   double tot[2];
-  combine_partials<2>(part, nblk, tot);
+  combine_slots<C>(part, nblk, tot);
   if (k.done) return;
-  if (threadIdx.x == 0) {
-    const double rnorm = sqrt(tot[0]), relres = rnorm / k.norm0;
-    ks->rnorm = rnorm;
-    ks->relres = relres;
-    if (relres < k.tol) {
-      ks->done = 1;
-    } else if (k.iters >= k.maxit) {
-      ks->done = 1;
-      ks->hit_maxit = 1;
-    } else {
-      const double pre_rho = k.rho, rho = tot[1];
-      ks->pre_rho = pre_rho;
-      ks->rho = rho;
-      ks->beta = (k.alpha / k.omega) * (rho / pre_rho);
-      const int restart = (k.timestep < 10 || fabs(pre_rho) > k.restart_tol) ? 0 : 1;
-      ks->restart = restart;
-      ks->restarts = k.restarts + restart;
-      ks->iters = k.iters + 1;
-    }
-  }
+  if (threadIdx.x == 0) *out = conv_next(k, tot[0], tot[1]);
 }
+
+void launch_alpha_finalize(const double *part, int nblk, KrylovScalars *ks, hipStream_t st) {
+  with_slots(nblk, [&](auto c) { alpha_finalize<decltype(c)::value><<<1, FIN_THREADS, 0, st>>>(part, nblk, ks); });
+}
+void launch_omega_finalize(const double *part, int nblk, KrylovScalars *ks, hipStream_t st) {
+  with_slots(nblk, [&](auto c) { omega_finalize<decltype(c)::value><<<1, FIN_THREADS, 0, st>>>(part, nblk, ks); });
+}
+void launch_conv_finalize(const double *part, int nblk, const KrylovScalars *in, KrylovScalars *out, hipStream_t st) {
+  with_slots(nblk, [&](auto c) { conv_finalize<decltype(c)::value><<<1, FIN_THREADS, 0, st>>>(part, nblk, in, out); });
+}
+
 
 template <typename T>
 __global__ void __launch_bounds__(256) p_update_kernel(int64_t N, const KrylovScalars *__restrict__ ks,
@@ -349,13 +426,169 @@ __global__ void __launch_bounds__(256) xr_update_pc_kernel(int64_t N, const Kryl
   double acc[2] = {0.0, 0.0};
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   for (int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; r < N; r += stride) {
-    ntstore((T)((double)x[r] + (alpha * (double)ph[r] + omega * (double)sh[r])), x + r);
+    ntstore((T)((double)x[r] + fma(alpha, (double)ph[r], omega * (double)sh[r])), x + r);
     const T rn = (T)((double)s1[r] - omega * (double)tv[r]);
     ntstore(rn, r1 + r);
     acc[0] += (double)rn * (double)rn;
     acc[1] += (double)rn * (double)r0[r];
   }
   block_partials<2>(acc, part);
+}
+
+// ---- the same updates with the reduction before them in each block ----------
+// A finalize kernel is one block: 3 to 6 us, most of it a launch and two round
+// trips to memory.  Small systems' updates combine the partials themselves, in
+// every block, while their rows are on their way from memory.  The scalars
+// then need two copies: ks[0] is read by K1 and written by K5, ks[1] is read
+// by K3, K4 and K5 and written by K2 (all of it) and K4 (omega), so that no
+// kernel writes what its blocks read.
+// row r0 + u * step of a thread, clamped into the system (loads past it are not used)
+__device__ inline int64_t fold_row(int64_t r0, int u, int64_t step, int64_t N) {
+  const int64_t r = r0 + u * step;
+  return r < N ? r : N - 1;
+}
+
+template <typename T, int BT, int ROWS, int C>
+__global__ void __launch_bounds__(BT, BT == 1024 ? 8 : 4) s_fold_kernel(int64_t N, const double *part, int nblk,
+                                                                    const KrylovScalars *__restrict__ ks0,
+                                                                    KrylovScalars *ks1, const T *__restrict__ r1,
+                                                                    const T *__restrict__ ap, T *__restrict__ s1) {
+  const int64_t step = (int64_t)gridDim.x * BT, t = (int64_t)blockIdx.x * BT + threadIdx.x;
+  T rv[ROWS], av[ROWS];
+#pragma unroll
+  for (int u = 0; u < ROWS; ++u) {
+    const int64_t r = fold_row(t, u, step, N);
+    rv[u] = r1[r];
+    av[u] = ap[r];
+  }
+  double tot[1];
+  combine_folded<BT, C>(part, nblk, tot);
+  const int done = ks0->done;
+  const double alpha = ks0->rho / tot[0];
+  if (t == 0) {
+    KrylovScalars k = *ks0;
+    if (!done) k.alpha = alpha;
+    *ks1 = k;
+  }
+  if (done) return;
+#pragma unroll
+  for (int u = 0; u < ROWS; ++u)
+    if (t + u * step < N) s1[t + u * step] = (T)((double)rv[u] - alpha * (double)av[u]);
+}
+
+// xr_update_kernel (PC: xr_update_pc_kernel, with ph and sh in the places of
+// p and s) of ROWS rows a thread, with that kernel's blocks and partials
+template <typename T, bool PC, int ROWS>
+__global__ void __launch_bounds__(256, 4)
+    xr_fold_kernel(int64_t N, const double *dots, int nblk, KrylovScalars *ks1, T *__restrict__ x,
+                   const T *__restrict__ ph, const T *__restrict__ sh, const T *__restrict__ s1,
+                   const T *__restrict__ as, T *__restrict__ r1, const T *__restrict__ r0, double *part) {
+  const int64_t step = (int64_t)gridDim.x * 256, t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  T xv[ROWS], pv[ROWS], hv[ROWS], sv[ROWS], av[ROWS], zv[ROWS];
+#pragma unroll
+  for (int u = 0; u < ROWS; ++u) {
+    const int64_t r = fold_row(t, u, step, N);
+    sv[u] = s1[r];
+    av[u] = as[r];
+    xv[u] = x[r];
+    pv[u] = ph[r];
+    hv[u] = PC ? sh[r] : T(0);
+    zv[u] = r0[r];
+  }
+  double tot[2];
+  combine_folded<256, 1>(dots, nblk, tot);
+  if (ks1->done) return;
+  const double alpha = ks1->alpha, omega = tot[0] / tot[1];
+  if (blockIdx.x == 0 && threadIdx.x == 0) ks1->omega = omega;
+  double acc[2] = {0.0, 0.0};
+#pragma unroll
+  for (int u = 0; u < ROWS; ++u) {
+    const int64_t r = t + u * step;
+    if (r < N) {
+      const double s = (double)sv[u];
+      const double d = PC ? fma(alpha, (double)pv[u], omega * (double)hv[u]) : fma(omega, s, alpha * (double)pv[u]);
+      ntstore((T)((double)xv[u] + d), x + r);
+      const T rn = (T)(s - omega * (double)av[u]);
+      ntstore(rn, r1 + r);
+      acc[0] += (double)rn * (double)rn;
+      acc[1] += (double)rn * (double)zv[u];
+    }
+  }
+  block_partials<2>(acc, part);
+}
+
+template <typename T, int ROWS>
+__global__ void __launch_bounds__(256, 4) p_fold_kernel(int64_t N, const double *part, int nblk,
+                                                                    const KrylovScalars *__restrict__ ks1,
+                                                                    KrylovScalars *ks0, const T *__restrict__ r1,
+                                                                    T *__restrict__ p1, const T *__restrict__ ap,
+                                                                    T *__restrict__ r0) {
+  const int64_t step = (int64_t)gridDim.x * 256, t = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  T rv[ROWS], pv[ROWS], av[ROWS];
+#pragma unroll
+  for (int u = 0; u < ROWS; ++u) {
+    const int64_t r = fold_row(t, u, step, N);
+    rv[u] = r1[r];
+    pv[u] = p1[r];
+    av[u] = ap[r];
+  }
+  double tot[2];
+  combine_folded<256, 1>(part, nblk, tot);
+  if (ks1->done) return;
+  const KrylovScalars k = conv_next(*ks1, tot[0], tot[1]);
+  if (t == 0) *ks0 = k;
+  if (k.done) return;
+#pragma unroll
+  for (int u = 0; u < ROWS; ++u) {
+    const int64_t r = t + u * step;
+    if (r < N) {
+      if (k.restart) {
+        r0[r] = rv[u];
+        p1[r] = rv[u];
+      } else {
+        p1[r] = (T)((double)rv[u] + k.beta * ((double)pv[u] - k.omega * (double)av[u]));
+      }
+    }
+  }
+}
+
+// How an iteration's reductions run, for nd partials of each of the dots of
+// K1 and K3 and nvb of K4's.  ALL: in K2, K4 and K5, up to 1024 partials each;
+// K2: in K2 alone, by blocks of 1024 threads, up to 4096 partials; NONE.
+// SPE iteration: 64x32x32 37 -> 23.5 us (ALL), 128x64x48 42 -> 29.5 (ALL),
+// 200x104x40 60 -> 47.5 (ALL), 190x210x40 81 -> 70 (K2).  K4 and K5 folded at
+// 190x210x40 take 22.7 + 14.8 us in blocks of 1024 threads that are all in
+// flight at once, unfolded 3.7 + 17.0 + 4.3 + 11.5: the rows wait for the
+// reduction, then all are stored at once.  Past 4096 partials every block would
+// read more than 33 KB of them.
+enum class Fold { NONE, K2, ALL };
+Fold fold_of(int nd, int nvb) {
+  if (nd <= FIN_THREADS && nvb <= FIN_THREADS) return Fold::ALL;
+  return nd <= 4 * FIN_THREADS ? Fold::K2 : Fold::NONE;
+}
+
+template <typename T>
+void launch_s_fold(Fold fold, int64_t N, const double *d1, int nd, KrylovScalars *ks, const T *r1, const T *ap, T *s1,
+                   hipStream_t st) {
+  auto blocks = [N](int rows) { return (unsigned)((N + rows - 1) / rows); };
+  if (fold == Fold::K2)
+    with_slots(nd, [&](auto c) {
+      constexpr int C = decltype(c)::value > 0 ? decltype(c)::value : 4;
+      s_fold_kernel<T, 1024, 4, C><<<blocks(4096), 1024, 0, st>>>(N, d1, nd, ks, ks + 1, r1, ap, s1);
+    });
+  else if (N <= 512 * 1024)
+    s_fold_kernel<T, 256, 2, 1><<<blocks(512), 256, 0, st>>>(N, d1, nd, ks, ks + 1, r1, ap, s1);
+  else
+    s_fold_kernel<T, 256, 4, 1><<<blocks(1024), 256, 0, st>>>(N, d1, nd, ks, ks + 1, r1, ap, s1);
+}
+
+template <typename T>
+void launch_p_fold(int64_t N, const double *part, int nvb, KrylovScalars *ks, const T *r1, T *p1, const T *ap, T *r0,
+                   hipStream_t st) {
+  if (N <= 512 * 1024)
+    p_fold_kernel<T, 2><<<(unsigned)((N + 511) / 512), 256, 0, st>>>(N, part, nvb, ks + 1, ks, r1, p1, ap, r0);
+  else
+    p_fold_kernel<T, 4><<<(unsigned)((N + 1023) / 1024), 256, 0, st>>>(N, part, nvb, ks + 1, ks, r1, p1, ap, r0);
 }
 
 // NaN / Inf reset after iters_max (bicgstabRe2.hpp:143-163)
@@ -441,6 +674,8 @@ hipError_t launch_iters(Ctx &c, const OpArgs &a, const Vecs<T> &v, KrylovScalars
   const bool spe = std::is_same<T, double>::value && a.op == CFD_OP_SPE && tiles.blocks <= RED_MAX_BLOCKS;
   const int nbs = spe ? (int)tiles.blocks : nb;
   const int pp = std::is_same<T, double>::value ? ell_grid_period(a, nb, SPMV_DOT_THREADS, {v.p1, v.ap, v.r0, v.s1, v.as}) : 0;
+  const Fold fold = fold_of(nbs, nbx);
+  KrylovScalars *ks3 = fold == Fold::NONE ? ks : ks + 1;  // from K2 to K4
   for (int it = 0; it < nit; ++it) {
     if (pp)
       launch_ell_grid<SPMV_DOT_THREADS, 1>(a, pp, ks, reinterpret_cast<const double *>(v.p1),
@@ -454,21 +689,31 @@ hipError_t launch_iters(Ctx &c, const OpArgs &a, const Vecs<T> &v, KrylovScalars
       spmv_dot_kernel<T, SPMV_DOT_THREADS><<<nb, SPMV_DOT_THREADS, 0, c.stream>>>(a, ks, v.p1, v.ap, v.r0, p1);
     else
       spmv_dot_kernel<T><<<nb, 256, op_lds_bytes(a), c.stream>>>(a, ks, v.p1, v.ap, v.r0, p1);
-    alpha_finalize<<<1, FIN_THREADS, 0, c.stream>>>(p1, nbs, ks);
-    s_update_kernel<T><<<nbu, 256, 0, c.stream>>>(N, ks, v.r1, v.ap, v.s1);
+    if (fold != Fold::NONE) {
+      launch_s_fold<T>(fold, N, p1, nbs, ks, v.r1, v.ap, v.s1, c.stream);
+    } else {
+      launch_alpha_finalize(p1, nbs, ks, c.stream);
+      s_update_kernel<T><<<nbu, 256, 0, c.stream>>>(N, ks, v.r1, v.ap, v.s1);
+    }
     if (pp)
-      launch_ell_grid<SPMV_DOT_THREADS, 2>(a, pp, ks, reinterpret_cast<const double *>(v.s1),
+      launch_ell_grid<SPMV_DOT_THREADS, 2>(a, pp, ks3, reinterpret_cast<const double *>(v.s1),
                                                reinterpret_cast<double *>(v.as), nullptr, p2, c.stream);
     else if (spe)
-      spe_spmv_dot2_kernel<<<nbs, 256, 0, c.stream>>>(a, tiles, ks, reinterpret_cast<const double *>(v.s1),
+      spe_spmv_dot2_kernel<<<nbs, 256, 0, c.stream>>>(a, tiles, ks3, reinterpret_cast<const double *>(v.s1),
                                                       reinterpret_cast<double *>(v.as), p2);
     else if (wide)
-      spmv_dot2_kernel<T, SPMV_DOT_THREADS><<<nb, SPMV_DOT_THREADS, 0, c.stream>>>(a, ks, v.s1, v.as, p2);
+      spmv_dot2_kernel<T, SPMV_DOT_THREADS><<<nb, SPMV_DOT_THREADS, 0, c.stream>>>(a, ks3, v.s1, v.as, p2);
     else
-      spmv_dot2_kernel<T><<<nb, 256, op_lds_bytes(a), c.stream>>>(a, ks, v.s1, v.as, p2);
-    omega_finalize<<<1, FIN_THREADS, 0, c.stream>>>(p2, nbs, ks);
-    xr_update_kernel<T><<<nbx, 256, 0, c.stream>>>(N, ks, v.x, v.p1, v.s1, v.as, v.r1, v.r0, p3);
-    conv_finalize<<<1, FIN_THREADS, 0, c.stream>>>(p3, nbx, ks);
+      spmv_dot2_kernel<T><<<nb, 256, op_lds_bytes(a), c.stream>>>(a, ks3, v.s1, v.as, p2);
+    if (fold == Fold::ALL) {
+      xr_fold_kernel<T, false, 4><<<nbx, 256, 0, c.stream>>>(N, p2, nbs, ks3, v.x, v.p1, nullptr, v.s1, v.as, v.r1, v.r0,
+                                                             p3);
+      launch_p_fold<T>(N, p3, nbx, ks, v.r1, v.p1, v.ap, v.r0, c.stream);
+      continue;
+    }
+    launch_omega_finalize(p2, nbs, ks3, c.stream);
+    xr_update_kernel<T><<<nbx, 256, 0, c.stream>>>(N, ks3, v.x, v.p1, v.s1, v.as, v.r1, v.r0, p3);
+    launch_conv_finalize(p3, nbx, ks3, ks, c.stream);
     p_update_kernel<T><<<nbu, 256, 0, c.stream>>>(N, ks, v.r1, v.p1, v.ap, v.r0);
   }
   return hipGetLastError();
@@ -650,6 +895,8 @@ int launch_pc_iters(Ctx &c, const OpArgs &a, const PVecs<T> &v, KrylovScalars *k
   const bool spe = std::is_same<T, double>::value && a.op == CFD_OP_SPE && tiles.blocks <= RED_MAX_BLOCKS;
   const int nbs = spe ? (int)tiles.blocks : nb;
   const int pp = std::is_same<T, double>::value ? ell_grid_period(a, nb, 256, {v.ph, v.v, v.r0, v.sh, v.t, v.s1}) : 0;
+  const Fold fold = fold_of(nbs, nbu);
+  KrylovScalars *ks3 = fold == Fold::NONE ? ks : ks + 1;  // from K2 to K4
   for (int it = 0; it < nit; ++it) {
     int rc = precondition<T>(c, v.p1, v.ph, ks, pc32);
     if (rc) return rc;
@@ -662,21 +909,31 @@ int launch_pc_iters(Ctx &c, const OpArgs &a, const PVecs<T> &v, KrylovScalars *k
                                                      reinterpret_cast<const double *>(v.r0), p1);
     else
       spmv_dot_kernel<T><<<nb, 256, op_lds_bytes(a), c.stream>>>(a, ks, v.ph, v.v, v.r0, p1);
-    alpha_finalize<<<1, FIN_THREADS, 0, c.stream>>>(p1, nbs, ks);
-    s_update_kernel<T><<<nbu, 256, 0, c.stream>>>(N, ks, v.r1, v.v, v.s1);
-    if ((rc = precondition<T>(c, v.s1, v.sh, ks, pc32))) return rc;
+    if (fold != Fold::NONE) {
+      launch_s_fold<T>(fold, N, p1, nbs, ks, v.r1, v.v, v.s1, c.stream);
+    } else {
+      launch_alpha_finalize(p1, nbs, ks, c.stream);
+      s_update_kernel<T><<<nbu, 256, 0, c.stream>>>(N, ks, v.r1, v.v, v.s1);
+    }
+    if ((rc = precondition<T>(c, v.s1, v.sh, ks3, pc32))) return rc;
     if (pp)
-      launch_ell_grid<256, 3>(a, pp, ks, reinterpret_cast<const double *>(v.sh), reinterpret_cast<double *>(v.t),
+      launch_ell_grid<256, 3>(a, pp, ks3, reinterpret_cast<const double *>(v.sh), reinterpret_cast<double *>(v.t),
                                   reinterpret_cast<const double *>(v.s1), p2, c.stream);
     else if (spe)
-      spe_spmv_dot2_pc_kernel<<<nbs, 256, 0, c.stream>>>(a, tiles, ks, reinterpret_cast<const double *>(v.sh),
+      spe_spmv_dot2_pc_kernel<<<nbs, 256, 0, c.stream>>>(a, tiles, ks3, reinterpret_cast<const double *>(v.sh),
                                                          reinterpret_cast<const double *>(v.s1),
                                                          reinterpret_cast<double *>(v.t), p2);
     else
-      spmv_dot2_pc_kernel<T><<<nb, 256, op_lds_bytes(a), c.stream>>>(a, ks, v.sh, v.s1, v.t, p2);
-    omega_finalize<<<1, FIN_THREADS, 0, c.stream>>>(p2, nbs, ks);
-    xr_update_pc_kernel<T><<<nbu, 256, 0, c.stream>>>(N, ks, v.x, v.ph, v.sh, v.s1, v.t, v.r1, v.r0, p3);
-    conv_finalize<<<1, FIN_THREADS, 0, c.stream>>>(p3, nbu, ks);
+      spmv_dot2_pc_kernel<T><<<nb, 256, op_lds_bytes(a), c.stream>>>(a, ks3, v.sh, v.s1, v.t, p2);
+    if (fold == Fold::ALL) {
+      xr_fold_kernel<T, true, 2><<<nbu, 256, 0, c.stream>>>(N, p2, nbs, ks3, v.x, v.ph, v.sh, v.s1, v.t, v.r1, v.r0, p3);
+      launch_p_fold<T>(N, p3, nbu, ks, v.r1, v.p1, v.v, v.r0, c.stream);
+      CFD_HIP(hipGetLastError());
+      continue;
+    }
+    launch_omega_finalize(p2, nbs, ks3, c.stream);
+    xr_update_pc_kernel<T><<<nbu, 256, 0, c.stream>>>(N, ks3, v.x, v.ph, v.sh, v.s1, v.t, v.r1, v.r0, p3);
+    launch_conv_finalize(p3, nbu, ks3, ks, c.stream);
     p_update_kernel<T><<<nbu, 256, 0, c.stream>>>(N, ks, v.r1, v.p1, v.v, v.r0);
     CFD_HIP(hipGetLastError());
   }
@@ -1203,7 +1460,7 @@ constexpr int64_t NOALLOC_ROWS = CFD_NOALLOC_MAX_ROWS;
 constexpr int NOALLOC_VECS = 7;  // r0 r1 p1 s1 ap as px1
 constexpr int64_t NOALLOC_PARTIALS = (int64_t)RED_SITES * 3 * RED_MAX_BLOCKS;
 constexpr int64_t NOALLOC_OUT = (int64_t)RED_SITES * 4;
-constexpr int64_t NOALLOC_KS = (sizeof(KrylovScalars) + 255) / 256 * 32;  // doubles, 256-byte multiple
+constexpr int64_t NOALLOC_KS = (2 * sizeof(KrylovScalars) + 255) / 256 * 32;  // doubles, 256-byte multiple
 constexpr int64_t NOALLOC_DOUBLES = NOALLOC_VECS * NOALLOC_ROWS + NOALLOC_PARTIALS + NOALLOC_OUT + NOALLOC_KS;
 static_assert(NOALLOC_PARTIALS % 32 == 0 && NOALLOC_OUT % 32 == 0, "256-byte sections");
 
