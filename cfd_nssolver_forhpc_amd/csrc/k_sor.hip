@@ -204,15 +204,60 @@ __global__ void sorp_setup_kernel(KrylovScalars *ks, double crit, int itmax) {
   ks->relres = 0.0;
 }
 
+// the do-while test of SorPipeLine_seq after a sweep of maximum `residual`
+__device__ inline bool sorp_stops(const KrylovScalars *ks, double residual) {
+  return !(residual > ks->tol) || ks->iters + 1 >= ks->maxit;
+}
+__device__ inline void sorp_advance(const KrylovScalars *in, KrylovScalars *out, double residual) {
+  const bool was = in->done != 0, stops = sorp_stops(in, residual);
+  const int iters = in->iters;
+  const double relres = in->relres;
+  out->tol = in->tol;
+  out->maxit = in->maxit;
+  out->relres = was ? relres : residual;
+  out->iters = was ? iters : iters + 1;
+  out->done = was || stops;
+}
+
+// A sweep is two dependent launches of a few microseconds on a small grid, and
+// was three: the one-block kernel that combines the maxima takes as long as a
+// colour (96x48x24: 3.6 us beside 2 x 4.3).  With at most SORP_FOLD blocks the
+// next sweep's first colour combines them in every block instead (a maximum
+// does not depend on the order), so the launch is gone: F1 -> F2 us a sweep.
+// The state then has two copies, read from one and written to the other.
+constexpr int SORP_FOLD = 1024;
+
 // one colour of a sweep; partial max |pNEW - p| per block
 // wrapz: periodic z, the z neighbours of the first and last planes are the
 // live pressure across the seam (not ghosts), which keeps the red-black
 // colouring valid for an even nz
+// FOLD: the sweep before this one left its maxima in prev[0 .. 2 RED_MAX_BLOCKS);
+// ks is the state before it, next (block 0's) the state after it
+template <bool FOLD>
 __global__ void __launch_bounds__(256) sorp_sweep_kernel(DevGrid g, int colour, double omega, int wrapz,
                                                          const double *__restrict__ cf6, double *__restrict__ p,
-                                                         const KrylovScalars *__restrict__ ks, double *part) {
+                                                         const KrylovScalars *__restrict__ ks, double *part,
+                                                         const double *__restrict__ prev, KrylovScalars *next) {
 #pragma clang fp contract(off)
-  if (ks->done) return;
+  if (FOLD) {
+    __shared__ double lds[4];
+    double m = 0.0;  // the maxima are not negative
+    if (!ks->done) {
+#pragma unroll
+      for (int u = 0; u < SORP_FOLD / 256; ++u) {
+        const int b = min((int)threadIdx.x + u * 256, (int)gridDim.x - 1);
+        m = fmax(m, fmax(prev[b], prev[RED_MAX_BLOCKS + b]));
+      }
+    }
+    m = wave_max(m);
+    if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = m;
+    __syncthreads();
+    const double residual = fmax(fmax(lds[0], lds[1]), fmax(lds[2], lds[3]));
+    if (blockIdx.x == 0 && threadIdx.x == 0) sorp_advance(ks, next, residual);
+    if (ks->done || sorp_stops(ks, residual)) return;
+  } else if (ks->done) {
+    return;
+  }
   double mx[1] = {0.0};
   const int nzh = (g.nzc + 1) / 2;
   const int64_t cnt = (int64_t)g.nxc * g.nyc * nzh;
@@ -247,19 +292,13 @@ __global__ void __launch_bounds__(256) sorp_sweep_kernel(DevGrid g, int colour, 
   block_partials<1, true>(mx, part);
 }
 
-// the sweep's maximum over both colours and the do-while test of SorPipeLine_seq
-__global__ void __launch_bounds__(FIN_THREADS) sorp_finalize_kernel(const double *part0, const double *part1,
-                                                                    int nblk, KrylovScalars *ks) {
-  if (ks->done) return;
+// the sweep's maximum over both colours
+__global__ void __launch_bounds__(FIN_THREADS) sorp_finalize_kernel(const double *part, int nblk,
+                                                                    const KrylovScalars *in, KrylovScalars *out) {
   double a[1], b[1];
-  combine_partials<1, true>(part0, nblk, a);
-  combine_partials<1, true>(part1, nblk, b);
-  if (threadIdx.x == 0) {
-    const double residual = fmax(a[0], b[0]);
-    ks->relres = residual;
-    ks->iters += 1;
-    if (!(residual > ks->tol) || ks->iters >= ks->maxit) ks->done = 1;
-  }
+  combine_partials<1, true>(part, nblk, a);
+  combine_partials<1, true>(part + RED_MAX_BLOCKS, nblk, b);
+  if (threadIdx.x == 0) sorp_advance(in, out, fmax(a[0], b[0]));
 }
 
 }  // namespace
@@ -274,15 +313,30 @@ int sor_pipeline_solve(Ctx &c, double omega, double crit, int itmax, int *iters,
   CFD_HIP(hipGetLastError());
   const int64_t cnt = (int64_t)g.nxc * g.nyc * ((g.nzc + 1) / 2);
   const int nb = blocks_for(cnt, 256, RED_MAX_BLOCKS);
-  double *part0 = red_part_host(c, RS_SPMV_DOT), *part1 = red_part_host(c, RS_SPMV_DOT2);
+  // a sweep's maxima, the first colour's and the second's; sweeps take turns (a
+  // block may still read the last one's)
+  double *part[2] = {red_part_host(c, RS_SPMV_DOT), red_part_host(c, RS_SPMV_DOT2)};
+  const bool fold = nb <= SORP_FOLD;
   int batch = 4, done_sweeps = 0;
   double prev = -1.0;
   int prev_it = 0;
   for (;;) {
+    KrylovScalars *st = c.ks;  // the state before the sweep, once it is known
     for (int s = 0; s < batch; ++s) {
-      sorp_sweep_kernel<<<nb, 256, 0, c.stream>>>(g, 0, omega, c.prm.periodic_z, cf6, c.f[CFD_P], c.ks, part0);
-      sorp_sweep_kernel<<<nb, 256, 0, c.stream>>>(g, 1, omega, c.prm.periodic_z, cf6, c.f[CFD_P], c.ks, part1);
-      sorp_finalize_kernel<<<1, FIN_THREADS, 0, c.stream>>>(part0, part1, nb, c.ks);
+      double *mx = part[s & 1];
+      if (s > 0 && fold) {
+        KrylovScalars *before = st;
+        st = before == c.ks ? c.ks + 1 : c.ks;
+        sorp_sweep_kernel<true><<<nb, 256, 0, c.stream>>>(g, 0, omega, c.prm.periodic_z, cf6, c.f[CFD_P], before, mx,
+                                                          part[(s - 1) & 1], st);
+      } else {
+        sorp_sweep_kernel<false><<<nb, 256, 0, c.stream>>>(g, 0, omega, c.prm.periodic_z, cf6, c.f[CFD_P], st, mx,
+                                                           nullptr, nullptr);
+      }
+      sorp_sweep_kernel<false><<<nb, 256, 0, c.stream>>>(g, 1, omega, c.prm.periodic_z, cf6, c.f[CFD_P], st,
+                                                         mx + RED_MAX_BLOCKS, nullptr, nullptr);
+      if (!fold || s == batch - 1)
+        sorp_finalize_kernel<<<1, FIN_THREADS, 0, c.stream>>>(mx, nb, st, c.ks);
     }
     CFD_HIP(hipGetLastError());
     CFD_HIP(hipMemcpyAsync(c.hks, c.ks, sizeof(KrylovScalars), hipMemcpyDeviceToHost, c.stream));
