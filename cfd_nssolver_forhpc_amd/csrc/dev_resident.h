@@ -9,13 +9,7 @@
 // needs (its own rows' and its halo's) in LDS.  What crosses workgroups per
 // iteration is two halos (p and s) and three sums.
 //
-// Values cross workgroups as self-validating words: a double travels as two
-// 64-bit words, each half the value and the 32-bit number of the exchange
-// (ll_store / ll_load).  Each word is one relaxed agent-scope atomic, so a
-// reader that finds the number it waits for has the value, with no fence and
-// no flag to read first; an exchange costs one store and one load to the
-// level the XCDs share.  A buffer is rewritten only after a sum that every
-// workgroup contributed to after its reads of the buffer.
+// Values cross workgroups as self-validating words (dev_exchange.h).
 //
 // The sums are those of the launch path bit for bit.  Its x / r update gives
 // a thread the rows v, v + S, v + 2S, v + 3S (S: the threads of its grid, a
@@ -33,6 +27,7 @@
 #pragma once
 
 #include "dev_common.h"
+#include "dev_exchange.h"
 #include "dev_spmv.h"
 
 namespace cfd {
@@ -52,8 +47,6 @@ static_assert(RES_OWN + RES_HALO < 65536, "16-bit LDS positions");
 // words of one exchanged sum: 5 entries a slot (resident_put), two words each
 constexpr int RES_RED_WORDS = RES_SLOTS * 5 * 2;
 
-enum { RES_PENDING = 0, RES_GO = 1, RES_ABORT = 2, RES_STUCK = 3 };
-
 struct ResArgs {
   int64_t N, S;               // rows; rows between a thread's rows (256 nbx)
   int nbx, nblk;              // blocks of the launch path's x / r update, workgroups here
@@ -67,47 +60,6 @@ struct ResArgs {
   int chunk;                  // iterations this launch runs at most
 };
 
-// Element q of an array of 8-byte elements by its 32-bit byte offset (the
-// arrays are at most 4 MB), so that an access is a scalar base and one
-// 32-bit register instead of a 64-bit address held per array and row.
-template <typename T>
-__device__ inline T *at32(T *p, unsigned q) {
-  static_assert(sizeof(T) == 8, "8-byte elements");
-  return reinterpret_cast<T *>(reinterpret_cast<char *>(p) + (q << 3));
-}
-template <typename T>
-__device__ inline const T *at32(const T *p, unsigned q) {
-  return reinterpret_cast<const T *>(reinterpret_cast<const char *>(p) + (q << 3));
-}
-
-__device__ inline uint64_t ll_get(const uint64_t *p) {
-  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-__device__ inline void ll_store(uint64_t *p0, uint64_t *p1, double v, unsigned epoch) {
-  const uint64_t b = (uint64_t)__double_as_longlong(v), e = (uint64_t)epoch << 32;
-  __hip_atomic_store(p0, e | (b & 0xffffffffu), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-  __hip_atomic_store(p1, e | (b >> 32), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-
-__device__ inline double ll_value(uint64_t w0, uint64_t w1) {
-  return __longlong_as_double((long long)((w0 & 0xffffffffu) | (w1 << 32)));
-}
-
-// Once every workgroup is known to be resident, each wait ends when the
-// others reach the same point, microseconds later.  No wave polls before
-// every wave of its workgroup has issued the words others wait for (a barrier
-// stands between): the memory pipeline takes older waves first, and waves
-// that poll scattered words keep it full, so a younger wave's stores could
-// wait for ever behind polls that wait for them.  The bound (some seconds of
-// polling, counted in polls so that a preempted kernel does not run into it)
-// is there so that the kernel ends whatever happens, with RES_STUCK for the
-// host to report.
-constexpr unsigned RES_SPIN = 1u << 22;
-// polls of the arrival handshake before a workgroup gives the launch up
-// (tens of milliseconds: the CUs are held by other kernels)
-constexpr unsigned RES_ARRIVE_SPIN = 1u << 15;
-
 struct ResLds {
   double vec[RES_OWN + RES_HALO];          // the gathered vector: own rows (m 512 + t), halo
   int32_t hcol[RES_HALO];                  // global column of a halo entry
@@ -116,39 +68,6 @@ struct ResLds {
   double one[2][4][2];                     // block sums of a lone workgroup (at most 4 slots)
   int nhalo, state, stuck;
 };
-
-// Loads U pairs of words at a time until each carries the epoch: get(u) is
-// the position of the u-th pair in w0 / w1 (RES_NONE: none), put(u, v) takes
-// its value.  False when the bound was reached.
-constexpr unsigned RES_NONE = ~0u;
-template <int U, typename G, typename P>
-__device__ inline bool ll_fetch(const uint64_t *p0, const uint64_t *p1, unsigned epoch, G get, P put) {
-  unsigned at[U];
-#pragma unroll
-  for (int u = 0; u < U; ++u) at[u] = get(u);
-#pragma unroll 1
-  for (unsigned spin = 0; spin < RES_SPIN; ++spin) {
-    uint64_t w0[U], w1[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const unsigned q = at[u] != RES_NONE ? at[u] : 0;  // position 0 exists; its words are not looked at
-      w0[u] = ll_get(at32(p0, q));
-      w1[u] = ll_get(at32(p1, q));
-    }
-    unsigned bad = 0;
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const unsigned d = ((unsigned)(w0[u] >> 32) ^ epoch) | ((unsigned)(w1[u] >> 32) ^ epoch);
-      bad |= at[u] != RES_NONE ? d : 0u;
-    }
-    if (bad == 0) {
-#pragma unroll
-      for (int u = 0; u < U; ++u) put(u, at[u] != RES_NONE, ll_value(w0[u], w1[u]));
-      return true;
-    }
-  }
-  return false;
-}
 
 // The workgroup's halo of the vector exchanged in ll, into its LDS entries.
 __device__ inline void resident_halo(ResLds &L, const ResArgs &a, unsigned epoch) {
@@ -287,31 +206,6 @@ __device__ inline void resident_total(const ResArgs &a, ResLds &L, const uint64_
   }
 }
 
-// Every workgroup resident, or none goes on: arrivals are counted, the last
-// one sets RES_GO, and a workgroup that waits too long (other kernels hold the
-// CUs) sets RES_ABORT instead; the first of the two to be set stands for all.
-// A halo that does not fit (a matrix that is no stencil) aborts the same way.
-__device__ inline int resident_arrive(const ResArgs &a, ResLds &L, bool fits) {
-  if (threadIdx.x == 0) {
-    unsigned *const st = reinterpret_cast<unsigned *>(&a.ks->pad1);
-    if (!fits) atomicCAS(st, (unsigned)RES_PENDING, (unsigned)RES_ABORT);
-    if (atomicAdd(reinterpret_cast<unsigned *>(&a.ks->pad0), 1u) + 1u == (unsigned)a.nblk)
-      atomicCAS(st, (unsigned)RES_PENDING, (unsigned)RES_GO);
-    unsigned s = RES_PENDING;
-    for (unsigned spin = 0; spin < RES_ARRIVE_SPIN; ++spin) {
-      s = __hip_atomic_load(st, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      if (s != RES_PENDING) break;
-    }
-    if (s == RES_PENDING) {
-      s = atomicCAS(st, (unsigned)RES_PENDING, (unsigned)RES_ABORT);
-      if (s == RES_PENDING) s = RES_ABORT;
-    }
-    L.state = (int)s;
-  }
-  __syncthreads();
-  return L.state;
-}
-
 // y = A (the vector in L.vec) on the thread's rows: ell_row's FMA chain.
 // pos holds two 16-bit positions a register; the empty asm keeps their
 // unpacked forms from being hoisted out of the iteration (28 registers).
@@ -395,7 +289,7 @@ __global__ void __launch_bounds__(RES_THREADS) bicg_resident_kernel(ResArgs a) {
     p[m] = own(m) ? *at32(a.p1, row) : 0.0;
   }
   fits = __syncthreads_and(fits);
-  if (resident_arrive(a, L, fits) != RES_GO) return;
+  if (resident_arrive(a.ks, a.nblk, &L.state, fits) != RES_GO) return;
   const int nslot = (int)((a.N + 511) / 512);
   double alpha = 0.0, omega = 0.0, beta = 0.0, pre_rho = 0.0, rnorm = 0.0, relres = 0.0;
   int done = 0, hit = 0, restart = 0;

@@ -719,31 +719,6 @@ hipError_t launch_iters(Ctx &c, const OpArgs &a, const Vecs<T> &v, KrylovScalars
   return hipGetLastError();
 }
 
-// Workgroups of resident solves in flight on each device.  They hold a CU
-// each, so a solve that would not find its CUs free takes the launch path.
-constexpr int MAX_DEVICES = 64;
-std::atomic<int> g_resident[MAX_DEVICES];
-
-struct ResidentSlots {
-  std::atomic<int> *n = nullptr;
-  int blocks = 0;
-  bool take(int device, int want) {
-    if (device < 0 || device >= MAX_DEVICES) return false;
-    int cus = 0;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) return false;
-    n = &g_resident[device];
-    if (n->fetch_add(want) + want > cus) {
-      n->fetch_sub(want);
-      return false;
-    }
-    blocks = want;
-    return true;
-  }
-  ~ResidentSlots() {
-    if (blocks) n->fetch_sub(blocks);
-  }
-};
-
 // The iterations of an FP64 solve on the ELL operator in one launch
 // (dev_resident.h) where its rows fit the chip's registers; the state after
 // init_kernel is the launch path's and so is every result, bit for bit.

@@ -11,6 +11,7 @@
 #include <cmath>
 
 #include "dev_common.h"
+#include "dev_exchange.h"
 #include "dev_spmv.h"
 
 namespace cfd {
@@ -221,10 +222,11 @@ __device__ inline void sorp_advance(const KrylovScalars *in, KrylovScalars *out,
 
 // A sweep is two dependent launches of a few microseconds on a small grid, and
 // was three: the one-block kernel that combines the maxima takes as long as a
-// colour (96x48x24: 3.6 us beside 2 x 4.3).  With at most SORP_FOLD blocks the
-// next sweep's first colour combines them in every block instead (a maximum
-// does not depend on the order), so the launch is gone: F1 -> F2 us a sweep.
-// The state then has two copies, read from one and written to the other.
+// colour (3.6 us beside 2 x 4.3).  With at most SORP_FOLD blocks the next
+// sweep's first colour combines them in every block instead (a maximum does
+// not depend on the order), so the launch is gone: 12.1 -> 9.9 us a sweep at
+// 8x8x1100.  The state then has two copies, read from one and written to the
+// other.
 constexpr int SORP_FOLD = 1024;
 
 // one colour of a sweep; partial max |pNEW - p| per block
@@ -301,6 +303,266 @@ __global__ void __launch_bounds__(FIN_THREADS) sorp_finalize_kernel(const double
   if (threadIdx.x == 0) sorp_advance(in, out, fmax(a[0], b[0]));
 }
 
+// ---- all the sweeps of a small grid in one launch ---------------------------
+// A colour of a small grid is a launch of 4.3 us whatever its size, most of it
+// launch, drain and the thirteen divisions of its coefficients.  Here every
+// workgroup keeps its cells for all the sweeps: a thread owns the two cells
+// of a pair in z (one of each colour), their coefficients in registers, their
+// pressure in LDS beside that of the halo and of the ghosts, which do
+// not change.  After a colour a workgroup leaves its new values for the others
+// and waits for those of its halo (dev_exchange.h).  The sweep's maximum
+// travels while the next sweep's first colour runs; if it ends the solve, that
+// colour is dropped.  Every cell's update is sorp_sweep_kernel's, operation for
+// operation, and a maximum has no order, so the results are the same bits.
+// A value is rewritten two colours later, after the neighbours' values of the
+// colour between, which they leave after their reads; a maximum two sweeps
+// later, after every workgroup's next one, left after its reads.
+// Bound by the two exchanges a sweep.  us a sweep, launches -> here: 512 cells
+// 11.2 -> 1.0 (one workgroup), 4096 11.8 -> 2.5, 110592 12.7 -> 4.4, 262144
+// 13.3 -> 5.8.  Two pairs a thread reach 524288 cells, but take 17.9 us there
+// against the launches' 15.7.
+constexpr int SORR_THREADS = 512, SORR_BLOCKS = 256;  // one workgroup a CU, all resident
+
+struct SorLds {
+  static constexpr int OWN = SORR_THREADS;      // pairs
+  static constexpr int HALO = OWN * 2 + 512;    // cells of a colour: x neighbours of every pair, two z lines and more
+  static constexpr int GHOST = 3072;
+  double p[2 * OWN + 2 * HALO + GHOST];         // own cells (parity of k), halo (colour), ghosts
+  int32_t hrow[2][HALO];
+  double wmax[SORR_THREADS / 64], tot[SORR_BLOCKS / 64];
+  int nhalo[2], nghost, state, stuck;
+};
+
+struct SorArgs {
+  uint64_t *ll0, *ll1;  // the two words of each cell
+  uint64_t *mx;         // maxima: [sweep parity][word][workgroup]
+  KrylovScalars *ks;    // pad0: arrivals, pad1: RES_* state
+  int nblk, chunk;      // chunk: sweeps this launch runs at most
+};
+
+__global__ void __launch_bounds__(SORR_THREADS) sorp_resident_kernel(DevGrid g, double omega, int wrapz,
+                                                                     const double *__restrict__ cf6,
+                                                                     double *__restrict__ p, SorArgs a) {
+#pragma clang fp contract(off)
+  __shared__ SorLds L;
+  constexpr int OWN = SorLds::OWN, HALO = SorLds::HALO, GHOST = SorLds::GHOST;
+  const int tid = threadIdx.x, blk = blockIdx.x;
+  const int nxc = g.nxc, nyc = g.nyc, nzc = g.nzc, nzh = (nzc + 1) / 2;
+  const int npair = nxc * nyc * nzh;
+  if (a.ks->done) return;  // uniform over the grid
+  const double tol = a.ks->tol;
+  const int maxit = a.ks->maxit;
+  int iters = a.ks->iters;
+  if (tid < 2) L.nhalo[tid] = 0;
+  if (tid == 2) L.nghost = L.stuck = 0;
+  __syncthreads();
+  const double *__restrict__ Dx = g.Dx, *__restrict__ Dy = g.Dy, *__restrict__ Dz = g.Dz;
+  const double *__restrict__ Dxs = g.Dxs, *__restrict__ Dys = g.Dys, *__restrict__ Dzs = g.Dzs;
+  double cf[2][6], rhs[2], cf7[2], cur[2];
+  unsigned pos[2][3], row[2], at[2];
+  bool own[2];
+  int fits = 1;
+  {
+    const int t = blk * OWN + tid, kh = t % nzh, rest = t / nzh, j0 = rest % nyc, i0 = rest / nyc;
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+      const int k0 = 2 * kh + ((i0 + j0 + c) & 1);
+      own[c] = t < npair && k0 < nzc;
+      const int ic_ = own[c] ? i0 : 0, jc = own[c] ? j0 : 0, kc = own[c] ? k0 : 0;
+      const int i = ic_ + GC, j = jc + GC, k = kc + GC;
+      const double cf0 = Dy[j] * Dz[k] / Dxs[i], cf1 = Dy[j] * Dz[k] / Dxs[i - 1];
+      const double cf2 = Dx[i] * Dz[k] / Dys[j], cf3 = Dx[i] * Dz[k] / Dys[j - 1];
+      const double cf4 = Dx[i] * Dy[j] / Dzs[k], cf5 = Dx[i] * Dy[j] / Dzs[k - 1];
+      const double coef = Dy[j] * Dz[k] / Dxs[i] + Dy[j] * Dz[k] / Dxs[i - 1] + Dx[i] * Dz[k] / Dys[j] +
+                          Dx[i] * Dz[k] / Dys[j - 1] + Dx[i] * Dy[j] / Dzs[k] + Dx[i] * Dy[j] / Dzs[k - 1];
+      cf[c][0] = cf0, cf[c][1] = cf1, cf[c][2] = cf2, cf[c][3] = cf3, cf[c][4] = cf4, cf[c][5] = cf5;
+      cf7[c] = -1.0 / coef;
+      row[c] = (unsigned)((ic_ * nyc + jc) * nzc + kc);
+      rhs[c] = cf6[row[c]];
+      cur[c] = p[icel(g, i, j, k)];
+      at[c] = (unsigned)((kc & 1) * OWN + tid);
+      if (own[c]) L.p[at[c]] = cur[c];
+      unsigned ps[6];
+#pragma unroll
+      for (int d = 0; d < 6; ++d) {  // +x, -x, +y, -y, +z, -z
+        int in = ic_, jn = jc, kn = kc;
+        if (d < 2) in += d == 0 ? 1 : -1;
+        else if (d < 4) jn += d == 2 ? 1 : -1;
+        else kn += d == 4 ? 1 : -1;
+        if (wrapz) kn = kn == nzc ? 0 : kn < 0 ? nzc - 1 : kn;
+        unsigned at_n = 0;
+        if (own[c]) {
+          const double v = p[icel(g, in + GC, jn + GC, kn + GC)];
+          if (in < 0 || in >= nxc || jn < 0 || jn >= nyc || kn < 0 || kn >= nzc) {
+            const int e = atomicAdd(&L.nghost, 1);
+            at_n = 2 * OWN + 2 * HALO + min(e, GHOST - 1);
+            if (e >= GHOST) fits = 0;
+            else L.p[at_n] = v;
+          } else {
+            const int tn = (in * nyc + jn) * nzh + (kn >> 1);
+            if (tn / OWN == blk) {
+              at_n = (kn & 1) * OWN + tn % OWN;
+            } else {
+              const int e = atomicAdd(&L.nhalo[1 - c], 1);
+              at_n = 2 * OWN + (1 - c) * HALO + min(e, HALO - 1);
+              if (e >= HALO) {
+                fits = 0;
+              } else {
+                L.hrow[1 - c][e] = (in * nyc + jn) * nzc + kn;
+                L.p[at_n] = v;
+              }
+            }
+          }
+        }
+        ps[d] = at_n;
+      }
+#pragma unroll
+      for (int d = 0; d < 3; ++d) pos[c][d] = ps[2 * d] | ps[2 * d + 1] << 16;
+    }
+  }
+  fits = __syncthreads_and(fits);
+  if (resident_arrive(a.ks, a.nblk, &L.state, fits) != RES_GO) return;
+
+  double mx = 0.0, old = 0.0;
+  // colour c of the sweep with exchange number epoch (1, 2, 3, ..)
+  auto colour = [&](auto cc, unsigned epoch) __attribute__((always_inline)) {
+#pragma clang fp contract(off)
+    constexpr int c = decltype(cc)::value;
+    {
+      double n[6];
+#pragma unroll
+      for (int d = 0; d < 6; ++d) n[d] = L.p[(d & 1) ? pos[c][d >> 1] >> 16 : pos[c][d >> 1] & 0xffffu];
+      const double *f = cf[c];
+      const double pc = cur[c];
+      const double pNEW = (-n[0] * f[0] - n[1] * f[1] - n[2] * f[2] - n[3] * f[3] - n[4] * f[4] - n[5] * f[5] +
+                           rhs[c]) * cf7[c];
+      if (c == 0) old = pc;
+      if (own[c]) {
+        mx = fmax(mx, fabs(pNEW - pc));
+        cur[c] = pc + omega * (pNEW - pc);
+        L.p[at[c]] = cur[c];
+        if (a.nblk > 1) ll_store(at32(a.ll0, row[c]), at32(a.ll1, row[c]), cur[c], epoch);
+      }
+    }
+  };
+  // the halo's cells of colour c with that number, by the threads from `busy` on
+  auto halo = [&](int c, unsigned epoch, int busy) __attribute__((always_inline)) {
+    const int nh = L.nhalo[c], step = SORR_THREADS - busy;
+    if (tid < busy) return;
+    for (int e0 = tid - busy; e0 < nh; e0 += 4 * step) {
+      const bool ok = ll_fetch<4>(
+          a.ll0, a.ll1, epoch, [&](int u) { return e0 + u * step < nh ? (unsigned)L.hrow[c][e0 + u * step] : RES_NONE; },
+          [&](int u, bool have, double v) {
+            if (have) L.p[2 * OWN + c * HALO + e0 + u * step] = v;
+          });
+      if (!ok) L.stuck = 1;
+    }
+  };
+  const int busy = (a.nblk + 63) / 64 * 64;  // threads that wait for the maxima, at most half
+  double residual = a.ks->relres;
+  int done = 0;
+  for (int s = 0;; ++s) {
+    const unsigned h = 2u * (unsigned)s;
+    if (s > 0) halo(1, h, 0);
+    __syncthreads();
+    colour(std::integral_constant<int, 0>(), h + 1);
+    __syncthreads();  // every wave has issued its words (RES_SPIN)
+    if (a.nblk > 1) {
+      if (s > 0 && tid < busy) {
+        double v = 0.0;
+        const uint64_t *w = a.mx + ((s - 1) & 1) * 2 * SORR_BLOCKS;
+        const bool ok = ll_fetch<1>(
+            w, w + SORR_BLOCKS, (unsigned)s, [&](int) { return tid < a.nblk ? (unsigned)tid : RES_NONE; },
+            [&](int, bool have, double x) { v = have ? x : 0.0; });
+        if (!ok) L.stuck = 1;
+        v = wave_max(v);
+        if ((tid & 63) == 0) L.tot[tid >> 6] = v;
+      }
+      halo(0, h + 1, s > 0 ? busy : 0);
+    } else if (s > 0 && tid == 0) {
+      double v = L.wmax[0];
+      for (int w = 1; w < SORR_THREADS / 64; ++w) v = fmax(v, L.wmax[w]);
+      L.tot[0] = v;
+    }
+    __syncthreads();
+    if (L.stuck) {  // a wait reached its bound
+      if (tid == 0) __hip_atomic_store(&a.ks->pad1, (int)RES_STUCK, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      return;
+    }
+    if (s > 0) {
+      residual = L.tot[0];
+      for (int w = 1; w < busy / 64; ++w) residual = fmax(residual, L.tot[w]);
+      iters += 1;
+      done = !(residual > tol) || iters >= maxit;
+      if (done || s >= a.chunk) {  // without the colour just done
+        cur[0] = old;
+        break;
+      }
+    }
+    colour(std::integral_constant<int, 1>(), h + 2);
+    const double m = wave_max(mx);
+    mx = 0.0;
+    if ((tid & 63) == 0) L.wmax[tid >> 6] = m;
+    __syncthreads();
+    if (tid == 0 && a.nblk > 1) {
+      double v = L.wmax[0];
+#pragma unroll
+      for (int w = 1; w < SORR_THREADS / 64; ++w) v = fmax(v, L.wmax[w]);
+      uint64_t *w = a.mx + (s & 1) * 2 * SORR_BLOCKS + blk;
+      ll_store(w, w + SORR_BLOCKS, v, (unsigned)s + 1);
+    }
+  }
+#pragma unroll
+  for (int c = 0; c < 2; ++c)
+    if (own[c]) {
+      const int r = (int)row[c], kc = r % nzc, rest = r / nzc;
+      p[icel(g, rest / nyc + GC, rest % nyc + GC, kc + GC)] = cur[c];
+    }
+  if (blk == 0 && tid == 0) {
+    a.ks->relres = residual;
+    a.ks->iters = iters;
+    a.ks->done = done;
+  }
+}
+
+__global__ void __launch_bounds__(256) sorp_clear_kernel(int64_t n, SorArgs a) {
+  const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (q < n) a.ll0[q] = a.ll1[q] = 0;
+  if (q < 4 * SORR_BLOCKS) a.mx[q] = 0;
+  if (q == 0) a.ks->pad0 = a.ks->pad1 = 0;
+}
+
+// *solved is false when the launches have to do it: more cells than the
+// workgroups hold (262144 at an even nz), a halo or ghosts that LDS does not
+// hold, or CUs that are taken.
+int sorp_resident(Ctx &c, double omega, const double *cf6, bool *solved) {
+  *solved = false;
+  const DevGrid &g = c.g;
+  const int64_t npair = (int64_t)g.nxc * g.nyc * ((g.nzc + 1) / 2);
+  if (npair > SORR_THREADS * SORR_BLOCKS) return CFD_OK;
+  SorArgs a;
+  a.ll0 = reinterpret_cast<uint64_t *>(c.s1);  // the Krylov solver's vectors
+  a.ll1 = reinterpret_cast<uint64_t *>(c.ap);
+  a.mx = reinterpret_cast<uint64_t *>(red_part_host(c, RS_SPMV_DOT));
+  a.ks = c.ks;
+  a.nblk = (int)((npair + SORR_THREADS - 1) / SORR_THREADS);
+  a.chunk = 4096;  // bounds one launch to some tens of milliseconds
+  ResidentSlots slots;
+  if (!slots.take(c.device, a.nblk)) return CFD_OK;
+  for (;;) {
+    sorp_clear_kernel<<<blocks_for(std::max<int64_t>(g.N, 4 * SORR_BLOCKS), 256, 1 << 30), 256, 0, c.stream>>>(g.N, a);
+    sorp_resident_kernel<<<a.nblk, SORR_THREADS, 0, c.stream>>>(g, omega, c.prm.periodic_z, cf6, c.f[CFD_P], a);
+    CFD_HIP(hipGetLastError());
+    CFD_HIP(hipMemcpyAsync(c.hks, c.ks, sizeof(KrylovScalars), hipMemcpyDeviceToHost, c.stream));
+    CFD_HIP(hipStreamSynchronize(c.stream));
+    if (c.hks->pad1 == RES_STUCK) return fail(CFD_ERR_RUNTIME, "resident SorPipeLine: a workgroup stopped answering");
+    if (c.hks->pad1 != RES_GO) return CFD_OK;
+    if (c.hks->done) break;
+  }
+  *solved = true;
+  return CFD_OK;
+}
+
 }  // namespace
 
 int sor_pipeline_solve(Ctx &c, double omega, double crit, int itmax, int *iters, double *error) {
@@ -311,6 +573,13 @@ int sor_pipeline_solve(Ctx &c, double omega, double crit, int itmax, int *iters,
                                                                       c.f[CFD_T1_V], c.f[CFD_T1_W], cf6);
   sorp_setup_kernel<<<1, 1, 0, c.stream>>>(c.ks, crit, itmax);
   CFD_HIP(hipGetLastError());
+  bool solved = false;
+  if (int rc = sorp_resident(c, omega, cf6, &solved)) return rc;
+  if (solved) {
+    *iters = c.hks->iters - 1;
+    *error = c.hks->relres;
+    return CFD_OK;
+  }
   const int64_t cnt = (int64_t)g.nxc * g.nyc * ((g.nzc + 1) / 2);
   const int nb = blocks_for(cnt, 256, RED_MAX_BLOCKS);
   // a sweep's maxima, the first colour's and the second's; sweeps take turns (a
