@@ -109,6 +109,8 @@ struct Ctx {
   // SPE coefficients (xm, xp over nxc; ym, yp over nyc; zm, zp over nzc) and jp
   double *spe_coef = nullptr;
   double *spe_jp = nullptr;
+  int spe_pd[6] = {};  // the boundary conditions that spe_jp was formed with
+  int spe_wrapz = 0;
   // CSR operator (createPressureMatrixCSR): row pointers (N+1), columns,
   // values and its own Jacobi scaling
   int32_t *csr_ptr = nullptr, *csr_col = nullptr;

@@ -58,7 +58,8 @@ struct EllGridPair {
   bool hym, hyp, ha, hb;
 };
 
-__device__ inline EllGridPair ell_grid_pair(const OpArgs &a, uint32_t at) {
+// wrap: the z faces are joined
+__device__ inline EllGridPair ell_grid_pair(const OpArgs &a, uint32_t at, bool wrap) {
   EllGridPair c;
   const uint32_t line = (uint32_t)a.nzc, seam = line - 1;
   c.j = (int)fastdiv(at, a.div_nz);
@@ -66,8 +67,8 @@ __device__ inline EllGridPair ell_grid_pair(const OpArgs &a, uint32_t at) {
   c.hym = c.j != 0;
   c.hyp = c.j != a.nyc - 1;
   const bool first = c.k == 0, last = c.k == a.nzc - 2;
-  c.ha = a.ewrapz || !first;
-  c.hb = a.ewrapz || !last;
+  c.ha = wrap || !first;
+  c.hb = wrap || !last;
   c.oc = at * 8u;
   c.oym = (c.hym ? at - line : at) * 8u;
   c.oyp = (c.hyp ? at + line : at) * 8u;
@@ -76,7 +77,47 @@ __device__ inline EllGridPair ell_grid_pair(const OpArgs &a, uint32_t at) {
   return c;
 }
 
-template <bool YW, bool ZW, bool W, typename F>
+struct SpeCoef {
+  double ym, yp, zm, zp, sym, syp, szm, szp;  // s: what a closed face takes off the diagonal
+};
+
+// spe_row from the coefficients, 1 / jp summed in spe_jp_kernel's order
+template <bool YW, bool ZW>
+__device__ inline double spe_grid_value(const EllGridPlane &e, bool hym, bool hyp, bool hzm, bool hzp, const SpeCoef &q,
+                                        double sxm, double sxp, double xc, double vxm, double vxp, double vym,
+                                        double vyp, double vzm, double vzp) {
+  double d = e.xm + q.ym;
+  d = d + q.zm;
+  d = d + e.xp;
+  d = d + q.yp;
+  d = d + q.zp;
+  d = d - sxm;
+  d = d - sxp;
+  if (!YW) {
+    d = d - q.sym;
+    d = d - q.syp;
+  }
+  if (!ZW) {
+    d = d - q.szm;
+    d = d - q.szp;
+  }
+  const double J = 1.0 / d;
+  double sum = 0.0, t = fma(-e.xm * J, vxm, sum);
+  sum = e.hxm ? t : sum;
+  t = fma(-q.ym * J, vym, sum);
+  sum = YW || hym ? t : sum;
+  t = fma(-q.zm * J, vzm, sum);
+  sum = ZW || hzm ? t : sum;
+  sum += xc;
+  t = fma(-q.zp * J, vzp, sum);
+  sum = ZW || hzp ? t : sum;
+  t = fma(-q.yp * J, vyp, sum);
+  sum = YW || hyp ? t : sum;
+  t = fma(-e.xp * J, vxp, sum);
+  return e.hxp ? t : sum;
+}
+
+template <bool SPE, bool YW, bool ZW, bool W, typename F>
 __device__ __attribute__((always_inline)) inline void ell_grid_march(const OpArgs &a, const EllGridPair &c, int first,
                                                                      int np, const double *__restrict__ x,
                                                                      const double *__restrict__ w, F fn) {
@@ -92,8 +133,8 @@ __device__ __attribute__((always_inline)) inline void ell_grid_march(const OpArg
     va[s] = at_bytes(x + o, c.oa);
     vb[s] = at_bytes(x + o, c.ob);
     if (W) wv[s] = at_bytes2(w + o, c.oc);
-    pxm[s] = a.ecoef[ic];
-    pxp[s] = a.ecoef[a.nxc + ic];
+    pxm[s] = (SPE ? a.coef : a.ecoef)[ic];
+    pxp[s] = (SPE ? a.coef : a.ecoef)[a.nxc + ic];
   };
   below = at_bytes2(x + max(first - 1, 0) * plane, c.oc);
   here = at_bytes2(x + first * plane, c.oc);
@@ -116,10 +157,27 @@ __device__ __attribute__((always_inline)) inline void ell_grid_march(const OpArg
   c0.hz2 = first_z ? c.ha : true;
   c1.hz1 = true;
   c1.hz2 = c.hb;
-  const EllGridCoef q0 = ell_grid_coef(a, c0);
-  EllGridCoef q1 = ell_grid_coef(a, c1);
-  q1.z1 = q1.zm;
-  q1.z2 = q1.zp;
+  EllGridCoef q0, q1;
+  SpeCoef w0, w1;
+  if (SPE) {
+    const double *ym = a.coef + 2 * a.nxc, *yp = ym + a.nyc, *zm = yp + a.nyc, *zp = zm + a.nzc;
+    w0.ym = w1.ym = ym[jl];
+    w0.yp = w1.yp = yp[jl];
+    w0.zm = zm[kl];
+    w0.zp = zp[kl];
+    w1.zm = zm[kl + 1];
+    w1.zp = zp[kl + 1];
+    w0.sym = w1.sym = jl == 0 && !a.spd[2] ? w0.ym : 0.0;
+    w0.syp = w1.syp = jl == a.nyc - 1 && !a.spd[3] ? w0.yp : 0.0;
+    w0.szm = kl == 0 && !a.spd[4] && !a.swrapz ? w0.zm : 0.0;
+    w1.szp = kl + 1 == a.nzc - 1 && !a.spd[5] && !a.swrapz ? w1.zp : 0.0;
+    w0.szp = w1.szm = 0.0;
+  } else {
+    q0 = ell_grid_coef(a, c0);
+    q1 = ell_grid_coef(a, c1);
+    q1.z1 = q1.zm;
+    q1.z2 = q1.zp;
+  }
 #pragma unroll 1
   for (int m = 0; m < np; m += R) {
 #pragma unroll
@@ -131,13 +189,21 @@ __device__ __attribute__((always_inline)) inline void ell_grid_march(const OpArg
       e.xp = pxp[s];
       e.hxm = i != 0;
       e.hxp = i != a.nxc - 1;
-      e.aa = 0.0;
-      if (!e.hxm && !a.epd[0]) e.aa = -e.xm;
-      if (!e.hxp && !a.epd[1]) e.aa = -e.xp;
-      const double z1 = first_z ? here.y : va[s], z2 = first_z ? va[s] : here.y;
       double2v y;
-      y.x = ell_grid_value<YW, ZW>(e, c0, q0, here.x, below.x, above.x, vym[s].x, vyp[s].x, z1, z2, xlast);
-      y.y = ell_grid_value<YW, ZW>(e, c1, q1, here.y, below.y, above.y, vym[s].y, vyp[s].y, here.x, vb[s], xlast);
+      if (SPE) {
+        const double sxm = !e.hxm && !a.spd[0] ? e.xm : 0.0, sxp = !e.hxp && !a.spd[1] ? e.xp : 0.0;
+        y.x = spe_grid_value<YW, ZW>(e, c.hym, c.hyp, c.ha, true, w0, sxm, sxp, here.x, below.x, above.x, vym[s].x,
+                                     vyp[s].x, va[s], here.y);
+        y.y = spe_grid_value<YW, ZW>(e, c.hym, c.hyp, true, c.hb, w1, sxm, sxp, here.y, below.y, above.y, vym[s].y,
+                                     vyp[s].y, here.x, vb[s]);
+      } else {
+        e.aa = 0.0;
+        if (!e.hxm && !a.epd[0]) e.aa = -e.xm;
+        if (!e.hxp && !a.epd[1]) e.aa = -e.xp;
+        const double z1 = first_z ? here.y : va[s], z2 = first_z ? va[s] : here.y;
+        y.x = ell_grid_value<YW, ZW>(e, c0, q0, here.x, below.x, above.x, vym[s].x, vyp[s].x, z1, z2, xlast);
+        y.y = ell_grid_value<YW, ZW>(e, c1, q1, here.y, below.y, above.y, vym[s].y, vyp[s].y, here.x, vb[s], xlast);
+      }
       fn(m + s, y, here, wv[s]);
       __builtin_amdgcn_sched_barrier(0);
       below = here;
@@ -175,7 +241,7 @@ __global__ void __launch_bounds__(BT / 2, 4) ell_grid_kernel(OpArgs a, int PP, i
   const int blk = (int)blockIdx.x;
   const int tile = blk % ntile, i0 = blk / ntile * M;
   const int tid = (int)threadIdx.x, half = tid >> 5;
-  const EllGridPair c = ell_grid_pair(a, (uint32_t)(tile * BT + 2 * tid));
+  const EllGridPair c = ell_grid_pair(a, (uint32_t)(tile * BT + 2 * tid), a.ewrapz);
   const int np0 = min(M, min(PP, a.nxc) - i0);
   if (MULTI) {
     for (int u = 0; u < M * NV; ++u) own[u][tid] = double2v{0.0, 0.0};
@@ -202,11 +268,11 @@ __global__ void __launch_bounds__(BT / 2, 4) ell_grid_kernel(OpArgs a, int PP, i
     };
     const bool yw = __all(c.hym && c.hyp);  // most waves have no y face, and with joined z faces no z one
     if (yw && a.ewrapz)
-      ell_grid_march<true, true, (DOTS & 1) != 0>(a, c, first, np, x, w, rows);
+      ell_grid_march<false, true, true, (DOTS & 1) != 0>(a, c, first, np, x, w, rows);
     else if (yw)
-      ell_grid_march<true, false, (DOTS & 1) != 0>(a, c, first, np, x, w, rows);
+      ell_grid_march<false, true, false, (DOTS & 1) != 0>(a, c, first, np, x, w, rows);
     else
-      ell_grid_march<false, false, (DOTS & 1) != 0>(a, c, first, np, x, w, rows);
+      ell_grid_march<false, false, false, (DOTS & 1) != 0>(a, c, first, np, x, w, rows);
   }
   if (!DOTS) return;
   if (MULTI) {
@@ -249,6 +315,94 @@ void launch_ell_grid(const OpArgs &a, int pp, const KrylovScalars *ks, const dou
     const int m = std::min(GRID_WALK, std::max(2, (int)((int64_t)pp * ntile / GRID_BLOCKS)));
     ell_grid_kernel<BT, DOTS, false><<<(pp + m - 1) / m * ntile, BT / 2, 0, st>>>(a, pp, m, ks, x, y, w, part);
   }
+}
+
+// The SPE operator the same way, with the dots and partials of the kernels
+// over plane columns (spe_column_rows): a tile is kb x jb columns (k, j) and
+// SPE_PLANES planes, a thread of 128 has two columns beside each other in k,
+// and a block walks G tiles above each other in i without loading their
+// borders again.  jp, 8 B/row, is formed again too.
+// us, K1 alone / an iteration, plane columns -> here: 512x256x64 46.5 / 273 ->
+// 38.9 / 253, 256x128x64 15.4 / 79.7 -> 12.5 / 72.3, 190x210x40 15.0 / 70.3 ->
+// 12.1 / 65.2 (1272 tiles), 200x104x40 10.3 / 44.0 -> 9.6 / 43.9 (650),
+// 64x32x32 5.9 / 23.2 -> 6.0 / 26.0 (64): a tile's planes come one behind the
+// other, so it takes SPE_TILES of them, four blocks a CU, to hide that.  Tiles
+// are walked on (G) as long as SPE_BLOCKS blocks remain.
+constexpr int SPE_WALK = 4, SPE_BLOCKS = 2048, SPE_TILES = 1024;
+
+template <int DOTS>
+__global__ void __launch_bounds__(128, 4) spe_walk_kernel(OpArgs a, SpeTiles T, int G,
+                                                          const KrylovScalars *__restrict__ ks,
+                                                          const double *__restrict__ x, double *__restrict__ y,
+                                                          const double *__restrict__ w, double *part) {
+  if (DOTS && ks->done) return;
+  constexpr int NV = DOTS < 2 ? 1 : 2;
+  __shared__ double red[SPE_WALK][NV][4];
+  const int b = blockIdx.x, tk = b % T.nkt, rest = b / T.nkt, jt = rest % T.njt, ig = rest / T.njt * G;
+  const int tid = (int)threadIdx.x;
+  const int k = tk * T.kb + 2 * tid % T.kb, j = jt * T.jb + 2 * tid / T.kb;
+  const bool ok = k < a.nzc && j < a.nyc;  // nzc is even: both columns or none
+  const EllGridPair c = ell_grid_pair(a, (uint32_t)(min(j, a.nyc - 1) * a.nzc + min(k, a.nzc - 2)), a.wrapz);
+  const int first = ig * SPE_PLANES, np = min(G * SPE_PLANES, a.nxc - first);
+  const int64_t nynz = (int64_t)a.nyc * a.nzc;
+  double *yi = y + first * nynz;
+  double2v acc[NV];
+#pragma unroll
+  for (int u = 0; u < NV; ++u) acc[u] = double2v{0.0, 0.0};
+  auto rows = [&](int m, double2v v, double2v xc, double2v wv) __attribute__((always_inline)) {
+    const double2v d = DOTS == 2 ? xc : wv;
+    if (ok) {
+      ntstore(v, reinterpret_cast<double2v *>(reinterpret_cast<char *>(yi + m * nynz) + c.oc));
+#pragma unroll
+      for (int u = 0; u < NV; ++u) {
+        const double2v f = u ? v : d;
+        if (DOTS) {
+          acc[u].x += v.x * f.x;
+          acc[u].y += v.y * f.y;
+        }
+      }
+    }
+    if (DOTS && (m % SPE_PLANES == SPE_PLANES - 1 || m == np - 1)) {
+#pragma unroll
+      for (int u = 0; u < NV; ++u) {
+        const double s = half_wave_sum(acc[u].x, acc[u].y);
+        if ((tid & 31) == 31) red[m / SPE_PLANES][u][tid >> 5] = s;
+        acc[u] = double2v{0.0, 0.0};
+      }
+    }
+  };
+  const bool yw = __all(c.hym && c.hyp);
+  if (yw && a.wrapz && a.swrapz)
+    ell_grid_march<true, true, true, (DOTS & 1) != 0>(a, c, first, np, x, w, rows);
+  else if (yw)
+    ell_grid_march<true, true, false, (DOTS & 1) != 0>(a, c, first, np, x, w, rows);
+  else
+    ell_grid_march<true, false, false, (DOTS & 1) != 0>(a, c, first, np, x, w, rows);
+  if (!DOTS) return;
+  __syncthreads();
+  const int ng = (np + SPE_PLANES - 1) / SPE_PLANES;
+  if (tid < ng * NV) {
+    const int g = tid / NV, u = tid % NV;
+    double s = red[g][u][0];
+#pragma unroll
+    for (int v = 1; v < 4; ++v) s += red[g][u][v];
+    part[u * RED_MAX_BLOCKS + ((ig + g) * T.njt + jt) * T.nkt + tk] = s;
+  }
+}
+
+// whether the operator's kernels walk pairs of columns
+inline bool spe_pairs(const OpArgs &a, const SpeTiles &T, std::initializer_list<const void *> vecs) {
+  for (const void *p : vecs)
+    if (reinterpret_cast<uintptr_t>(p) % 16 != 0) return false;
+  return a.op == CFD_OP_SPE && T.blocks >= SPE_TILES && a.nzc % 2 == 0 && (int64_t)a.nyc * a.nzc < (int64_t)1 << 29;
+}
+
+template <int DOTS>
+void launch_spe_walk(const OpArgs &a, const SpeTiles &T, const KrylovScalars *ks, const double *x, double *y,
+                     const double *w, double *part, hipStream_t st) {
+  const int64_t col = (int64_t)T.nkt * T.njt;
+  const int G = (int)std::min<int64_t>(SPE_WALK, std::max<int64_t>(1, T.blocks / SPE_BLOCKS));
+  spe_walk_kernel<DOTS><<<(unsigned)(col * ((T.nig + G - 1) / G)), 128, 0, st>>>(a, T, G, ks, x, y, w, part);
 }
 
 }  // namespace

@@ -136,6 +136,8 @@ struct OpArgs {
   const double *ecoef;  // OP_ELL_GRID: axis coefficients, boundary conditions
   int epd[6];
   bool ewrapz;
+  int spd[6];           // SPE: the boundary conditions in jp
+  bool swrapz;
 };
 
 // internal operator id: the ELL operator as cfd_ell_assemble built it, its
@@ -479,6 +481,8 @@ inline OpArgs op_args(const Ctx &c, int op) {
   a.ecoef = c.ell_coef;
   for (int f = 0; f < 6; ++f) a.epd[f] = c.ell_pd[f];
   a.ewrapz = c.ell_wrapz != 0;
+  for (int f = 0; f < 6; ++f) a.spd[f] = c.spe_pd[f];
+  a.swrapz = c.spe_wrapz != 0;
   a.N = c.g.N;
   a.sliced = c.ell_sliced;
   a.col = c.col;

@@ -266,6 +266,8 @@ hipError_t launch_csr_assemble(Ctx &c) {
 }
 
 hipError_t launch_spe_assemble(Ctx &c) {
+  for (int f = 0; f < 6; ++f) c.spe_pd[f] = c.prm.p_dirichlet[f];
+  c.spe_wrapz = c.prm.periodic_z;
   spe_jp_kernel<<<blocks_for(c.g.N, 256, 1 << 30), 256, 0, c.stream>>>(c.g.nxc, c.g.nyc, c.g.nzc, pbc_of(c),
                                                                        c.spe_coef, c.spe_jp);
   return hipGetLastError();
@@ -276,6 +278,8 @@ hipError_t launch_spmv(Ctx &c, int op, int precision, const double *x, double *y
   const SpeTiles T = spe_tiles(c.g.nxc, c.g.nyc, c.g.nzc);
   if (precision == CFD_MIXED && op == CFD_OP_ELL)
     spmv32_from64_kernel<<<stream_blocks(c.g.N), 256, 0, c.stream>>>(a, x, y);
+  else if (op == CFD_OP_SPE && spe_pairs(a, T, {x, y}))
+    launch_spe_walk<0>(a, T, nullptr, x, y, nullptr, nullptr, c.stream);
   else if (op == CFD_OP_SPE && T.blocks <= (1 << 30))
     spe_spmv_kernel<<<(unsigned)T.blocks, 256, 0, c.stream>>>(a, T, x, y);
   else if (const int pp = ell_grid_period(a, c.g.N / 256, 256, {x, y}))

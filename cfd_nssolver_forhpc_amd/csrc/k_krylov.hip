@@ -672,6 +672,7 @@ hipError_t launch_iters(Ctx &c, const OpArgs &a, const Vecs<T> &v, KrylovScalars
   // the SPE operator's SpMV-dot kernels over plane columns (FP64)
   const SpeTiles tiles = spe_tiles(c.g.nxc, c.g.nyc, c.g.nzc);
   const bool spe = std::is_same<T, double>::value && a.op == CFD_OP_SPE && tiles.blocks <= RED_MAX_BLOCKS;
+  const bool pairs = spe && spe_pairs(a, tiles, {v.p1, v.ap, v.r0, v.s1, v.as});
   const int nbs = spe ? (int)tiles.blocks : nb;
   const int pp = std::is_same<T, double>::value ? ell_grid_period(a, nb, SPMV_DOT_THREADS, {v.p1, v.ap, v.r0, v.s1, v.as}) : 0;
   const Fold fold = fold_of(nbs, nbx);
@@ -681,6 +682,9 @@ hipError_t launch_iters(Ctx &c, const OpArgs &a, const Vecs<T> &v, KrylovScalars
       launch_ell_grid<SPMV_DOT_THREADS, 1>(a, pp, ks, reinterpret_cast<const double *>(v.p1),
                                                reinterpret_cast<double *>(v.ap),
                                                reinterpret_cast<const double *>(v.r0), p1, c.stream);
+    else if (pairs)
+      launch_spe_walk<1>(a, tiles, ks, reinterpret_cast<const double *>(v.p1), reinterpret_cast<double *>(v.ap),
+                         reinterpret_cast<const double *>(v.r0), p1, c.stream);
     else if (spe)
       spe_spmv_dot_kernel<<<nbs, 256, 0, c.stream>>>(a, tiles, ks, reinterpret_cast<const double *>(v.p1),
                                                      reinterpret_cast<double *>(v.ap),
@@ -698,6 +702,9 @@ hipError_t launch_iters(Ctx &c, const OpArgs &a, const Vecs<T> &v, KrylovScalars
     if (pp)
       launch_ell_grid<SPMV_DOT_THREADS, 2>(a, pp, ks3, reinterpret_cast<const double *>(v.s1),
                                                reinterpret_cast<double *>(v.as), nullptr, p2, c.stream);
+    else if (pairs)
+      launch_spe_walk<2>(a, tiles, ks3, reinterpret_cast<const double *>(v.s1), reinterpret_cast<double *>(v.as),
+                         nullptr, p2, c.stream);
     else if (spe)
       spe_spmv_dot2_kernel<<<nbs, 256, 0, c.stream>>>(a, tiles, ks3, reinterpret_cast<const double *>(v.s1),
                                                       reinterpret_cast<double *>(v.as), p2);
@@ -868,6 +875,7 @@ int launch_pc_iters(Ctx &c, const OpArgs &a, const PVecs<T> &v, KrylovScalars *k
   // the SPE operator's kernels over plane columns (FP64), as in launch_iters
   const SpeTiles tiles = spe_tiles(c.g.nxc, c.g.nyc, c.g.nzc);
   const bool spe = std::is_same<T, double>::value && a.op == CFD_OP_SPE && tiles.blocks <= RED_MAX_BLOCKS;
+  const bool pairs = spe && spe_pairs(a, tiles, {v.ph, v.v, v.r0, v.sh, v.t, v.s1});
   const int nbs = spe ? (int)tiles.blocks : nb;
   const int pp = std::is_same<T, double>::value ? ell_grid_period(a, nb, 256, {v.ph, v.v, v.r0, v.sh, v.t, v.s1}) : 0;
   const Fold fold = fold_of(nbs, nbu);
@@ -878,6 +886,9 @@ int launch_pc_iters(Ctx &c, const OpArgs &a, const PVecs<T> &v, KrylovScalars *k
     if (pp)
       launch_ell_grid<256, 1>(a, pp, ks, reinterpret_cast<const double *>(v.ph), reinterpret_cast<double *>(v.v),
                                   reinterpret_cast<const double *>(v.r0), p1, c.stream);
+    else if (pairs)
+      launch_spe_walk<1>(a, tiles, ks, reinterpret_cast<const double *>(v.ph), reinterpret_cast<double *>(v.v),
+                         reinterpret_cast<const double *>(v.r0), p1, c.stream);
     else if (spe)
       spe_spmv_dot_kernel<<<nbs, 256, 0, c.stream>>>(a, tiles, ks, reinterpret_cast<const double *>(v.ph),
                                                      reinterpret_cast<double *>(v.v),
@@ -894,6 +905,9 @@ int launch_pc_iters(Ctx &c, const OpArgs &a, const PVecs<T> &v, KrylovScalars *k
     if (pp)
       launch_ell_grid<256, 3>(a, pp, ks3, reinterpret_cast<const double *>(v.sh), reinterpret_cast<double *>(v.t),
                                   reinterpret_cast<const double *>(v.s1), p2, c.stream);
+    else if (pairs)
+      launch_spe_walk<3>(a, tiles, ks3, reinterpret_cast<const double *>(v.sh), reinterpret_cast<double *>(v.t),
+                         reinterpret_cast<const double *>(v.s1), p2, c.stream);
     else if (spe)
       spe_spmv_dot2_pc_kernel<<<nbs, 256, 0, c.stream>>>(a, tiles, ks3, reinterpret_cast<const double *>(v.sh),
                                                          reinterpret_cast<const double *>(v.s1),
@@ -1065,6 +1079,8 @@ hipError_t launch_spmv_dot(Ctx &c) {
   if (const int pp = ell_grid_period(a, blocks_for(c.g.N, SPMV_DOT_THREADS, RED_MAX_BLOCKS), SPMV_DOT_THREADS,
                                       {c.p1, c.ap, c.r0}))
     launch_ell_grid<SPMV_DOT_THREADS, 1>(a, pp, c.ks32, c.p1, c.ap, c.r0, part, c.stream);
+  else if (a.op == CFD_OP_SPE && tiles.blocks <= RED_MAX_BLOCKS && spe_pairs(a, tiles, {c.p1, c.ap, c.r0}))
+    launch_spe_walk<1>(a, tiles, c.ks32, c.p1, c.ap, c.r0, part, c.stream);
   else if (a.op == CFD_OP_SPE && tiles.blocks <= RED_MAX_BLOCKS)
     spe_spmv_dot_kernel<<<(int)tiles.blocks, 256, 0, c.stream>>>(a, tiles, c.ks32, c.p1, c.ap, c.r0, part);
   else if (a.op != CFD_OP_CSR)  // launch_iters' launch
