@@ -449,9 +449,16 @@ __global__ void __launch_bounds__(256) mg_split_sweep_kernel(MGView L, MGView C,
 // a cell 6.1 TB/s of FP64 traffic.  With a branch per stage the compiler
 // drained every load before its use and an FP64 pass took 59-68 us.  One
 // workgroup a CU: tiles of 24 rows and 23 planes at that size, each computing
-// 1.5 times its cells, are what 256 CUs leave.  Three timesteps
+// 1.5 times its cells, are what 256 CUs leave (two workgroups a CU, with twice
+// the overlap: a cycle of 490 us against 422).  Three timesteps
 // there went from 73.9 to 57.2 ms (FP64; mixed 65.5 to 50.8), the 256x128x32
 // adjoint from 110 to 83 ms.
+//
+// The cycle's first pass (SCL) forms the right-hand side r / jp from the
+// natural-order vectors on the way in and starts from x = 0, so that neither a
+// kernel that scales nor the first red half-sweep touches memory on its own:
+// at 512x256x64 48 + 34 -> 66 us FP64, 46 + 25 -> 41 FP32, a cycle 422 -> 400
+// and 303 -> 278.  It reads pairs of cells, so nz has to be even.
 constexpr int FUSED_THREADS = 1024;
 constexpr int FUSED_RING = 6;     // planes of x and b a thread holds
 constexpr int FUSED_CHUNK = 512;  // planes of a run at most (its coefficients sit in LDS)
@@ -490,6 +497,15 @@ __device__ inline float div_by(float n, float d, float y) {
 }
 
 // the column a thread of mg_fused_kernel owns and what it carries
+// SCL: the pass forms the right-hand side r / jp itself (natural order, nz
+// even), from x = 0, and leaves it in b
+template <typename T, typename V>
+struct FusedRhs {
+  const V *r;
+  const double *jp;
+  T *b;
+};
+
 template <typename T, int NS>
 struct FusedCol {
   T in[FUSED_RING], bA[FUSED_RING], bB[FUSED_RING];  // other colour before the pass; right-hand sides
@@ -506,13 +522,14 @@ struct alignas(2 * sizeof(T)) CoefX {
   T m, p;  // to the -x and +x neighbour
 };
 
-template <typename T, typename V, int NS, int START, bool PRO, bool OUT>
+template <typename T, typename V, int NS, int START, bool PRO, bool OUT, bool SCL = false>
 __global__ void __launch_bounds__(FUSED_THREADS) mg_fused_kernel(MGView L, MGView C, FusedShape S,
                                                                  const T *__restrict__ b, const T *__restrict__ xin,
                                                                  T *__restrict__ xout, const T *__restrict__ xc,
-                                                                 V *__restrict__ out, const KrylovScalars *ks) {
+                                                                 V *__restrict__ out, FusedRhs<T, V> R,
+                                                                 const KrylovScalars *ks) {
   if (ks && ks->done) return;
-  constexpr int PD = sizeof(T) == 8 ? 2 : 3;
+  constexpr int PD = sizeof(T) == 8 || SCL ? 2 : 3;
   constexpr bool KEEP_D = sizeof(T) == 4;  // FP64 adds the diagonal again instead of holding it
   __shared__ T half[2][NS][FUSED_THREADS];
   __shared__ CoefX<T> cxl[FUSED_CHUNK + 2 * NS];
@@ -562,7 +579,19 @@ __global__ void __launch_bounds__(FUSED_THREADS) mg_fused_kernel(MGView L, MGVie
   }
   if (row >= S.R) c.side[0] = c.side[1] = tid;
   const int im = row > 0 ? tid - hz : tid, ip = row + 1 < S.R ? tid + hz : tid;
+  // SCL: the right-hand side's pair of cells at a plane, r and jp as they come
+  typedef V V2 __attribute__((ext_vector_type(2)));
+  typedef double D2 __attribute__((ext_vector_type(2)));
+  V2 rr[3];
+  D2 rj[3];
+  const unsigned pair = (unsigned)(jc * L.nz + 2 * k2);
+  auto load_pair = [&](int s, int plane) {
+    const int64_t o = (int64_t)min(max(plane, 0), L.nx - 1) * L.ny * L.nz;
+    rr[s] = *reinterpret_cast<const V2 *>(reinterpret_cast<const char *>(R.r + o) + pair * (unsigned)sizeof(V));
+    rj[s] = *reinterpret_cast<const D2 *>(reinterpret_cast<const char *>(R.jp + o) + pair * 8u);
+  };
   auto load_in = [&](int plane, int q) -> T {  // q: parity index of the other colour at that plane
+    if (SCL) return (T)0;
     plane = min(max(plane, 0), L.nx - 1);
     T v = in_plane(xo, plane);
     if (PRO) {
@@ -580,16 +609,22 @@ __global__ void __launch_bounds__(FUSED_THREADS) mg_fused_kernel(MGView L, MGVie
   // ring positions: plane ta + m of x at (m + 1) mod 6, of b at m mod 6
 #pragma unroll
   for (int m = -1; m <= PD; ++m) c.in[m + 1] = load_in(ta + m, (m + 1) & 1);
+  if (SCL) {
 #pragma unroll
-  for (int m = 0; m < PD; ++m) c.bA[m] = load_b(bA, ta + m, m & 1);
+    for (int m = 0; m < FUSED_RING; ++m) c.bA[m] = c.bB[m] = (T)0;
 #pragma unroll
-  for (int m = 0; m < PD - 1; ++m) c.bB[m] = load_b(bB, ta + m, (m + 1) & 1);
+    for (int m = 0; m < PD; ++m) load_pair(m, ta + m);
+  } else {
 #pragma unroll
-  for (int m = PD; m < FUSED_RING; ++m) {
-    if (m > PD + 1) c.in[m] = (T)0;
-    c.bA[m] = c.bB[m] = (T)0;
+    for (int m = 0; m < PD; ++m) c.bA[m] = load_b(bA, ta + m, m & 1);
+#pragma unroll
+    for (int m = 0; m < PD - 1; ++m) c.bB[m] = load_b(bB, ta + m, (m + 1) & 1);
+#pragma unroll
+    for (int m = PD; m < FUSED_RING; ++m) c.bA[m] = c.bB[m] = (T)0;
+    c.bB[PD - 1] = (T)0;
   }
-  c.bB[PD - 1] = (T)0;
+#pragma unroll
+  for (int m = PD + 2; m < FUSED_RING; ++m) c.in[m] = (T)0;
 #pragma unroll
   for (int q = 0; q < 3; ++q) {
     c.yA[q] = c.yB[q] = c.dA[q] = c.dB[q] = (T)1;
@@ -615,8 +650,22 @@ __global__ void __launch_bounds__(FUSED_THREADS) mg_fused_kernel(MGView L, MGVie
     T(*cur)[FUSED_THREADS] = half[u & 1];
     // loads of the planes PD ahead of their first use
     c.in[(u + 2 + PD) % 6] = load_in(min(ta + n + 1 + PD, te + 1), (u + PD) & 1);
-    c.bA[(u + PD) % 6] = load_b(bA, min(ta + n + PD, te), (u + PD) & 1);
-    c.bB[(u + PD - 1) % 6] = load_b(bB, min(ta + n + PD - 1, te), (u + PD) & 1);
+    if (SCL) {
+      load_pair((u + PD) % 3, min(ta + n + PD, te));
+      // b of plane ta + n, mg_scale_kernel's
+      const T b0 = (T)((double)rr[u % 3].x / rj[u % 3].x), b1 = (T)((double)rr[u % 3].y / rj[u % 3].y);
+      c.bA[u] = c.up[q] ? b1 : b0;
+      c.bB[u] = c.up[q] ? b0 : b1;
+      if (ta + n >= i0 && ta + n < i1 && store) {
+        char *o = reinterpret_cast<char *>(R.b + (int64_t)(ta + n) * sx);
+        *reinterpret_cast<T *>(o + (START ? ns * (int64_t)sizeof(T) : 0) + atb) = c.bA[u];
+        *reinterpret_cast<T *>(o + (START ? 0 : ns * (int64_t)sizeof(T)) + atb) = c.bB[u];
+      }
+      if (sizeof(T) == 8) __builtin_amdgcn_sched_barrier(0);
+    } else {
+      c.bA[(u + PD) % 6] = load_b(bA, min(ta + n + PD, te), (u + PD) & 1);
+      c.bB[(u + PD - 1) % 6] = load_b(bB, min(ta + n + PD - 1, te), (u + PD) & 1);
+    }
     // a stage's LDS reads are issued before the stage ahead of it is computed,
     // and not earlier (all at once they take registers that FP64 lacks)
     T vym[NS], vyp[NS], vs[NS];
@@ -627,7 +676,7 @@ __global__ void __launch_bounds__(FUSED_THREADS) mg_fused_kernel(MGView L, MGVie
       vs[s] = prev[s][c.side[q]];
       cx[s] = cxl[min(max(n - s, 0), ilast)];
     };
-    fetch(0);
+    if (!SCL) fetch(0);  // SCL: the first stage's neighbours are zero
     const double dx0 = dxl[min(n, ilast)], dx1 = dxl[min(max(n - 1, 0), ilast)];
     double dx2 = 0.0, dx3 = 0.0;
     if (!KEEP_D) {
@@ -651,17 +700,20 @@ __global__ void __launch_bounds__(FUSED_THREADS) mg_fused_kernel(MGView L, MGVie
       const T d = KEEP_D ? ((s & 1) ? c.dB[r0] : c.dA[r0])
                          : (T)((s == 0 ? dx0 : s == 1 ? dx1 : s == 2 ? dx2 : dx3) + c.dy + c.dz[q]);
       const T y = (s & 1) ? c.yB[r0] : c.yA[r0];
-      T v = fma(cx[s].m, xm, (T)0);
-      v = fma(cx[s].p, xp, v);
-      v = fma(c.cym, vym[s], v);
-      v = fma(c.cyp, vyp[s], v);
-      const T v1 = c.up[q] ? x0 : vs[s], v2 = c.up[q] ? vs[s] : x0;  // -z, +z
-      v = fma(c.czm[q], v1, v);
-      v = fma(c.czp[q], v2, v);
+      T v = (T)0;
+      if (!SCL || s > 0) {
+        v = fma(cx[s].m, xm, (T)0);
+        v = fma(cx[s].p, xp, v);
+        v = fma(c.cym, vym[s], v);
+        v = fma(c.cyp, vyp[s], v);
+        const T v1 = c.up[q] ? x0 : vs[s], v2 = c.up[q] ? vs[s] : x0;  // -z, +z
+        v = fma(c.czm[q], v1, v);
+        v = fma(c.czp[q], v2, v);
+      }
       c.st[s][r0] = div_by(bv + v, d, y);
       if (s + 1 < NS) cur[s + 1 < NS ? s + 1 : 0][tid] = c.st[s][r0];
     }
-    cur[0][tid] = c.in[(u + 2) % 6];
+    if (!SCL) cur[0][tid] = c.in[(u + 2) % 6];
     // the pass's result of plane ta + n - NS + 1: the last half-sweep's colour and the other
     const int p = ta + n - (NS - 1);
     if (p >= i0 && p < i1 && store) {
@@ -1140,7 +1192,17 @@ void launch_fused(const MGView &v, const MGView &C, const T *b, const T *xin, T 
   const FusedShape s = fused_shape(v, NS);
   const int threads = (s.R * s.hz + 63) / 64 * 64;
   mg_fused_kernel<T, V, NS, START, PRO, OUT>
-      <<<s.njt * s.nci, threads, 0, st>>>(v, C, s, b, xin, xout, xc, out, ks);
+      <<<s.njt * s.nci, threads, 0, st>>>(v, C, s, b, xin, xout, xc, out, FusedRhs<T, V>{}, ks);
+}
+
+// the first four half-sweeps from x = 0 with the right-hand side r / jp
+template <typename T, typename V>
+void launch_fused_scaled(const MGView &v, const V *r, const double *jp, T *b, T *xout, const KrylovScalars *ks,
+                         hipStream_t st) {
+  const FusedShape s = fused_shape(v, 4);
+  const int threads = (s.R * s.hz + 63) / 64 * 64;
+  mg_fused_kernel<T, V, 4, 0, false, false, true><<<s.njt * s.nci, threads, 0, st>>>(
+      v, v, s, b, nullptr, xout, nullptr, nullptr, FusedRhs<T, V>{r, jp, b}, ks);
 }
 
 int nblk(int64_t n) { return blocks_for(n, 256, 1 << 30); }
@@ -1212,7 +1274,12 @@ int mg_apply(Ctx &c, const V *r, V *out, const KrylovScalars *ks) {
   T *x0 = (same && !split) ? reinterpret_cast<T *>(out) : lx<T>(M.lv[0]);
   if (!b0 || !x0) return fail(CFD_ERR_STATE, "multigrid buffers of this precision are not allocated");
   auto X = [&](int l) { return l == 0 ? x0 : lx<T>(M.lv[l]); };
-  if (split)
+  const MGView &v0 = M.lv[0].v;
+  const bool scaled = split && M.nu >= 2 && v0.nz % 2 == 0 && fused_shape(v0, 4).R > 0 &&
+                      reinterpret_cast<uintptr_t>(r) % (2 * sizeof(V)) == 0;
+  if (scaled)
+    launch_fused_scaled<T, V>(v0, r, c.f[CFD_JP], b0, x0, ks, c.stream);
+  else if (split)
     LevelOps<T, ColourSplit>::scale_from(M.lv[0].v, r, c.f[CFD_JP], b0, x0, ks, c.stream);
   else
     LevelOps<T, Natural>::scale_from(M.lv[0].v, r, c.f[CFD_JP], b0, x0, ks, c.stream);
@@ -1248,6 +1315,18 @@ int mg_apply(Ctx &c, const V *r, V *out, const KrylovScalars *ks) {
     T *other = xs[l] == X(l) ? lxb<T>(M.lv[l]) : X(l);
     auto swap = [&] { std::swap(xs[l], other); };
     T *const none = nullptr;
+    if (pre && l == 0 && scaled) {
+      int left = 2 * M.nu - 4;  // red first
+      for (; left >= 4; left -= 4) {
+        launch_fused<T, T, 4, 0, false, false>(v, C, bl, xs[l], other, none, none, ks, c.stream);
+        swap();
+      }
+      if (left == 2) {
+        single(l, 0, SWEEP_PLAIN);
+        single(l, 1, SWEEP_PLAIN);
+      }
+      return;
+    }
     if (pre) {
       int left = 2 * M.nu - 1;  // black first
       for (; left >= 4; left -= 4) {
