@@ -897,7 +897,7 @@ int cfd_dfib_update(cfd_ctx *ctx) {
   Ctx &c = *reinterpret_cast<Ctx *>(ctx);
   int rc = sync_p(c);
   if (rc) return rc;
-  RET_LAUNCH(launch_dfib_update_into(c, UPD_WRITE_T3, c.f[CFD_P], nullptr, nullptr));
+  RET_LAUNCH(launch_dfib_update_into(c, UPD_WRITE_T3 | UPD_WRITE_F, c.f[CFD_P], nullptr, nullptr));
   CFD_HIP(hipStreamSynchronize(c.stream));
   return CFD_OK;
 }
@@ -1081,7 +1081,8 @@ int step_impl(Ctx &c, cfd_step_stats *stats) {
     CFD_HIP(mark(CFD_PHASE_PRESSURE));
     int mode = UPD_DRAG;
     if (c.p_from_x) mode |= UPD_P_FROM_X;
-    if (corrector) mode |= UPD_WRITE_T3 | UPD_WRITE_T0 | UPD_MAXDIFF;
+    // the force of a pass is kept as its source; the array holds the corrector's
+    if (corrector) mode |= UPD_WRITE_T3 | UPD_WRITE_T0 | UPD_WRITE_F | UPD_MAXDIFF;
     else mode |= (pass == 0 ? UPD_SRC_SET : UPD_SRC_ADD);
     const double *pp = c.p_from_x ? c.f[CFD_X] : c.f[CFD_P];
     double *t2 = c.t2_rec ? c.t2_rec + (size_t)3 * c.g.N * pass : nullptr;

@@ -220,7 +220,7 @@ hipError_t launch_rhs(Ctx &c, const double *u1, const double *v1, const double *
 hipError_t launch_scatter_p(Ctx &c, const double *X, double *p);
 // mode bits for the DFIB update
 enum { UPD_WRITE_T3 = 1, UPD_WRITE_T0 = 2, UPD_SRC_SET = 4, UPD_SRC_ADD = 8, UPD_DRAG = 16, UPD_MAXDIFF = 32,
-       UPD_P_FROM_X = 64 };
+       UPD_P_FROM_X = 64, UPD_WRITE_F = 128 };
 hipError_t launch_dfib_update_into(Ctx &c, int mode, const double *p_or_x, double *drag_out, double *max_out,
                                    double *t2out = nullptr);
 hipError_t launch_source_accumulate(Ctx &c);
