@@ -749,7 +749,11 @@ __global__ void __launch_bounds__(FUSED_THREADS) mg_fused_kernel(MGView L, MGVie
 // 2K + 1).  The kernel loads those pairs, the pairs of the eight columns
 // beside them and the single entries below (2K - 1) and above (2K + 2) each
 // column (40 loads for 8 children, with b), and sums the children's
-// residuals in restrict_at's order with child_res's arithmetic.
+// residuals in restrict_at's order with child_res's arithmetic.  Bound by its
+// instructions (three quarters of the VALU's cycles in FP32): with the 40
+// addresses formed from uniform plane bases and six offsets 512x256x64 takes
+// 33.8 us FP64 and 20.9 FP32, from indexes of their own 36.7 and 25.  Four
+// waves a SIMD instead of three spill (49.5 and 43.6 us).
 template <typename T, typename CLay = Natural>
 __global__ void __launch_bounds__(256) mg_restrict_split_kernel(MGView F, MGView C, const T *__restrict__ bf,
                                                                 const T *__restrict__ xf, T *__restrict__ bc,
@@ -759,14 +763,25 @@ __global__ void __launch_bounds__(256) mg_restrict_split_kernel(MGView F, MGView
   if (K >= C.nz || J >= C.ny) return;
   const int hz = F.nz >> 1;  // nz is even where z is halved
   const int64_t ns = (int64_t)F.nx * F.ny * hz;
-  // entry at k = 2 KK + m (m = 0, 1) of column (i, j), both clamped into the
-  // grid (KK wraps across the periodic seam)
-  auto ld = [&](const T *a, int i, int j, int KK, int m) -> T {
-    i = min(max(i, 0), F.nx - 1);
-    j = min(max(j, 0), F.ny - 1);
-    if (F.wz) KK = KK < 0 ? hz - 1 : (KK >= hz ? 0 : KK);
-    KK = min(max(KK, 0), hz - 1);
-    return a[(((i + j + m) & 1) ? ns : 0) + ((int64_t)i * F.ny + j) * hz + KK];
+  // The entry at k = 2 KK + m of column (2I - 1 + a, 2J - 1 + c) is in colour
+  // half (a + c + m) & 1: a plane's base is uniform, a thread's place in it one
+  // of six 32-bit offsets.  Columns outside the grid are clamped into it (KK
+  // wraps across the periodic seam); what they load is not used.
+  const int Km = K > 0 ? K - 1 : F.wz ? hz - 1 : 0, Kp = K < hz - 1 ? K + 1 : F.wz ? 0 : hz - 1;
+  unsigned row[4], rkm[2], rkp[2];
+#pragma unroll
+  for (int c = 0; c < 4; ++c) {
+    const int j = min(max(2 * J - 1 + c, 0), F.ny - 1);
+    row[c] = (unsigned)(j * hz + K) * (unsigned)sizeof(T);
+    if (c == 1 || c == 2) {
+      rkm[c - 1] = (unsigned)(j * hz + Km) * (unsigned)sizeof(T);
+      rkp[c - 1] = (unsigned)(j * hz + Kp) * (unsigned)sizeof(T);
+    }
+  }
+  auto ld = [&](const T *f, int a, int half, unsigned off) -> T {
+    const int i = min(max(2 * I - 1 + a, 0), F.nx - 1);
+    const T *base = f + ((half & 1) ? ns : 0) + (int64_t)i * F.ny * hz;
+    return *reinterpret_cast<const T *>(reinterpret_cast<const char *>(base) + off);
   };
   // X[a][c] = the pair of column (2I - 1 + a, 2J - 1 + c): the four children's
   // columns (a, c in 1..2) and the eight beside them (no corners)
@@ -777,16 +792,15 @@ __global__ void __launch_bounds__(256) mg_restrict_split_kernel(MGView F, MGView
     for (int c = 0; c < 4; ++c)
 #pragma unroll
       for (int m = 0; m < 2; ++m)
-        X[a][c][m] = ((a == 0 || a == 3) && (c == 0 || c == 3)) ? (T)0 : ld(xf, 2 * I - 1 + a, 2 * J - 1 + c, K, m);
+        X[a][c][m] = ((a == 0 || a == 3) && (c == 0 || c == 3)) ? (T)0 : ld(xf, a, a + c + m, row[c]);
 #pragma unroll
   for (int di = 0; di < 2; ++di)
 #pragma unroll
     for (int dj = 0; dj < 2; ++dj) {
-      const int i = 2 * I + di, j = 2 * J + dj;
-      B[di][dj][0] = ld(bf, i, j, K, 0);
-      B[di][dj][1] = ld(bf, i, j, K, 1);
-      xkm[di][dj] = ld(xf, i, j, K - 1, 1);  // k = 2K - 1
-      xkp[di][dj] = ld(xf, i, j, K + 1, 0);  // k = 2K + 2
+      B[di][dj][0] = ld(bf, di + 1, di + dj, row[dj + 1]);
+      B[di][dj][1] = ld(bf, di + 1, di + dj + 1, row[dj + 1]);
+      xkm[di][dj] = ld(xf, di + 1, di + dj + 1, rkm[dj]);  // k = 2K - 1
+      xkp[di][dj] = ld(xf, di + 1, di + dj, rkp[dj]);      // k = 2K + 2
     }
   double acc = 0.0;
 #pragma unroll
