@@ -21,9 +21,12 @@
 //
 // What bounds it is the latency of the five exchanges, about 2 us each, and,
 // past 10^5 rows, the halo words.  Measured on one MI355X, us an iteration,
-// launch path -> here: 512 rows 26.4 -> 4.7 (one workgroup: sums through
-// LDS), 4096 33.0 -> 10.9, 32768 33.3 -> 11.8, 65536 34.4 -> 14.4, 303750
-// 47.7 -> 22.4, 524288 53.1 -> 19.5.
+// launch path -> here: 512 rows 15.4 -> 4.6 (one workgroup: sums through
+// LDS), 4096 19.2 -> 9.7, 32768 19.3 -> 10.9, 65536 21.0 -> 13.6, 303750
+// 30.6 -> 22.3, 524288 28.5 -> 19.7.  Of the 12 us that 32768 rows took before
+// the wave sums were packed, every wave formed the total of up to 128 slots
+// itself and the next p left ahead of the stop test: halos 2.8, the sums'
+// way 5.5, products with their wave sums 1.9, the rest 1.6.
 #pragma once
 
 #include "dev_common.h"
@@ -67,6 +70,8 @@ struct ResLds {
   double fin[2][FIN_THREADS / 64];
   double one[2][4][2];                     // block sums of a lone workgroup (at most 4 slots)
   int nhalo, state, stuck;
+  double norm0, tol, restart_tol;
+  int maxit, timestep;
 };
 
 // The workgroup's halo of the vector exchanged in ll, into its LDS entries.
@@ -81,6 +86,44 @@ __device__ inline void resident_halo(ResLds &L, const ResArgs &a, unsigned epoch
         });
     if (!ok) L.stuck = 1;
   }
+}
+
+// wave_sum of two and of four values at once.  wave_sum adds neighbouring
+// lanes, then neighbouring pairs, quads, .. and every lane of a group holds the
+// group's sum; here the copies are given up for other values (lane & 1, lane &
+// 3 says whose sum a lane holds), so that the steps are shared.  The sums are
+// wave_sum's bit for bit in lanes 62, 63 and 60 .. 63: lanes of the last quad
+// of 16, whose order of the quads is the one that wave_sum returns.
+__device__ inline double wave_rows(double v) {  // the steps across quads and rows
+  v += dpp_move<0x124>(v);                      // row_ror:4
+  v += dpp_move<0x128>(v);                      // row_ror:8
+  const long long b = __double_as_longlong(v);
+  const auto l16 = __builtin_amdgcn_permlane16_swap((unsigned)b, (unsigned)b, false, false);
+  const auto h16 = __builtin_amdgcn_permlane16_swap((unsigned)(b >> 32), (unsigned)(b >> 32), false, false);
+  v = __longlong_as_double((long long)h16[0] << 32 | l16[0]) + __longlong_as_double((long long)h16[1] << 32 | l16[1]);
+  const long long d = __double_as_longlong(v);
+  const auto l32 = __builtin_amdgcn_permlane32_swap((unsigned)d, (unsigned)d, false, false);
+  const auto h32 = __builtin_amdgcn_permlane32_swap((unsigned)(d >> 32), (unsigned)(d >> 32), false, false);
+  return __longlong_as_double((long long)h32[0] << 32 | l32[0]) + __longlong_as_double((long long)h32[1] << 32 | l32[1]);
+}
+__device__ inline double pair_pack(double a, double b) {  // even lanes: a of the pair, odd lanes: b
+  const bool odd = threadIdx.x & 1;
+  return (odd ? b : a) + dpp_move<0xb1>(odd ? a : b);
+}
+__device__ inline double wave_sum2(double a, double b) {
+  double v = pair_pack(a, b);
+  v += dpp_move<0x4e>(v);
+  return wave_rows(v);
+}
+__device__ inline double wave_sum4(double a, double b, double c, double d) {
+  const double ab = pair_pack(a, b), cd = pair_pack(c, d);
+  const bool hi = threadIdx.x & 2;
+  return wave_rows((hi ? cd : ab) + dpp_move<0x4e>(hi ? ab : cd));
+}
+__device__ inline double lane_value(double v, int lane) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_readlane((int)b, lane), hi = __builtin_amdgcn_readlane((int)(b >> 32), lane);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
 
 // Where a workgroup leaves a slot's sum (e = 0) or the sum of its first half
@@ -164,16 +207,35 @@ __device__ inline void resident_total(const ResArgs &a, ResLds &L, const uint64_
                                       double (&tot)[NV]) {
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   __syncthreads();  // this workgroup's sums are left (L.one, or issued: RES_SPIN)
-  if (a.nblk == 1) {
-    if (wid < NV) {  // at most 4 slots: the first finalize wave's lanes
-      double v = 0.0;
-      if (lane < nslot) v = L.one[wid][lane][0];
-      v = wave_sum(0.0 + v);
-      if (lane == 0) L.fin[wid][0] = v;
-    }
-    __syncthreads();
+  // Up to two of the finalize kernel's waves (N <= 65536): every wave of the
+  // workgroup forms the total itself; the other waves' sums are zero.
+  if (nslot <= 128) {
+    double v[2][NV];
+    if (a.nblk == 1) {
 #pragma unroll
-    for (int q = 0; q < NV; ++q) tot[q] = L.fin[q][0] + 0.0;  // the other 15 waves' sums are zero
+      for (int q = 0; q < NV; ++q) {
+        v[0][q] = lane < nslot ? L.one[q][lane & 3][0] : 0.0;
+        v[1][q] = 0.0;
+      }
+    } else {
+      const bool ok = ll_fetch<2 * NV>(
+          red, red + 1, epoch,
+          [&](int u) {
+            const int q = u % NV, slot = lane + u / NV * 64;
+            return slot < nslot ? (unsigned)(q * RES_RED_WORDS + slot * 4) : RES_NONE;
+          },
+          [&](int u, bool have, double x) { v[u / NV][u % NV] = have ? x : 0.0; });
+      if (!ok) L.stuck = 1;
+    }
+    // combine_partials adds the slot to a zero
+    if constexpr (NV == 1) {
+      const double w = wave_sum2(0.0 + v[0][0], 0.0 + v[1][0]);
+      tot[0] = (lane_value(w, 62) + lane_value(w, 63)) + 0.0;
+    } else {
+      const double w = wave_sum4(0.0 + v[0][0], 0.0 + v[0][1], 0.0 + v[1][0], 0.0 + v[1][1]);
+      tot[0] = (lane_value(w, 60) + lane_value(w, 62)) + 0.0;
+      tot[1] = (lane_value(w, 61) + lane_value(w, 63)) + 0.0;
+    }
     return;
   }
 #pragma unroll 1
@@ -188,20 +250,27 @@ __device__ inline void resident_total(const ResArgs &a, ResLds &L, const uint64_
           red, red + 1, epoch, [&](int q) { return mine ? (unsigned)(q * RES_RED_WORDS + slot * 4) : RES_NONE; },
           [&](int q, bool have, double x) { v[q] = have ? x : 0.0; });
       if (!ok) L.stuck = 1;
-#pragma unroll
-      for (int q = 0; q < NV; ++q) v[q] = wave_sum(0.0 + v[q]);  // combine_partials adds the slot to a zero
+      // combine_partials adds the slot to a zero
+      if constexpr (NV == 1)
+        v[0] = wave_sum(0.0 + v[0]);
+      else
+        v[0] = wave_sum2(0.0 + v[0], 0.0 + v[1]);
     }
-    if (lane == 0) {
-#pragma unroll
-      for (int q = 0; q < NV; ++q) L.fin[q][wid + half * (RES_THREADS / 64)] = v[q];
-    }
+    if (NV == 1 && lane == 0) L.fin[0][wid + half * (RES_THREADS / 64)] = v[0];
+    if (NV == 2 && lane >= 62) L.fin[lane - 62][wid + half * (RES_THREADS / 64)] = v[0];
   }
   __syncthreads();
 #pragma unroll
   for (int q = 0; q < NV; ++q) {
     double s = L.fin[q][0];
+#pragma unroll 1
+    for (int w = 0; w < FIN_THREADS / 64; w += 8) {  // eight in flight: the register file is full
+      double f[8];
 #pragma unroll
-    for (int w = 1; w < FIN_THREADS / 64; ++w) s += L.fin[q][w];
+      for (int u = 0; u < 8; ++u) f[u] = L.fin[q][w + u];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) s = w + u ? s + f[u] : s;
+    }
     tot[q] = s;
   }
 }
@@ -241,14 +310,16 @@ __global__ void __launch_bounds__(RES_THREADS) bicg_resident_kernel(ResArgs a) {
   auto own = [&](int m) { return v + m * S < vend; };
   if (a.ks->done) return;  // uniform over the grid: written by an earlier kernel
   double rho = a.ks->rho;
-  const double norm0 = a.ks->norm0;
-  const double tol = a.ks->tol, restart_tol = a.ks->restart_tol;
-  const int maxit = a.ks->maxit, timestep = a.ks->timestep;
   int iters = a.ks->iters, restarts = a.ks->restarts;
   if (t == 0) {
     L.nhalo = a.nblk > 1 ? 1 : 0;  // entry 0: column N - 1, where every padding slot points
     L.hcol[0] = (int32_t)(N - 1);
     L.stuck = 0;
+    L.norm0 = a.ks->norm0;
+    L.tol = a.ks->tol;
+    L.restart_tol = a.ks->restart_tol;
+    L.maxit = a.ks->maxit;
+    L.timestep = a.ks->timestep;
   }
   __syncthreads();
   double val[RES_ROWS][KSLOTS];
@@ -293,28 +364,31 @@ __global__ void __launch_bounds__(RES_THREADS) bicg_resident_kernel(ResArgs a) {
   const int nslot = (int)((a.N + 511) / 512);
   double alpha = 0.0, omega = 0.0, beta = 0.0, pre_rho = 0.0, rnorm = 0.0, relres = 0.0;
   int done = 0, hit = 0, restart = 0;
+  auto publish_p = [&](unsigned epoch) {
+#pragma unroll
+    for (int m = 0; m < RES_ROWS; ++m) {
+      L.vec[m * RES_THREADS + t] = p[m];
+      if (own(m) && a.nblk > 1) ll_store(at32(a.ll0, v + m * S), at32(a.ll1, v + m * S), p[m], epoch);
+    }
+  };
+  publish_p(1);
 #pragma unroll 1
   for (int it = 0; it < a.chunk && !done; ++it) {
     const unsigned epoch = (unsigned)it + 1u;  // of the sums; the halos of p and s are numbered 2 it + 1 and 2 it + 2
     // ap = A p, ap . r0
     double r0[RES_ROWS];
 #pragma unroll
-    for (int m = 0; m < RES_ROWS; ++m) {
-      L.vec[m * RES_THREADS + t] = p[m];
-      if (own(m) && a.nblk > 1) ll_store(at32(a.ll0, v + m * S), at32(a.ll1, v + m * S), p[m], 2 * epoch - 1);
-      r0[m] = own(m) ? *at32(a.r0, v + m * S) : 0.0;
-    }
+    for (int m = 0; m < RES_ROWS; ++m) r0[m] = own(m) ? *at32(a.r0, v + m * S) : 0.0;
     __syncthreads();  // every wave has issued its words (RES_SPIN)
     resident_halo(L, a, 2 * epoch - 1);
     __syncthreads();
+    if (L.stuck) break;  // a wait reached its bound (uniform: set before this barrier or after the next)
     resident_rows(L, val, pos, ap);
+    double acc1[RES_ROWS], acc2[RES_ROWS];
 #pragma unroll
-    for (int m = 0; m < RES_ROWS; ++m) {
-      double acc = 0.0;
-      if (own(m)) acc += ap[m] * r0[m];
-      acc = wave_sum(acc);
-      if (lane == 0) L.wsum[0][m][wid] = acc;
-    }
+    for (int m = 0; m < RES_ROWS; ++m) acc1[m] = own(m) ? fma(ap[m], r0[m], 0.0) : 0.0;
+    const double w1 = wave_sum4(acc1[0], acc1[1], acc1[2], acc1[3]);
+    if (lane >= 60) L.wsum[0][lane - 60][wid] = w1;
     __syncthreads();
     resident_put_rows<1>(a, L, a.red[0], epoch);
     double ta[1];
@@ -333,17 +407,14 @@ __global__ void __launch_bounds__(RES_THREADS) bicg_resident_kernel(ResArgs a) {
     resident_rows(L, val, pos, as);
 #pragma unroll
     for (int m = 0; m < RES_ROWS; ++m) {
-      double acc0 = 0.0, acc1 = 0.0;
-      if (own(m)) {
-        acc0 += as[m] * s[m];
-        acc1 += as[m] * as[m];
-      }
-      acc0 = wave_sum(acc0);
-      acc1 = wave_sum(acc1);
-      if (lane == 0) {
-        L.wsum[0][m][wid] = acc0;
-        L.wsum[1][m][wid] = acc1;
-      }
+      acc1[m] = own(m) ? fma(as[m], s[m], 0.0) : 0.0;
+      acc2[m] = own(m) ? fma(as[m], as[m], 0.0) : 0.0;
+    }
+    const double w2 = wave_sum4(acc1[0], acc1[1], acc1[2], acc1[3]);
+    const double w3 = wave_sum4(acc2[0], acc2[1], acc2[2], acc2[3]);
+    if (lane >= 60) {
+      L.wsum[0][lane - 60][wid] = w2;
+      L.wsum[1][lane - 60][wid] = w3;
     }
     __syncthreads();
     resident_put_rows<2>(a, L, a.red[1], epoch);
@@ -367,46 +438,45 @@ __global__ void __launch_bounds__(RES_THREADS) bicg_resident_kernel(ResArgs a) {
         acc[1] += rn * r0[m];
       }
     }
-    acc[0] = wave_sum(acc[0]);
-    acc[1] = wave_sum(acc[1]);
-    if (lane == 0) {
-      L.wsum[0][0][wid] = acc[0];
-      L.wsum[1][0][wid] = acc[1];
-    }
+    const double wx = wave_sum2(acc[0], acc[1]);
+    if (lane >= 62) L.wsum[lane - 62][0][wid] = wx;
     __syncthreads();
     resident_put_xr(a, L, a.red[2], epoch);
+    const double ao = alpha / omega;
     double tc[2];
     resident_total<2>(a, L, a.red[2], a.nbx, epoch, tc);
-    if (L.stuck) {  // a wait reached its bound
-      if (t == 0) __hip_atomic_store(&a.ks->pad1, (int)RES_STUCK, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      return;
-    }
-    // the stop test, beta and the restart rule (conv_finalize)
+    // beta, the restart rule and the next p (conv_finalize, p_update_kernel),
+    // on its way before the stop test: nothing reads it after the last iteration
+    const double next_beta = ao * (tc[1] / rho);
+    const int next_restart = (L.timestep < 10 || fabs(rho) > L.restart_tol) ? 0 : 1;
+#pragma unroll
+    for (int m = 0; m < RES_ROWS; ++m) p[m] = next_restart ? r[m] : r[m] + next_beta * (p[m] - omega * ap[m]);
+    publish_p(2 * epoch + 1);
     rnorm = sqrt(tc[0]);
-    relres = rnorm / norm0;
-    if (relres < tol) {
+    relres = rnorm / L.norm0;
+    if (relres < L.tol) {
       done = 1;
-    } else if (iters >= maxit) {
+    } else if (iters >= L.maxit) {
       done = 1;
       hit = 1;
     } else {
       pre_rho = rho;
       rho = tc[1];
-      beta = (alpha / omega) * (rho / pre_rho);
-      restart = (timestep < 10 || fabs(pre_rho) > restart_tol) ? 0 : 1;
+      beta = next_beta;
+      restart = next_restart;
       restarts += restart;
       iters += 1;
       if (restart) {
 #pragma unroll
-        for (int m = 0; m < RES_ROWS; ++m) {
-          p[m] = r[m];
+        for (int m = 0; m < RES_ROWS; ++m)
           if (own(m)) *at32(a.r0, v + m * S) = r[m];
-        }
-      } else {
-#pragma unroll
-        for (int m = 0; m < RES_ROWS; ++m) p[m] = r[m] + beta * (p[m] - omega * ap[m]);
       }
     }
+  }
+  __syncthreads();
+  if (L.stuck) {
+    if (t == 0) __hip_atomic_store(&a.ks->pad1, (int)RES_STUCK, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return;
   }
   if (!done) {  // the next launch goes on from here
 #pragma unroll
