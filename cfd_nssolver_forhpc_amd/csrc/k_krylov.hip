@@ -307,36 +307,69 @@ __global__ void __launch_bounds__(256) xr_update_kernel(int64_t N, const KrylovS
 }
 
 // stop test, beta and the restart rule (bicgstabRe2.hpp:137-183)
-// the scalars after an iteration with (r . r) = rr, (r . r0) = rho
-__device__ inline KrylovScalars conv_next(KrylovScalars k, double rr, double rho) {
-  const double pre_rho = k.rho;
-  k.rnorm = sqrt(rr);
-  k.relres = k.rnorm / k.norm0;
-  if (k.relres < k.tol) {
-    k.done = 1;
-  } else if (k.iters >= k.maxit) {
-    k.done = 1;
-    k.hit_maxit = 1;
+// The scalars after an iteration with (r . r) = rr, (r . r0) = rho, from those
+// within it (`in`) into those between iterations (`out`, the same or another
+// copy, whose constants are there).  Field by field: a copy of the structure
+// lands in scratch memory.
+struct ConvNext {
+  double rnorm, relres, beta;
+  int stop, hit, restart;  // stop: done after this iteration
+};
+__device__ inline ConvNext conv_next(const KrylovScalars *in, double rr, double rho) {
+  ConvNext n;
+  const double pre_rho = in->rho;
+  n.rnorm = sqrt(rr);
+  n.relres = n.rnorm / in->norm0;
+  const bool converged = n.relres < in->tol;
+  n.hit = !converged && in->iters >= in->maxit;
+  n.stop = converged || n.hit;
+  n.beta = (in->alpha / in->omega) * (rho / pre_rho);
+  n.restart = (in->timestep < 10 || fabs(pre_rho) > in->restart_tol) ? 0 : 1;
+  return n;
+}
+__device__ inline void conv_store(const KrylovScalars *in, KrylovScalars *out, const ConvNext &n, double rho) {
+  const double pre_rho = in->rho, alpha = in->alpha, omega = in->omega;
+  const int iters = in->iters, restarts = in->restarts;
+  out->alpha = alpha;
+  out->omega = omega;
+  out->rnorm = n.rnorm;
+  out->relres = n.relres;
+  if (n.stop) {
+    out->done = 1;
+    if (n.hit) out->hit_maxit = 1;
   } else {
-    k.pre_rho = pre_rho;
-    k.rho = rho;
-    k.beta = (k.alpha / k.omega) * (rho / pre_rho);
-    k.restart = (k.timestep < 10 || fabs(pre_rho) > k.restart_tol) ? 0 : 1;
-    k.restarts += k.restart;
-    k.iters += 1;
+    out->pre_rho = pre_rho;
+    out->rho = rho;
+    out->beta = n.beta;
+    out->restart = n.restart;
+    out->restarts = restarts + n.restart;
+    out->iters = iters + 1;
   }
-  return k;
+}
+// K2's copy of the scalars between iterations (in) for those within (out)
+__device__ inline void begin_iteration(const KrylovScalars *in, KrylovScalars *out, double alpha) {
+  const int done = in->done;
+  out->rho = in->rho;
+  out->norm0 = in->norm0;
+  out->tol = in->tol;
+  out->restart_tol = in->restart_tol;
+  out->iters = in->iters;
+  out->maxit = in->maxit;
+  out->timestep = in->timestep;
+  out->restarts = in->restarts;
+  out->done = done;
+  if (!done) out->alpha = alpha;
 }
 
 template <int C>
 __global__ void __launch_bounds__(FIN_THREADS) conv_finalize(const double *part, int nblk, const KrylovScalars *in,
                                                              KrylovScalars *out) {
-  const KrylovScalars k = *in;
+  const int done = in->done;
   asm volatile("" ::: "memory");
   double tot[2];
   combine_slots<C>(part, nblk, tot);
-  if (k.done) return;
-  if (threadIdx.x == 0) *out = conv_next(k, tot[0], tot[1]);
+  if (done) return;
+  if (threadIdx.x == 0) conv_store(in, out, conv_next(in, tot[0], tot[1]), tot[1]);
 }
 
 void launch_alpha_finalize(const double *part, int nblk, KrylovScalars *ks, hipStream_t st) {
@@ -465,11 +498,7 @@ __global__ void __launch_bounds__(BT, BT == 1024 ? 8 : 4) s_fold_kernel(int64_t 
   combine_folded<BT, C>(part, nblk, tot);
   const int done = ks0->done;
   const double alpha = ks0->rho / tot[0];
-  if (t == 0) {
-    KrylovScalars k = *ks0;
-    if (!done) k.alpha = alpha;
-    *ks1 = k;
-  }
+  if (t == 0) begin_iteration(ks0, ks1, alpha);
   if (done) return;
 #pragma unroll
   for (int u = 0; u < ROWS; ++u)
@@ -535,18 +564,19 @@ __global__ void __launch_bounds__(256, 4) p_fold_kernel(int64_t N, const double 
   double tot[2];
   combine_folded<256, 1>(part, nblk, tot);
   if (ks1->done) return;
-  const KrylovScalars k = conv_next(*ks1, tot[0], tot[1]);
-  if (t == 0) *ks0 = k;
-  if (k.done) return;
+  const ConvNext n = conv_next(ks1, tot[0], tot[1]);
+  const double omega = ks1->omega;
+  if (t == 0) conv_store(ks1, ks0, n, tot[1]);
+  if (n.stop) return;
 #pragma unroll
   for (int u = 0; u < ROWS; ++u) {
     const int64_t r = t + u * step;
     if (r < N) {
-      if (k.restart) {
+      if (n.restart) {
         r0[r] = rv[u];
         p1[r] = rv[u];
       } else {
-        p1[r] = (T)((double)rv[u] + k.beta * ((double)pv[u] - k.omega * (double)av[u]));
+        p1[r] = (T)((double)rv[u] + n.beta * ((double)pv[u] - omega * (double)av[u]));
       }
     }
   }
