@@ -49,9 +49,9 @@ except (AttributeError, OSError):
 # algorithmic bytes per row.  The assembled ELL operator's FP64 products form its
 # entries again from the axis coefficients: SpMV x + y; with the dot of the
 # iteration's K1 r0 too; BiCGSTAB iteration K1 24, s 24, K3 16, x/r 56, p 32.
-# An uploaded matrix is read (..._stored): 7 x (val + col) more.  SPE x + jp + y;
-# RB-SOR sweep 84 + x + b + x(w) + x(nbr)
-BYTES = {"spmv_fp64": 16, "spmv_fp32": 64, "spe_fp64": 24, "bicg_iter": 152, "sor_sweep": 116,
+# An uploaded matrix is read (..._stored): 7 x (val + col) more.  SPE x + y (its
+# diagonal is formed again too); RB-SOR sweep 84 + x + b + x(w) + x(nbr)
+BYTES = {"spmv_fp64": 16, "spmv_fp32": 64, "spe_fp64": 16, "bicg_iter": 152, "sor_sweep": 116,
          "copy": 16, "predictor": 48, "spmv_dot": 24, "spmv_stored": 100, "spmv_dot_stored": 108,
          "bicg_iter_stored": 320}
 
