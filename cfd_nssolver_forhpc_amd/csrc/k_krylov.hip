@@ -589,12 +589,15 @@ __global__ void __launch_bounds__(256, 4) p_fold_kernel(int64_t N, const double 
 // 200x104x40 60 -> 47.5 (ALL), 190x210x40 81 -> 70 (K2).  K4 and K5 folded at
 // 190x210x40 take 22.7 + 14.8 us in blocks of 1024 threads that are all in
 // flight at once, unfolded 3.7 + 17.0 + 4.3 + 11.5: the rows wait for the
-// reduction, then all are stored at once.  Past 4096 partials every block would
-// read more than 33 KB of them.
+// reduction, then all are stored at once.  The same holds K2 back where its
+// blocks are more than the CUs take at once (two each, 4096 rows a block):
+// 41.7 us at 512x256x64 with 4096 partials, 33 + 3.7 unfolded.  Past 4096
+// partials every block would read more than 33 KB of them.
 enum class Fold { NONE, K2, ALL };
-Fold fold_of(int nd, int nvb) {
+constexpr int64_t FOLD_K2_ROWS = 512 * 4096;
+Fold fold_of(int nd, int nvb, int64_t N) {
   if (nd <= FIN_THREADS && nvb <= FIN_THREADS) return Fold::ALL;
-  return nd <= 4 * FIN_THREADS ? Fold::K2 : Fold::NONE;
+  return nd <= 4 * FIN_THREADS && N <= FOLD_K2_ROWS ? Fold::K2 : Fold::NONE;
 }
 
 template <typename T>
@@ -705,7 +708,7 @@ hipError_t launch_iters(Ctx &c, const OpArgs &a, const Vecs<T> &v, KrylovScalars
   const bool pairs = spe && spe_pairs(a, tiles, {v.p1, v.ap, v.r0, v.s1, v.as});
   const int nbs = spe ? (int)tiles.blocks : nb;
   const int pp = std::is_same<T, double>::value ? ell_grid_period(a, nb, SPMV_DOT_THREADS, {v.p1, v.ap, v.r0, v.s1, v.as}) : 0;
-  const Fold fold = fold_of(nbs, nbx);
+  const Fold fold = fold_of(nbs, nbx, N);
   KrylovScalars *ks3 = fold == Fold::NONE ? ks : ks + 1;  // from K2 to K4
   for (int it = 0; it < nit; ++it) {
     if (pp)
@@ -908,7 +911,7 @@ int launch_pc_iters(Ctx &c, const OpArgs &a, const PVecs<T> &v, KrylovScalars *k
   const bool pairs = spe && spe_pairs(a, tiles, {v.ph, v.v, v.r0, v.sh, v.t, v.s1});
   const int nbs = spe ? (int)tiles.blocks : nb;
   const int pp = std::is_same<T, double>::value ? ell_grid_period(a, nb, 256, {v.ph, v.v, v.r0, v.sh, v.t, v.s1}) : 0;
-  const Fold fold = fold_of(nbs, nbu);
+  const Fold fold = fold_of(nbs, nbu, N);
   KrylovScalars *ks3 = fold == Fold::NONE ? ks : ks + 1;  // from K2 to K4
   for (int it = 0; it < nit; ++it) {
     int rc = precondition<T>(c, v.p1, v.ph, ks, pc32);
