@@ -450,7 +450,9 @@ __global__ void __launch_bounds__(256) mg_split_sweep_kernel(MGView L, MGView C,
 // drained every load before its use and an FP64 pass took 59-68 us.  One
 // workgroup a CU: tiles of 24 rows and 23 planes at that size, each computing
 // 1.5 times its cells, are what 256 CUs leave (two workgroups a CU, with twice
-// the overlap: a cycle of 490 us against 422).  Three timesteps
+// the overlap: a cycle of 490 us against 422).  Choosing tiles by waves and
+// steps (fused_shape) instead of the fewest tiles of rows: 396 -> 385 us a
+// cycle there, 159 -> 152 at 256x128x32, 151 -> 140 at 200x104x40.  Three timesteps
 // there went from 73.9 to 57.2 ms (FP64; mixed 65.5 to 50.8), the 256x128x32
 // adjoint from 110 to 83 ms.
 //
@@ -461,6 +463,7 @@ __global__ void __launch_bounds__(256) mg_split_sweep_kernel(MGView L, MGView C,
 // and 303 -> 278.  It reads pairs of cells, so nz has to be even.
 constexpr int FUSED_THREADS = 1024;
 constexpr int FUSED_RING = 6;     // planes of x and b a thread holds
+constexpr int FUSED_WAVES = 16, FUSED_START = 3;  // fused_shape's cost
 constexpr int FUSED_CHUNK = 512;  // planes of a run at most (its coefficients sit in LDS)
 
 struct FusedShape {
@@ -1182,21 +1185,30 @@ FusedShape fused_shape(const MGView &v, int ns) {
   s.hz = (v.nz + 1) / 2;
   const int rmax = FUSED_THREADS / s.hz;
   if (rmax < 4 * ns) return s;
-  if (v.ny <= rmax) {
-    s.R = s.TJ = v.ny;
-    s.njt = 1;
-    s.halo = 0;
-  } else {
-    s.halo = ns;
-    const int tj = rmax - 2 * ns;
-    s.njt = (v.ny + tj - 1) / tj;
-    s.TJ = (v.ny + s.njt - 1) / s.njt;
-    s.R = s.TJ + 2 * ns;
+  // As many tiles as leave one workgroup a CU, split between rows and planes
+  // for the least time: a step takes about FUSED_WAVES + the waves of a
+  // workgroup (latency and instructions; fitted to the passes of 512x256x64,
+  // its levels, 256x128x32 and 200x104x40), and a run of `chunk` planes takes
+  // chunk + 2 (ns - 1) steps and some for its start.
+  const int fewest = v.ny <= rmax ? 1 : (v.ny + rmax - 2 * ns - 1) / (rmax - 2 * ns);
+  int64_t best = INT64_MAX;
+  for (int njt = fewest; njt < fewest + 64 && njt <= v.ny; ++njt) {
+    FusedShape t = s;
+    t.njt = njt;
+    t.TJ = (v.ny + njt - 1) / njt;
+    t.halo = njt > 1 ? ns : 0;
+    t.R = t.TJ + 2 * t.halo;
+    if (t.R > rmax || (njt - 1) * t.TJ >= v.ny) continue;
+    const int runs = std::max(1, 256 / njt);
+    t.chunk = std::min((v.nx + runs - 1) / runs, FUSED_CHUNK);
+    t.nci = (v.nx + t.chunk - 1) / t.chunk;
+    const int64_t rounds = ((int64_t)njt * t.nci + 255) / 256;
+    const int64_t cost = rounds * ((t.R * t.hz + 63) / 64 + FUSED_WAVES) * (t.chunk + 2 * (ns - 1) + FUSED_START);
+    if (cost < best) {
+      best = cost;
+      s = t;
+    }
   }
-  // one workgroup a CU: as many runs of planes as keep the tiles within 256
-  const int runs = std::max(1, 256 / s.njt);
-  s.chunk = std::min((v.nx + runs - 1) / runs, FUSED_CHUNK);
-  s.nci = (v.nx + s.chunk - 1) / s.chunk;
   return s;
 }
 

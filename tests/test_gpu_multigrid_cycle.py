@@ -145,7 +145,8 @@ def grids(name):
     ((64, 32, 16), 1, False, False), ((48, 48, 64), 4, True, False), ((40, 96, 64), 4, False, True),
     ((44, 100, 40), 5, False, False), ((24, 20, 132), 4, True, False), ((24, 16, 260), 2, False, False),
     ((34, 50, 21), 4, False, False), ((20, 36, 27), 6, False, True), ((16, 12, 8), 4, False, False),
-    ((50, 26, 10), 4, False, False), ("stretched", 4, True, False), ((8, 64, 64), 4, False, True)])
+    ((50, 26, 10), 4, False, False), ("stretched", 4, True, False), ((8, 64, 64), 4, False, True),
+    ((6, 640, 128), 4, False, False), ((2, 33, 32), 4, True, False)])
 def test_two_iterations_against_numpy(require_gpu, ncal, nu, periodic, mixed):
     print(f"multigrid cycle ncal={ncal} nu={nu} periodic={periodic} mixed={mixed}", flush=True)
     grid = grids(ncal)
