@@ -129,6 +129,10 @@ class CfdSolverCounters(C.Structure):
                 ("iters", C.c_longlong)]
 
 
+class CfdOneLaunchCounters(C.Structure):
+    _fields_ = [("finished", C.c_longlong), ("handed_back", C.c_longlong)]
+
+
 class CfdAdjointStats(C.Structure):
     _fields_ = [
         ("steps", C.c_int), ("checkpoints", C.c_int), ("recomputed_steps", C.c_int),
@@ -287,6 +291,8 @@ def _declare(L: C.CDLL) -> None:
                               C.c_int),
         "cfd_checkpoint_save": ([vp, C.c_char_p], C.c_int),
         "cfd_get_solver_counters": ([vp, C.POINTER(CfdSolverCounters)], C.c_int),
+        "cfd_get_one_launch_counters": ([vp, C.POINTER(CfdOneLaunchCounters)], C.c_int),
+        "cfd_set_one_launch_bounds": ([vp, C.c_int, C.c_int, C.c_int], C.c_int),
         "cfd_phase_timing": ([vp, C.c_int], C.c_int),
         "cfd_phase_times": ([vp, dp, ip], C.c_int),
         "cfd_checkpoint_load": ([vp, C.c_char_p], C.c_int),

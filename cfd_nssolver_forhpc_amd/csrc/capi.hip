@@ -1185,6 +1185,25 @@ int cfd_get_solver_counters(cfd_ctx *ctx, cfd_solver_counters *out) {
   return CFD_OK;
 }
 
+int cfd_get_one_launch_counters(cfd_ctx *ctx, cfd_one_launch_counters *out) {
+  CTX_CHECK(ctx);
+  if (!out) return fail(CFD_ERR_ARG, "out is NULL");
+  const OneLaunch &o = reinterpret_cast<Ctx *>(ctx)->one;
+  out->finished = o.finished;
+  out->handed_back = o.handed_back;
+  return CFD_OK;
+}
+
+int cfd_set_one_launch_bounds(cfd_ctx *ctx, int arrive, int wait, int wait_first) {
+  CTX_CHECK(ctx);
+  if (wait < 0 || wait_first < 0) return fail(CFD_ERR_ARG, "the bounds of a wait must be >= 0");
+  OneLaunch &o = reinterpret_cast<Ctx *>(ctx)->one;
+  o.arrive = arrive;
+  o.wait = wait;
+  o.wait_first = wait_first;
+  return CFD_OK;
+}
+
 // ---- measurement -----------------------------------------------------------------
 int cfd_time_kernel(cfd_ctx *ctx, int what, int nrep, double *ms_avg) {
   CTX_CHECK(ctx);

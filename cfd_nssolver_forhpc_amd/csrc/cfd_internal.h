@@ -78,6 +78,14 @@ struct RedWork {
 };
 enum RedSite { RS_SPMV_DOT = 0, RS_SPMV_DOT2, RS_XR, RS_INIT, RS_NORM, RS_DRAG, RS_MAX, RS_MISC, RED_SITES };
 
+// The pressure solves that run as one kernel (dev_exchange.h): the bounds of
+// their waits in polls (0: the default, arrive < 0: no such solve) and how many
+// solves they finished or handed back to the launches.
+struct OneLaunch {
+  int arrive = 0, wait = 0, wait_first = 0;
+  long long finished = 0, handed_back = 0;
+};
+
 struct Ctx {
   int device = 0;
   hipStream_t stream = nullptr;
@@ -160,6 +168,7 @@ struct Ctx {
   // the step's prediction (u, v, w; ghosted), kept by its first pass
   double *pred[3] = {nullptr, nullptr, nullptr};
   double *viseff = nullptr;  // Smagorinsky eddy viscosity (N), when prm.les
+  OneLaunch one;
 };
 
 // k_mg.hip

@@ -58,17 +58,30 @@ constexpr unsigned RES_SPIN = 1u << 22;
 // (tens of milliseconds: the CUs are held by other kernels)
 constexpr unsigned RES_ARRIVE_SPIN = 1u << 15;
 
+// the bounds of a launch: the arrival's, the first workgroup's and the others'
+struct ResBounds {
+  unsigned arrive, first, others;
+};
+inline ResBounds res_bounds(const OneLaunch &o) {
+  ResBounds b;
+  b.arrive = o.arrive > 0 ? (unsigned)o.arrive : RES_ARRIVE_SPIN;
+  b.others = o.wait > 0 ? (unsigned)o.wait : RES_SPIN;
+  b.first = o.wait_first > 0 ? (unsigned)o.wait_first : b.others;
+  return b;
+}
+__device__ inline unsigned res_spin(const ResBounds &b) { return blockIdx.x ? b.others : b.first; }
+
 // Loads U pairs of words at a time until each carries the epoch: get(u) is
 // the position of the u-th pair in w0 / w1 (RES_NONE: none), put(u, v) takes
 // its value.  False when the bound was reached.
 constexpr unsigned RES_NONE = ~0u;
 template <int U, typename G, typename P>
-__device__ inline bool ll_fetch(const uint64_t *p0, const uint64_t *p1, unsigned epoch, G get, P put) {
+__device__ inline bool ll_fetch(const uint64_t *p0, const uint64_t *p1, unsigned epoch, unsigned bound, G get, P put) {
   unsigned at[U];
 #pragma unroll
   for (int u = 0; u < U; ++u) at[u] = get(u);
 #pragma unroll 1
-  for (unsigned spin = 0; spin < RES_SPIN; ++spin) {
+  for (unsigned spin = 0; spin < bound; ++spin) {
     uint64_t w0[U], w1[U];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -95,14 +108,14 @@ __device__ inline bool ll_fetch(const uint64_t *p0, const uint64_t *p1, unsigned
 // one sets RES_GO, and a workgroup that waits too long (other kernels hold the
 // CUs) sets RES_ABORT instead; the first of the two to be set stands for all.
 // What does not fit a workgroup (fits) aborts the same way.
-__device__ inline int resident_arrive(KrylovScalars *ks, int nblk, int *state, bool fits) {
+__device__ inline int resident_arrive(KrylovScalars *ks, int nblk, int *state, bool fits, unsigned bound) {
   if (threadIdx.x == 0) {
     unsigned *const st = reinterpret_cast<unsigned *>(&ks->pad1);
     if (!fits) atomicCAS(st, (unsigned)RES_PENDING, (unsigned)RES_ABORT);
     if (atomicAdd(reinterpret_cast<unsigned *>(&ks->pad0), 1u) + 1u == (unsigned)nblk)
       atomicCAS(st, (unsigned)RES_PENDING, (unsigned)RES_GO);
     unsigned s = RES_PENDING;
-    for (unsigned spin = 0; spin < RES_ARRIVE_SPIN; ++spin) {
+    for (unsigned spin = 0; spin < bound; ++spin) {
       s = __hip_atomic_load(st, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       if (s != RES_PENDING) break;
     }

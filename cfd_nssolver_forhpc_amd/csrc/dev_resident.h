@@ -61,6 +61,7 @@ struct ResArgs {
   uint64_t *red[3];           // exchanged sums: 2 x RES_RED_WORDS words each
   KrylovScalars *ks;          // pad0: arrivals, pad1: RES_* state
   int chunk;                  // iterations this launch runs at most
+  ResBounds bounds;
 };
 
 struct ResLds {
@@ -79,7 +80,7 @@ __device__ inline void resident_halo(ResLds &L, const ResArgs &a, unsigned epoch
   const int nh = L.nhalo;
   for (int e0 = (int)threadIdx.x; e0 < nh; e0 += RES_THREADS * RES_FETCH) {
     const bool ok = ll_fetch<RES_FETCH>(
-        a.ll0, a.ll1, epoch,
+        a.ll0, a.ll1, epoch, res_spin(a.bounds),
         [&](int u) { return e0 + u * RES_THREADS < nh ? (unsigned)L.hcol[e0 + u * RES_THREADS] : RES_NONE; },
         [&](int u, bool have, double v) {
           if (have) L.vec[RES_OWN + e0 + u * RES_THREADS] = v;
@@ -178,7 +179,7 @@ __device__ inline void resident_put_rows(const ResArgs &a, ResLds &L, uint64_t *
       const double *wf = L.wsum[q][mf] + 4 * hf;
       s = ((wf[0] + wf[1]) + wf[2]) + wf[3];
     } else if (!ll_fetch<1>(
-                   red, red + 1, epoch, [&](int) { return (unsigned)(q * RES_RED_WORDS + slot * 4 + 2); },
+                   red, red + 1, epoch, res_spin(a.bounds), [&](int) { return (unsigned)(q * RES_RED_WORDS + slot * 4 + 2); },
                    [&](int, bool, double x) { s = x; })) {
       L.stuck = 1;
     }
@@ -219,7 +220,7 @@ __device__ inline void resident_total(const ResArgs &a, ResLds &L, const uint64_
       }
     } else {
       const bool ok = ll_fetch<2 * NV>(
-          red, red + 1, epoch,
+          red, red + 1, epoch, res_spin(a.bounds),
           [&](int u) {
             const int q = u % NV, slot = lane + u / NV * 64;
             return slot < nslot ? (unsigned)(q * RES_RED_WORDS + slot * 4) : RES_NONE;
@@ -247,7 +248,7 @@ __device__ inline void resident_total(const ResArgs &a, ResLds &L, const uint64_
       const int slot = (int)threadIdx.x + half * RES_THREADS;
       const bool mine = slot < nslot;
       const bool ok = ll_fetch<NV>(
-          red, red + 1, epoch, [&](int q) { return mine ? (unsigned)(q * RES_RED_WORDS + slot * 4) : RES_NONE; },
+          red, red + 1, epoch, res_spin(a.bounds), [&](int q) { return mine ? (unsigned)(q * RES_RED_WORDS + slot * 4) : RES_NONE; },
           [&](int q, bool have, double x) { v[q] = have ? x : 0.0; });
       if (!ok) L.stuck = 1;
       // combine_partials adds the slot to a zero
@@ -360,7 +361,7 @@ __global__ void __launch_bounds__(RES_THREADS) bicg_resident_kernel(ResArgs a) {
     p[m] = own(m) ? *at32(a.p1, row) : 0.0;
   }
   fits = __syncthreads_and(fits);
-  if (resident_arrive(a.ks, a.nblk, &L.state, fits) != RES_GO) return;
+  if (resident_arrive(a.ks, a.nblk, &L.state, fits, a.bounds.arrive) != RES_GO) return;
   const int nslot = (int)((a.N + 511) / 512);
   double alpha = 0.0, omega = 0.0, beta = 0.0, pre_rho = 0.0, rnorm = 0.0, relres = 0.0;
   int done = 0, hit = 0, restart = 0;

@@ -790,8 +790,12 @@ int solve_resident(Ctx &c, const OpArgs &a, const Vecs<double> &v, KrylovScalars
   for (int q = 0; q < 3; ++q) r.red[q] = reinterpret_cast<uint64_t *>(red_part_host(c, sites[q]));
   r.ks = ks;
   r.chunk = 4096;  // bounds one launch to some tens of milliseconds
+  r.bounds = res_bounds(c.one);
   ResidentSlots slots;
-  if (!slots.take(c.device, r.nblk)) return CFD_OK;
+  if (c.one.arrive < 0 || !slots.take(c.device, r.nblk)) {
+    c.one.handed_back++;
+    return CFD_OK;
+  }
   const int nbc = blocks_for(std::max<int64_t>(a.N, 2 * RES_RED_WORDS), 256, 1 << 30);
   for (;;) {
     resident_clear_kernel<<<nbc, 256, 0, c.stream>>>(r);
@@ -800,9 +804,13 @@ int solve_resident(Ctx &c, const OpArgs &a, const Vecs<double> &v, KrylovScalars
     CFD_HIP(hipMemcpyAsync(c.hks, ks, sizeof(KrylovScalars), hipMemcpyDeviceToHost, c.stream));
     CFD_HIP(hipStreamSynchronize(c.stream));
     if (c.hks->pad1 == RES_STUCK) return fail(CFD_ERR_RUNTIME, "resident BiCGSTAB: a workgroup stopped answering");
-    if (c.hks->pad1 != RES_GO) return CFD_OK;
+    if (c.hks->pad1 != RES_GO) {
+      c.one.handed_back++;
+      return CFD_OK;
+    }
     if (c.hks->done) break;
   }
+  c.one.finished++;
   *solved = true;
   return CFD_OK;
 }

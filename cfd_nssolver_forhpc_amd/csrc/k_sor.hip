@@ -338,6 +338,7 @@ struct SorArgs {
   uint64_t *mx;         // maxima: [sweep parity][word][workgroup]
   KrylovScalars *ks;    // pad0: arrivals, pad1: RES_* state
   int nblk, chunk;      // chunk: sweeps this launch runs at most
+  ResBounds bounds;
 };
 
 __global__ void __launch_bounds__(SORR_THREADS) sorp_resident_kernel(DevGrid g, double omega, int wrapz,
@@ -421,7 +422,7 @@ __global__ void __launch_bounds__(SORR_THREADS) sorp_resident_kernel(DevGrid g, 
     }
   }
   fits = __syncthreads_and(fits);
-  if (resident_arrive(a.ks, a.nblk, &L.state, fits) != RES_GO) return;
+  if (resident_arrive(a.ks, a.nblk, &L.state, fits, a.bounds.arrive) != RES_GO) return;
 
   double mx = 0.0, old = 0.0;
   // colour c of the sweep with exchange number epoch (1, 2, 3, ..)
@@ -451,7 +452,7 @@ __global__ void __launch_bounds__(SORR_THREADS) sorp_resident_kernel(DevGrid g, 
     if (tid < busy) return;
     for (int e0 = tid - busy; e0 < nh; e0 += 4 * step) {
       const bool ok = ll_fetch<4>(
-          a.ll0, a.ll1, epoch, [&](int u) { return e0 + u * step < nh ? (unsigned)L.hrow[c][e0 + u * step] : RES_NONE; },
+          a.ll0, a.ll1, epoch, res_spin(a.bounds), [&](int u) { return e0 + u * step < nh ? (unsigned)L.hrow[c][e0 + u * step] : RES_NONE; },
           [&](int u, bool have, double v) {
             if (have) L.p[2 * OWN + c * HALO + e0 + u * step] = v;
           });
@@ -472,7 +473,7 @@ __global__ void __launch_bounds__(SORR_THREADS) sorp_resident_kernel(DevGrid g, 
         double v = 0.0;
         const uint64_t *w = a.mx + ((s - 1) & 1) * 2 * SORR_BLOCKS;
         const bool ok = ll_fetch<1>(
-            w, w + SORR_BLOCKS, (unsigned)s, [&](int) { return tid < a.nblk ? (unsigned)tid : RES_NONE; },
+            w, w + SORR_BLOCKS, (unsigned)s, res_spin(a.bounds), [&](int) { return tid < a.nblk ? (unsigned)tid : RES_NONE; },
             [&](int, bool have, double x) { v = have ? x : 0.0; });
         if (!ok) L.stuck = 1;
         v = wave_max(v);
@@ -547,8 +548,12 @@ int sorp_resident(Ctx &c, double omega, const double *cf6, bool *solved) {
   a.ks = c.ks;
   a.nblk = (int)((npair + SORR_THREADS - 1) / SORR_THREADS);
   a.chunk = 4096;  // bounds one launch to some tens of milliseconds
+  a.bounds = res_bounds(c.one);
   ResidentSlots slots;
-  if (!slots.take(c.device, a.nblk)) return CFD_OK;
+  if (c.one.arrive < 0 || !slots.take(c.device, a.nblk)) {
+    c.one.handed_back++;
+    return CFD_OK;
+  }
   for (;;) {
     sorp_clear_kernel<<<blocks_for(std::max<int64_t>(g.N, 4 * SORR_BLOCKS), 256, 1 << 30), 256, 0, c.stream>>>(g.N, a);
     sorp_resident_kernel<<<a.nblk, SORR_THREADS, 0, c.stream>>>(g, omega, c.prm.periodic_z, cf6, c.f[CFD_P], a);
@@ -556,9 +561,13 @@ int sorp_resident(Ctx &c, double omega, const double *cf6, bool *solved) {
     CFD_HIP(hipMemcpyAsync(c.hks, c.ks, sizeof(KrylovScalars), hipMemcpyDeviceToHost, c.stream));
     CFD_HIP(hipStreamSynchronize(c.stream));
     if (c.hks->pad1 == RES_STUCK) return fail(CFD_ERR_RUNTIME, "resident SorPipeLine: a workgroup stopped answering");
-    if (c.hks->pad1 != RES_GO) return CFD_OK;
+    if (c.hks->pad1 != RES_GO) {
+      c.one.handed_back++;
+      return CFD_OK;
+    }
     if (c.hks->done) break;
   }
+  c.one.finished++;
   *solved = true;
   return CFD_OK;
 }

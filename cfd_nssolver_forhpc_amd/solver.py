@@ -298,6 +298,18 @@ class Simulation:
         check(self.lib.cfd_get_solver_counters(self.h, C.byref(out)), "cfd_get_solver_counters")
         return {"solves": out.solves, "restarts": out.restarts, "resets": out.resets, "iters": out.iters}
 
+    def one_launch_counters(self) -> tuple:
+        """Pressure solves that ran as one kernel, and those that could have by
+        their size and were handed back to the launches."""
+        out = capi.CfdOneLaunchCounters()
+        check(self.lib.cfd_get_one_launch_counters(self.h, C.byref(out)), "cfd_get_one_launch_counters")
+        return out.finished, out.handed_back
+
+    def one_launch_bounds(self, arrive: int = 0, wait: int = 0, wait_first: int = 0):
+        """Bounds of the one-kernel solves' waits in polls; 0: the default,
+        arrive < 0: every solve by launches (cfd_set_one_launch_bounds)."""
+        check(self.lib.cfd_set_one_launch_bounds(self.h, arrive, wait, wait_first), "cfd_set_one_launch_bounds")
+
     def save_checkpoint(self, path):
         """Exact FP64 snapshot of the step state (cfd_checkpoint_save)."""
         check(self.lib.cfd_checkpoint_save(self.h, os.fsencode(path)), "cfd_checkpoint_save")

@@ -347,6 +347,23 @@ typedef struct cfd_solver_counters {
 } cfd_solver_counters;
 int cfd_get_solver_counters(cfd_ctx *ctx, cfd_solver_counters *out);
 
+/* Small pressure solves (BiCGSTAB in FP64 on an ELL operator of at most 524288
+   rows, SorPipeLine on at most about 262144 cells) run as one kernel, whose
+   workgroups hold a CU each and wait for each other's values; where that
+   cannot be done -- the CUs are taken, a workgroup's halo does not fit -- the
+   solve is handed back to launches of one kernel an operation, with the same
+   result bit for bit.  This context's tallies (a system too large for it is in
+   neither): */
+typedef struct cfd_one_launch_counters {
+  long long finished, handed_back;
+} cfd_one_launch_counters;
+int cfd_get_one_launch_counters(cfd_ctx *ctx, cfd_one_launch_counters *out);
+/* Bounds of the waits, in polls of the awaited memory, 0 for the default:
+   arrive, until every workgroup has its CU (negative: no solve of this context
+   runs as one kernel, for a GPU shared with others); wait, for a value once
+   they have; wait_first, the first workgroup's, for tests. */
+int cfd_set_one_launch_bounds(cfd_ctx *ctx, int arrive, int wait, int wait_first);
+
 /* ---- discrete adjoint (no reference counterpart) ---------------------- */
 /* Objective J = mean of the corrector pass's cD (virtualF_Int,
    virtualForceIntergrator.hpp:5-37) over steps [avg_from, nsteps) of a run
