@@ -59,7 +59,8 @@ struct ResArgs {
   double *x, *r0, *r1, *p1;
   uint64_t *ll0, *ll1;        // exchanged p and s: the two words of each row
   uint64_t *red[3];           // exchanged sums: 2 x RES_RED_WORDS words each
-  KrylovScalars *ks;          // pad0: arrivals, pad1: RES_* state
+  double *keep;               // x as it was before the solve
+  KrylovScalars *ks;          // pad0: arrivals, pad1: RES_* state; ks[1].restarts as it was before the solve
   int chunk;                  // iterations this launch runs at most
   ResBounds bounds;
 };
@@ -70,17 +71,20 @@ struct ResLds {
   double wsum[2][RES_ROWS][RES_THREADS / 64];
   double fin[2][FIN_THREADS / 64];
   double one[2][4][2];                     // block sums of a lone workgroup (at most 4 slots)
-  int nhalo, state, stuck;
+  int nhalo, state;
+  alignas(8) int stuck;                    // a wait reached its bound
+  int done;                                // the stop test's result, from the first wave
   double norm0, tol, restart_tol;
   int maxit, timestep;
 };
 
 // The workgroup's halo of the vector exchanged in ll, into its LDS entries.
+template <bool SET>
 __device__ inline void resident_halo(ResLds &L, const ResArgs &a, unsigned epoch) {
   const int nh = L.nhalo;
   for (int e0 = (int)threadIdx.x; e0 < nh; e0 += RES_THREADS * RES_FETCH) {
     const bool ok = ll_fetch<RES_FETCH>(
-        a.ll0, a.ll1, epoch, res_spin(a.bounds),
+        a.ll0, a.ll1, epoch, res_spin<SET>(a.bounds),
         [&](int u) { return e0 + u * RES_THREADS < nh ? (unsigned)L.hcol[e0 + u * RES_THREADS] : RES_NONE; },
         [&](int u, bool have, double v) {
           if (have) L.vec[RES_OWN + e0 + u * RES_THREADS] = v;
@@ -149,7 +153,7 @@ __device__ inline void resident_put(const ResArgs &a, ResLds &L, uint64_t *red, 
 // it: one more hop, in every second slab of an odd nbx.  (Leaving the five
 // parts for every reader to add instead took 58 us an iteration at 303750
 // rows against 30: each workgroup reads every slot.)
-template <int NV>
+template <int NV, bool SET>
 __device__ inline void resident_put_rows(const ResArgs &a, ResLds &L, uint64_t *red, unsigned epoch) {
   const int t = threadIdx.x;
   if (t >= NV * RES_ROWS * 2) return;
@@ -179,7 +183,7 @@ __device__ inline void resident_put_rows(const ResArgs &a, ResLds &L, uint64_t *
       const double *wf = L.wsum[q][mf] + 4 * hf;
       s = ((wf[0] + wf[1]) + wf[2]) + wf[3];
     } else if (!ll_fetch<1>(
-                   red, red + 1, epoch, res_spin(a.bounds), [&](int) { return (unsigned)(q * RES_RED_WORDS + slot * 4 + 2); },
+                   red, red + 1, epoch, res_spin<SET>(a.bounds), [&](int) { return (unsigned)(q * RES_RED_WORDS + slot * 4 + 2); },
                    [&](int, bool, double x) { s = x; })) {
       L.stuck = 1;
     }
@@ -203,7 +207,7 @@ __device__ inline void resident_put_xr(const ResArgs &a, ResLds &L, uint64_t *re
 // The totals of nslot slots in combine_partials' order: slot t belongs to
 // finalize thread t, whose 64 lanes are summed by wave_sum and whose 16 waves
 // in turn.
-template <int NV>
+template <int NV, bool SET>
 __device__ inline void resident_total(const ResArgs &a, ResLds &L, const uint64_t *red, int nslot, unsigned epoch,
                                       double (&tot)[NV]) {
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
@@ -211,7 +215,7 @@ __device__ inline void resident_total(const ResArgs &a, ResLds &L, const uint64_
   // Up to two of the finalize kernel's waves (N <= 65536): every wave of the
   // workgroup forms the total itself; the other waves' sums are zero.
   if (nslot <= 128) {
-    double v[2][NV];
+    double v[2][NV] = {};  // a wait that reaches its bound leaves zeros
     if (a.nblk == 1) {
 #pragma unroll
       for (int q = 0; q < NV; ++q) {
@@ -220,7 +224,7 @@ __device__ inline void resident_total(const ResArgs &a, ResLds &L, const uint64_
       }
     } else {
       const bool ok = ll_fetch<2 * NV>(
-          red, red + 1, epoch, res_spin(a.bounds),
+          red, red + 1, epoch, res_spin<SET>(a.bounds),
           [&](int u) {
             const int q = u % NV, slot = lane + u / NV * 64;
             return slot < nslot ? (unsigned)(q * RES_RED_WORDS + slot * 4) : RES_NONE;
@@ -248,7 +252,7 @@ __device__ inline void resident_total(const ResArgs &a, ResLds &L, const uint64_
       const int slot = (int)threadIdx.x + half * RES_THREADS;
       const bool mine = slot < nslot;
       const bool ok = ll_fetch<NV>(
-          red, red + 1, epoch, res_spin(a.bounds), [&](int q) { return mine ? (unsigned)(q * RES_RED_WORDS + slot * 4) : RES_NONE; },
+          red, red + 1, epoch, res_spin<SET>(a.bounds), [&](int q) { return mine ? (unsigned)(q * RES_RED_WORDS + slot * 4) : RES_NONE; },
           [&](int q, bool have, double x) { v[q] = have ? x : 0.0; });
       if (!ok) L.stuck = 1;
       // combine_partials adds the slot to a zero
@@ -302,6 +306,7 @@ __device__ inline void resident_rows(const ResLds &L, const double (&val)[RES_RO
 // launch_iters<double>'s kernels, expression for expression.  x and r0, which
 // nothing gathers, stay in memory (each thread its own rows; the register
 // file holds the rest).
+template <bool SET>
 __global__ void __launch_bounds__(RES_THREADS) bicg_resident_kernel(ResArgs a) {
   __shared__ ResLds L;
   const int t = threadIdx.x, lane = t & 63, wid = t >> 6;
@@ -315,7 +320,7 @@ __global__ void __launch_bounds__(RES_THREADS) bicg_resident_kernel(ResArgs a) {
   if (t == 0) {
     L.nhalo = a.nblk > 1 ? 1 : 0;  // entry 0: column N - 1, where every padding slot points
     L.hcol[0] = (int32_t)(N - 1);
-    L.stuck = 0;
+    L.stuck = L.done = 0;
     L.norm0 = a.ks->norm0;
     L.tol = a.ks->tol;
     L.restart_tol = a.ks->restart_tol;
@@ -374,16 +379,20 @@ __global__ void __launch_bounds__(RES_THREADS) bicg_resident_kernel(ResArgs a) {
   };
   publish_p(1);
 #pragma unroll 1
-  for (int it = 0; it < a.chunk && !done; ++it) {
+  for (int it = 0; it < a.chunk; ++it) {
     const unsigned epoch = (unsigned)it + 1u;  // of the sums; the halos of p and s are numbered 2 it + 1 and 2 it + 2
     // ap = A p, ap . r0
     double r0[RES_ROWS];
 #pragma unroll
     for (int m = 0; m < RES_ROWS; ++m) r0[m] = own(m) ? *at32(a.r0, v + m * S) : 0.0;
     __syncthreads();  // every wave has issued its words (RES_SPIN)
-    resident_halo(L, a, 2 * epoch - 1);
+    resident_halo<SET>(L, a, 2 * epoch - 1);
     __syncthreads();
-    if (L.stuck) break;  // a wait reached its bound (uniform: set before this barrier or after the next)
+    // Every wave leaves here or none: both flags are set before this barrier or
+    // after the next, and waves whose waits failed have totals of their own, so
+    // a wave's own `done` must not end its loop.  (The halo just fetched is of
+    // the p that is published before the stop test.)
+    if (L.stuck | L.done) break;
     resident_rows(L, val, pos, ap);
     double acc1[RES_ROWS], acc2[RES_ROWS];
 #pragma unroll
@@ -391,9 +400,9 @@ __global__ void __launch_bounds__(RES_THREADS) bicg_resident_kernel(ResArgs a) {
     const double w1 = wave_sum4(acc1[0], acc1[1], acc1[2], acc1[3]);
     if (lane >= 60) L.wsum[0][lane - 60][wid] = w1;
     __syncthreads();
-    resident_put_rows<1>(a, L, a.red[0], epoch);
+    resident_put_rows<1, SET>(a, L, a.red[0], epoch);
     double ta[1];
-    resident_total<1>(a, L, a.red[0], nslot, epoch, ta);
+    resident_total<1, SET>(a, L, a.red[0], nslot, epoch, ta);
     alpha = rho / ta[0];
     // s = r - alpha ap; as = A s, as . s, as . as
 #pragma unroll
@@ -403,7 +412,7 @@ __global__ void __launch_bounds__(RES_THREADS) bicg_resident_kernel(ResArgs a) {
       if (own(m) && a.nblk > 1) ll_store(at32(a.ll0, v + m * S), at32(a.ll1, v + m * S), s[m], 2 * epoch);
     }
     __syncthreads();
-    resident_halo(L, a, 2 * epoch);
+    resident_halo<SET>(L, a, 2 * epoch);
     __syncthreads();
     resident_rows(L, val, pos, as);
 #pragma unroll
@@ -418,14 +427,14 @@ __global__ void __launch_bounds__(RES_THREADS) bicg_resident_kernel(ResArgs a) {
       L.wsum[1][lane - 60][wid] = w3;
     }
     __syncthreads();
-    resident_put_rows<2>(a, L, a.red[1], epoch);
+    resident_put_rows<2, SET>(a, L, a.red[1], epoch);
     double to[2], xo[RES_ROWS];
 #pragma unroll
     for (int m = 0; m < RES_ROWS; ++m) {
       xo[m] = own(m) ? *at32(a.x, v + m * S) : 0.0;
       r0[m] = own(m) ? *at32(a.r0, v + m * S) : 0.0;
     }
-    resident_total<2>(a, L, a.red[1], nslot, epoch, to);
+    resident_total<2, SET>(a, L, a.red[1], nslot, epoch, to);
     omega = to[0] / to[1];
     // x += alpha p + omega s; r = s - omega as; r . r, r . r0
     double acc[2] = {0.0, 0.0};
@@ -445,7 +454,7 @@ __global__ void __launch_bounds__(RES_THREADS) bicg_resident_kernel(ResArgs a) {
     resident_put_xr(a, L, a.red[2], epoch);
     const double ao = alpha / omega;
     double tc[2];
-    resident_total<2>(a, L, a.red[2], a.nbx, epoch, tc);
+    resident_total<2, SET>(a, L, a.red[2], a.nbx, epoch, tc);
     // beta, the restart rule and the next p (conv_finalize, p_update_kernel),
     // on its way before the stop test: nothing reads it after the last iteration
     const double next_beta = ao * (tc[1] / rho);
@@ -473,6 +482,7 @@ __global__ void __launch_bounds__(RES_THREADS) bicg_resident_kernel(ResArgs a) {
           if (own(m)) *at32(a.r0, v + m * S) = r[m];
       }
     }
+    if (t == 0) L.done = done;
   }
   __syncthreads();
   if (L.stuck) {
@@ -503,12 +513,21 @@ __global__ void __launch_bounds__(RES_THREADS) bicg_resident_kernel(ResArgs a) {
   }
 }
 
-// no exchange has taken place: every word's number is 0 before a launch
-__global__ void __launch_bounds__(256) resident_clear_kernel(ResArgs a) {
+// no exchange has taken place: every word's number is 0 before a launch; the
+// first one of a solve keeps what the solve changes and init_kernel does not set
+__global__ void __launch_bounds__(256) resident_clear_kernel(ResArgs a, bool first) {
   const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (first && q < a.N) a.keep[q] = a.x[q];
+  if (first && q == 0) a.ks[1].restarts = a.ks->restarts;
   if (q < a.N) a.ll0[q] = a.ll1[q] = 0;
   if (q < 2 * RES_RED_WORDS) a.red[0][q] = a.red[1][q] = a.red[2][q] = 0;
   if (q == 0) a.ks->pad0 = a.ks->pad1 = 0;
+}
+
+__global__ void __launch_bounds__(256) resident_restore_kernel(ResArgs a) {
+  const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (q < a.N) a.x[q] = a.keep[q];
+  if (q == 0) a.ks->restarts = a.ks[1].restarts;
 }
 
 }  // namespace cfd

@@ -763,12 +763,14 @@ hipError_t launch_iters(Ctx &c, const OpArgs &a, const Vecs<T> &v, KrylovScalars
 // (dev_resident.h) where its rows fit the chip's registers; the state after
 // init_kernel is the launch path's and so is every result, bit for bit.
 // *solved is false when the launch path has to go on from where the state is:
-// the system is too large, its matrix is no stencil, or the CUs are taken.
+// the system is too large, a workgroup's halo does not fit, or the CUs are
+// taken; *lost, when it has to start again, from the x that is back in place: a
+// wait reached its bound.
 // The limit is what the registers of 256 one-workgroup CUs hold (RES_MAX_N,
 // 524288 rows); it is the faster path over that whole range (at the limit
 // 19.7 us an iteration against 28.5, at one workgroup 4.6 against 15.4).
-int solve_resident(Ctx &c, const OpArgs &a, const Vecs<double> &v, KrylovScalars *ks, bool *solved) {
-  *solved = false;
+int solve_resident(Ctx &c, const OpArgs &a, const Vecs<double> &v, KrylovScalars *ks, bool *solved, bool *lost) {
+  *solved = *lost = false;
   if ((a.op != CFD_OP_ELL && a.op != OP_ELL_GRID) || a.N > RES_MAX_N) return CFD_OK;
   ResArgs r;
   r.N = a.N;
@@ -782,9 +784,10 @@ int solve_resident(Ctx &c, const OpArgs &a, const Vecs<double> &v, KrylovScalars
   r.r0 = v.r0;
   r.r1 = v.r1;
   r.p1 = v.p1;
-  // the launch path's s and A p are its only users of these two vectors
+  // the launch path's s, A p and A s are its only users of these vectors
   r.ll0 = reinterpret_cast<uint64_t *>(v.s1);
   r.ll1 = reinterpret_cast<uint64_t *>(v.ap);
+  r.keep = v.as;
   static_assert(2 * RES_RED_WORDS <= 3 * RED_MAX_BLOCKS, "an exchanged sum fits its site's partials");
   const int sites[3] = {RS_SPMV_DOT, RS_SPMV_DOT2, RS_XR};
   for (int q = 0; q < 3; ++q) r.red[q] = reinterpret_cast<uint64_t *>(red_part_host(c, sites[q]));
@@ -797,14 +800,21 @@ int solve_resident(Ctx &c, const OpArgs &a, const Vecs<double> &v, KrylovScalars
     return CFD_OK;
   }
   const int nbc = blocks_for(std::max<int64_t>(a.N, 2 * RES_RED_WORDS), 256, 1 << 30);
-  for (;;) {
-    resident_clear_kernel<<<nbc, 256, 0, c.stream>>>(r);
-    bicg_resident_kernel<<<r.nblk, RES_THREADS, 0, c.stream>>>(r);
+  for (bool first = true;; first = false) {
+    resident_clear_kernel<<<nbc, 256, 0, c.stream>>>(r, first);
+    if (r.bounds.set)
+      bicg_resident_kernel<true><<<r.nblk, RES_THREADS, 0, c.stream>>>(r);
+    else
+      bicg_resident_kernel<false><<<r.nblk, RES_THREADS, 0, c.stream>>>(r);
     CFD_HIP(hipGetLastError());
     CFD_HIP(hipMemcpyAsync(c.hks, ks, sizeof(KrylovScalars), hipMemcpyDeviceToHost, c.stream));
     CFD_HIP(hipStreamSynchronize(c.stream));
-    if (c.hks->pad1 == RES_STUCK) return fail(CFD_ERR_RUNTIME, "resident BiCGSTAB: a workgroup stopped answering");
     if (c.hks->pad1 != RES_GO) {
+      if (c.hks->pad1 == RES_STUCK) {
+        resident_restore_kernel<<<nbc, 256, 0, c.stream>>>(r);
+        CFD_HIP(hipGetLastError());
+        *lost = true;
+      }
       c.one.handed_back++;
       return CFD_OK;
     }
@@ -824,14 +834,19 @@ int solve_bicg(Ctx &c, const OpArgs &a, const Vecs<T> &v, KrylovScalars *ks, int
                int *iters, double *relres) {
   const int64_t N = c.g.N;
   const int nb = blocks_for(N, 256, RED_MAX_BLOCKS);
-  ks_setup_kernel<<<1, 1, 0, c.stream>>>(ks, tol, 1e-7 * tol, maxit, timestep);
-  init_kernel<T><<<nb, 256, op_lds_bytes(a), c.stream>>>(a, v.b, v.x, v.r0, v.r1, v.p1, v.px1, v.px2,
-                                                      red_part_host(c, RS_INIT));
-  init_finalize<<<1, FIN_THREADS, 0, c.stream>>>(red_part_host(c, RS_INIT), nb, ks);
-  CFD_HIP(hipGetLastError());
+  auto init = [&](double *px1, double *px2) {
+    ks_setup_kernel<<<1, 1, 0, c.stream>>>(ks, tol, 1e-7 * tol, maxit, timestep);
+    init_kernel<T><<<nb, 256, op_lds_bytes(a), c.stream>>>(a, v.b, v.x, v.r0, v.r1, v.p1, px1, px2,
+                                                        red_part_host(c, RS_INIT));
+    init_finalize<<<1, FIN_THREADS, 0, c.stream>>>(red_part_host(c, RS_INIT), nb, ks);
+    return hipGetLastError();
+  };
+  CFD_HIP(init(v.px1, v.px2));
   bool solved = false;
   if constexpr (std::is_same<T, double>::value) {
-    if (int rc = solve_resident(c, a, v, ks, &solved)) return rc;
+    bool lost = false;
+    if (int rc = solve_resident(c, a, v, ks, &solved, &lost)) return rc;
+    if (lost) CFD_HIP(init(nullptr, nullptr));  // the history has its entry
   }
   int batch = 2;
   double prev_rel = -1.0;

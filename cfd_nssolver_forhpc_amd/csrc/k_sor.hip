@@ -336,6 +336,7 @@ struct SorLds {
 struct SorArgs {
   uint64_t *ll0, *ll1;  // the two words of each cell
   uint64_t *mx;         // maxima: [sweep parity][word][workgroup]
+  double *keep;         // the cells' pressure before the solve
   KrylovScalars *ks;    // pad0: arrivals, pad1: RES_* state
   int nblk, chunk;      // chunk: sweeps this launch runs at most
   ResBounds bounds;
@@ -452,7 +453,7 @@ __global__ void __launch_bounds__(SORR_THREADS) sorp_resident_kernel(DevGrid g, 
     if (tid < busy) return;
     for (int e0 = tid - busy; e0 < nh; e0 += 4 * step) {
       const bool ok = ll_fetch<4>(
-          a.ll0, a.ll1, epoch, res_spin(a.bounds), [&](int u) { return e0 + u * step < nh ? (unsigned)L.hrow[c][e0 + u * step] : RES_NONE; },
+          a.ll0, a.ll1, epoch, res_spin<true>(a.bounds), [&](int u) { return e0 + u * step < nh ? (unsigned)L.hrow[c][e0 + u * step] : RES_NONE; },
           [&](int u, bool have, double v) {
             if (have) L.p[2 * OWN + c * HALO + e0 + u * step] = v;
           });
@@ -473,7 +474,7 @@ __global__ void __launch_bounds__(SORR_THREADS) sorp_resident_kernel(DevGrid g, 
         double v = 0.0;
         const uint64_t *w = a.mx + ((s - 1) & 1) * 2 * SORR_BLOCKS;
         const bool ok = ll_fetch<1>(
-            w, w + SORR_BLOCKS, (unsigned)s, res_spin(a.bounds), [&](int) { return tid < a.nblk ? (unsigned)tid : RES_NONE; },
+            w, w + SORR_BLOCKS, (unsigned)s, res_spin<true>(a.bounds), [&](int) { return tid < a.nblk ? (unsigned)tid : RES_NONE; },
             [&](int, bool have, double x) { v = have ? x : 0.0; });
         if (!ok) L.stuck = 1;
         v = wave_max(v);
@@ -526,18 +527,32 @@ __global__ void __launch_bounds__(SORR_THREADS) sorp_resident_kernel(DevGrid g, 
   }
 }
 
-__global__ void __launch_bounds__(256) sorp_clear_kernel(int64_t n, SorArgs a) {
-  const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+// the ghosted position of cell q
+__device__ inline int64_t sorp_cell(const DevGrid &g, int64_t q) {
+  const int r = (int)q, kc = r % g.nzc, rest = r / g.nzc;
+  return icel(g, rest / g.nyc + GC, rest % g.nyc + GC, kc + GC);
+}
+
+__global__ void __launch_bounds__(256) sorp_clear_kernel(DevGrid g, const double *__restrict__ p, SorArgs a,
+                                                         bool first) {
+  const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x, n = g.N;
+  if (first && q < n) a.keep[q] = p[sorp_cell(g, q)];
   if (q < n) a.ll0[q] = a.ll1[q] = 0;
   if (q < 4 * SORR_BLOCKS) a.mx[q] = 0;
   if (q == 0) a.ks->pad0 = a.ks->pad1 = 0;
 }
 
+__global__ void __launch_bounds__(256) sorp_restore_kernel(DevGrid g, double *__restrict__ p, SorArgs a) {
+  const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (q < g.N) p[sorp_cell(g, q)] = a.keep[q];
+}
+
 // *solved is false when the launches have to do it: more cells than the
 // workgroups hold (262144 at an even nz), a halo or ghosts that LDS does not
-// hold, or CUs that are taken.
-int sorp_resident(Ctx &c, double omega, const double *cf6, bool *solved) {
-  *solved = false;
+// hold, or CUs that are taken.  *lost: they start again, from the pressure that
+// is back in place (a wait reached its bound).
+int sorp_resident(Ctx &c, double omega, const double *cf6, bool *solved, bool *lost) {
+  *solved = *lost = false;
   const DevGrid &g = c.g;
   const int64_t npair = (int64_t)g.nxc * g.nyc * ((g.nzc + 1) / 2);
   if (npair > SORR_THREADS * SORR_BLOCKS) return CFD_OK;
@@ -545,6 +560,7 @@ int sorp_resident(Ctx &c, double omega, const double *cf6, bool *solved) {
   a.ll0 = reinterpret_cast<uint64_t *>(c.s1);  // the Krylov solver's vectors
   a.ll1 = reinterpret_cast<uint64_t *>(c.ap);
   a.mx = reinterpret_cast<uint64_t *>(red_part_host(c, RS_SPMV_DOT));
+  a.keep = c.as;
   a.ks = c.ks;
   a.nblk = (int)((npair + SORR_THREADS - 1) / SORR_THREADS);
   a.chunk = 4096;  // bounds one launch to some tens of milliseconds
@@ -554,14 +570,19 @@ int sorp_resident(Ctx &c, double omega, const double *cf6, bool *solved) {
     c.one.handed_back++;
     return CFD_OK;
   }
-  for (;;) {
-    sorp_clear_kernel<<<blocks_for(std::max<int64_t>(g.N, 4 * SORR_BLOCKS), 256, 1 << 30), 256, 0, c.stream>>>(g.N, a);
+  const int nbc = blocks_for(std::max<int64_t>(g.N, 4 * SORR_BLOCKS), 256, 1 << 30);
+  for (bool first = true;; first = false) {
+    sorp_clear_kernel<<<nbc, 256, 0, c.stream>>>(g, c.f[CFD_P], a, first);
     sorp_resident_kernel<<<a.nblk, SORR_THREADS, 0, c.stream>>>(g, omega, c.prm.periodic_z, cf6, c.f[CFD_P], a);
     CFD_HIP(hipGetLastError());
     CFD_HIP(hipMemcpyAsync(c.hks, c.ks, sizeof(KrylovScalars), hipMemcpyDeviceToHost, c.stream));
     CFD_HIP(hipStreamSynchronize(c.stream));
-    if (c.hks->pad1 == RES_STUCK) return fail(CFD_ERR_RUNTIME, "resident SorPipeLine: a workgroup stopped answering");
     if (c.hks->pad1 != RES_GO) {
+      if (c.hks->pad1 == RES_STUCK) {
+        sorp_restore_kernel<<<nbc, 256, 0, c.stream>>>(g, c.f[CFD_P], a);
+        CFD_HIP(hipGetLastError());
+        *lost = true;
+      }
       c.one.handed_back++;
       return CFD_OK;
     }
@@ -582,8 +603,9 @@ int sor_pipeline_solve(Ctx &c, double omega, double crit, int itmax, int *iters,
                                                                       c.f[CFD_T1_V], c.f[CFD_T1_W], cf6);
   sorp_setup_kernel<<<1, 1, 0, c.stream>>>(c.ks, crit, itmax);
   CFD_HIP(hipGetLastError());
-  bool solved = false;
-  if (int rc = sorp_resident(c, omega, cf6, &solved)) return rc;
+  bool solved = false, lost = false;
+  if (int rc = sorp_resident(c, omega, cf6, &solved, &lost)) return rc;
+  if (lost) sorp_setup_kernel<<<1, 1, 0, c.stream>>>(c.ks, crit, itmax);
   if (solved) {
     *iters = c.hks->iters - 1;
     *error = c.hks->relres;

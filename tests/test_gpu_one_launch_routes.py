@@ -106,3 +106,49 @@ def test_sor_pipeline(require_gpu, ncal, route):
         assert way == route
     assert (it1, err1) == (it0, err0)
     assert np.array_equal(got, want)
+
+
+# a wait that runs out at once: every workgroup's, the first one's only (the
+# others wait for a workgroup that has left)
+@pytest.mark.parametrize("bounds", [dict(wait=1), dict(wait=512, wait_first=1)])
+@pytest.mark.parametrize("ncal", [(17, 11, 11), (37, 25, 11), (64, 64, 16), (64, 64, 128)])
+def test_bicgstab_whose_waits_run_out(require_gpu, ncal, bounds):
+    print(f"one-launch waits ncal={ncal} {bounds}", flush=True)
+    b = np.random.default_rng(3).standard_normal(int(np.prod(ncal)))
+    b -= b.mean()
+    got = []
+    for lim in (dict(arrive=-1), bounds):
+        with make_sim(ncal) as sim:
+            sim.init_state()
+            sim.createPressureMatrix()
+            sim.upload(capi.X, np.zeros(sim.N))
+            sim.one_launch_bounds(**lim)
+            for k in range(12):  # from the last x; the restart rule starts at the tenth solve
+                sim.upload(capi.RHS, (1.0 + 0.1 * k) * b)
+                it, rel = sim.bicgstab(tol=1e-6, maxit=40)
+            fin, back = sim.one_launch_counters()
+            assert fin + back == 12 and back > 0  # a first workgroup may find every value at its first look
+            assert lim == bounds or fin == 0
+            got.append((sim.download(capi.X), it, rel, sim.solver_counters()))
+    assert np.isfinite(got[0][0]).all()
+    assert got[1][1:] == got[0][1:]
+    assert np.array_equal(got[1][0], got[0][0])
+
+
+@pytest.mark.parametrize("bounds", [dict(wait=1), dict(wait=512, wait_first=1)])
+def test_timesteps_whose_sweeps_run_out(require_gpu, bounds):
+    grid = uniform_grid((33, 18, 12), (8.0, 6.0, 4.0))
+    prm = configs.cylinder_params(100.0, 0.002, 2.0, 1.0, 0.5, 1e-3)
+    prm.solver, prm.maxit = capi.CFD_SOLVER_SOR_PIPELINE, 60
+    got = []
+    for lim in (dict(arrive=-1), bounds):
+        with Simulation(grid, prm) as sim:
+            sim.setup(noise=1e-3, seed=1)
+            sim.one_launch_bounds(**lim)
+            steps = [sim.step().as_dict() for _ in range(3)]
+            fin, back = sim.one_launch_counters()
+            assert fin + back == 8 and back > 0  # none in the first step, four in each that follows
+            got.append((steps, sim.download(capi.P), sim.download(capi.T0_U)))
+    assert got[0][0] == got[1][0]
+    assert np.isfinite(got[0][1]).all()
+    assert np.array_equal(got[0][1], got[1][1]) and np.array_equal(got[0][2], got[1][2])
