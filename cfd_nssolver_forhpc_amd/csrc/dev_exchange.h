@@ -49,12 +49,14 @@ __device__ inline double ll_value(uint64_t w0, uint64_t w1) {
 // every wave of its workgroup has issued the words others wait for (a barrier
 // stands between): the memory pipeline takes older waves first, and waves
 // that poll scattered words keep it full, so a younger wave's stores could
-// wait for ever behind polls that wait for them.  The bound (some seconds of
+// wait for ever behind polls that wait for them.  The bound (a second of
 // polling, counted in polls so that a preempted kernel does not run into it)
-// is there so that the kernel ends whatever happens, with RES_STUCK: the host
-// then takes the solve back to its start (every such solve keeps a copy of what
-// it writes to) and runs it by launches.
-constexpr unsigned RES_SPIN = 1u << 22;
+// holds for a workgroup, not for each of its waits: once one has run out, the
+// others end RES_LOOK polls later (the resident BiCGSTAB's halos: a small part of
+// the bound).  It is there so that the kernel ends whatever
+// happens, with RES_STUCK: the host then takes the solve back to its start
+// (every such solve keeps a copy of what it writes to) and runs it by launches.
+constexpr unsigned RES_SPIN = 1u << 22, RES_LOOK = 1u << 10;
 // polls of the arrival handshake before a workgroup gives the launch up
 // (tens of milliseconds: the CUs are held by other kernels)
 constexpr unsigned RES_ARRIVE_SPIN = 1u << 15;
@@ -81,10 +83,12 @@ __device__ inline unsigned res_spin(const ResBounds &b) {
 
 // Loads U pairs of words at a time until each carries the epoch: get(u) is
 // the position of the u-th pair in w0 / w1 (RES_NONE: none), put(u, v) takes
-// its value.  False when the bound was reached.
+// its value.  False when the bound was reached, here or (LOOK; stuck, in LDS, set
+// by the callers) in another of the workgroup's waits.
 constexpr unsigned RES_NONE = ~0u;
-template <int U, typename G, typename P>
-__device__ inline bool ll_fetch(const uint64_t *p0, const uint64_t *p1, unsigned epoch, unsigned bound, G get, P put) {
+template <int U, bool LOOK = true, typename G, typename P>
+__device__ inline bool ll_fetch(const uint64_t *p0, const uint64_t *p1, unsigned epoch, unsigned bound,
+                                const int &stuck, G get, P put) {
   unsigned at[U];
 #pragma unroll
   for (int u = 0; u < U; ++u) at[u] = get(u);
@@ -108,6 +112,9 @@ __device__ inline bool ll_fetch(const uint64_t *p0, const uint64_t *p1, unsigned
       for (int u = 0; u < U; ++u) put(u, at[u] != RES_NONE, ll_value(w0[u], w1[u]));
       return true;
     }
+    if (LOOK && spin % RES_LOOK == RES_LOOK - 1 &&
+        __hip_atomic_load(&stuck, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP))
+      break;
   }
   return false;
 }

@@ -453,7 +453,8 @@ __global__ void __launch_bounds__(SORR_THREADS) sorp_resident_kernel(DevGrid g, 
     if (tid < busy) return;
     for (int e0 = tid - busy; e0 < nh; e0 += 4 * step) {
       const bool ok = ll_fetch<4>(
-          a.ll0, a.ll1, epoch, res_spin<true>(a.bounds), [&](int u) { return e0 + u * step < nh ? (unsigned)L.hrow[c][e0 + u * step] : RES_NONE; },
+          a.ll0, a.ll1, epoch, res_spin<true>(a.bounds), L.stuck,
+          [&](int u) { return e0 + u * step < nh ? (unsigned)L.hrow[c][e0 + u * step] : RES_NONE; },
           [&](int u, bool have, double v) {
             if (have) L.p[2 * OWN + c * HALO + e0 + u * step] = v;
           });
@@ -474,7 +475,8 @@ __global__ void __launch_bounds__(SORR_THREADS) sorp_resident_kernel(DevGrid g, 
         double v = 0.0;
         const uint64_t *w = a.mx + ((s - 1) & 1) * 2 * SORR_BLOCKS;
         const bool ok = ll_fetch<1>(
-            w, w + SORR_BLOCKS, (unsigned)s, res_spin<true>(a.bounds), [&](int) { return tid < a.nblk ? (unsigned)tid : RES_NONE; },
+            w, w + SORR_BLOCKS, (unsigned)s, res_spin<true>(a.bounds), L.stuck,
+            [&](int) { return tid < a.nblk ? (unsigned)tid : RES_NONE; },
             [&](int, bool have, double x) { v = have ? x : 0.0; });
         if (!ok) L.stuck = 1;
         v = wave_max(v);
