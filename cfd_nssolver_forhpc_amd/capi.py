@@ -130,7 +130,7 @@ class CfdSolverCounters(C.Structure):
 
 
 class CfdOneLaunchCounters(C.Structure):
-    _fields_ = [("finished", C.c_longlong), ("handed_back", C.c_longlong)]
+    _fields_ = [("finished", C.c_longlong), ("handed_back", C.c_longlong), ("waited", C.c_longlong)]
 
 
 class CfdAdjointStats(C.Structure):

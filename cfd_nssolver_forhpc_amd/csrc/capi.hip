@@ -770,6 +770,7 @@ int cfd_ell_upload(cfd_ctx *ctx, const int32_t *col, const double *val, size_t n
     }
   }
   c.ell_grid = false;  // from here on the stored entries are the operator
+  c.one.forget();
   CFD_HIP(hipMemcpyAsync(c.col, hc.data(), sizeof(int32_t) * hc.size(), hipMemcpyHostToDevice, c.stream));
   CFD_HIP(hipMemcpyAsync(c.val, hv.data(), sizeof(double) * hv.size(), hipMemcpyHostToDevice, c.stream));
   CFD_HIP(hipStreamSynchronize(c.stream));  // the staging vectors go out of scope
@@ -1191,6 +1192,7 @@ int cfd_get_one_launch_counters(cfd_ctx *ctx, cfd_one_launch_counters *out) {
   const OneLaunch &o = reinterpret_cast<Ctx *>(ctx)->one;
   out->finished = o.finished;
   out->handed_back = o.handed_back;
+  out->waited = o.waited;
   return CFD_OK;
 }
 
@@ -1201,6 +1203,7 @@ int cfd_set_one_launch_bounds(cfd_ctx *ctx, int arrive, int wait, int wait_first
   o.arrive = arrive;
   o.wait = wait;
   o.wait_first = wait_first;
+  o.forget();
   return CFD_OK;
 }
 

@@ -80,10 +80,32 @@ enum RedSite { RS_SPMV_DOT = 0, RS_SPMV_DOT2, RS_XR, RS_INIT, RS_NORM, RS_DRAG, 
 
 // The pressure solves that run as one kernel (dev_exchange.h): the bounds of
 // their waits in polls (0: the default, arrive < 0: no such solve) and how many
-// solves they finished or handed back to the launches.
+// solves they finished or handed back to the launches (waited: of these, after a
+// launch).  A launch that did not get its CUs will hardly get them in the next
+// solve, microseconds later, and a halo that does not fit never will, so 1, 2,
+// 4 .. 64 solves go straight to the launches before the next try.
 struct OneLaunch {
   int arrive = 0, wait = 0, wait_first = 0;
-  long long finished = 0, handed_back = 0;
+  long long finished = 0, handed_back = 0, waited = 0;
+  int skip = 0, backoff = 0;
+
+  bool due() {
+    if (arrive >= 0 && skip == 0) return true;
+    if (skip > 0) skip--;
+    handed_back++;
+    return false;
+  }
+  void gave_up() {
+    handed_back++;
+    waited++;
+    backoff = backoff == 0 ? 1 : backoff < 64 ? 2 * backoff : 64;
+    skip = backoff;
+  }
+  void finish() {
+    finished++;
+    backoff = 0;
+  }
+  void forget() { skip = backoff = 0; }  // another operator, other bounds
 };
 
 struct Ctx {

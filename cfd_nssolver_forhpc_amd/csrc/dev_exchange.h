@@ -57,9 +57,10 @@ __device__ inline double ll_value(uint64_t w0, uint64_t w1) {
 // happens, with RES_STUCK: the host then takes the solve back to its start
 // (every such solve keeps a copy of what it writes to) and runs it by launches.
 constexpr unsigned RES_SPIN = 1u << 22, RES_LOOK = 1u << 10;
-// polls of the arrival handshake before a workgroup gives the launch up
-// (tens of milliseconds: the CUs are held by other kernels)
-constexpr unsigned RES_ARRIVE_SPIN = 1u << 15;
+// polls of the arrival handshake before a workgroup gives the launch up (the CUs
+// are held by other kernels): a millisecond, which is what the launches take for
+// such a solve; workgroups that find their CUs arrive within some 20 us
+constexpr unsigned RES_ARRIVE_SPIN = 1u << 12;
 
 // the bounds of a launch: the arrival's, the first workgroup's and the others'
 struct ResBounds {

@@ -243,6 +243,7 @@ hipError_t launch_ell_assemble(Ctx &c) {
   for (int f = 0; f < 6; ++f) c.ell_pd[f] = c.prm.p_dirichlet[f];
   c.ell_wrapz = c.prm.periodic_z;
   c.ell_grid = true;
+  c.one.forget();
   ell_assemble_kernel<<<blocks_for(c.g.N, 256, 1 << 30), 256, 0, c.stream>>>(c.g, pbc_of(c), c.ell_sliced, c.col,
                                                                              c.val, c.val32, c.f[CFD_JP]);
   return hipGetLastError();

@@ -795,7 +795,8 @@ int solve_resident(Ctx &c, const OpArgs &a, const Vecs<double> &v, KrylovScalars
   r.chunk = 4096;  // bounds one launch to some tens of milliseconds
   r.bounds = res_bounds(c.one);
   ResidentSlots slots;
-  if (c.one.arrive < 0 || !slots.take(c.device, r.nblk)) {
+  if (!c.one.due()) return CFD_OK;
+  if (!slots.take(c.device, r.nblk)) {
     c.one.handed_back++;
     return CFD_OK;
   }
@@ -815,12 +816,12 @@ int solve_resident(Ctx &c, const OpArgs &a, const Vecs<double> &v, KrylovScalars
         CFD_HIP(hipGetLastError());
         *lost = true;
       }
-      c.one.handed_back++;
+      c.one.gave_up();
       return CFD_OK;
     }
     if (c.hks->done) break;
   }
-  c.one.finished++;
+  c.one.finish();
   *solved = true;
   return CFD_OK;
 }

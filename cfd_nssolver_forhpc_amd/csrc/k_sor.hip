@@ -568,7 +568,8 @@ int sorp_resident(Ctx &c, double omega, const double *cf6, bool *solved, bool *l
   a.chunk = 4096;  // bounds one launch to some tens of milliseconds
   a.bounds = res_bounds(c.one);
   ResidentSlots slots;
-  if (c.one.arrive < 0 || !slots.take(c.device, a.nblk)) {
+  if (!c.one.due()) return CFD_OK;
+  if (!slots.take(c.device, a.nblk)) {
     c.one.handed_back++;
     return CFD_OK;
   }
@@ -585,12 +586,12 @@ int sorp_resident(Ctx &c, double omega, const double *cf6, bool *solved, bool *l
         CFD_HIP(hipGetLastError());
         *lost = true;
       }
-      c.one.handed_back++;
+      c.one.gave_up();
       return CFD_OK;
     }
     if (c.hks->done) break;
   }
-  c.one.finished++;
+  c.one.finish();
   *solved = true;
   return CFD_OK;
 }

@@ -300,10 +300,10 @@ class Simulation:
 
     def one_launch_counters(self) -> tuple:
         """Pressure solves that ran as one kernel, and those that could have by
-        their size and were handed back to the launches."""
+        their size and were handed back to the launches; of these, after a try."""
         out = capi.CfdOneLaunchCounters()
         check(self.lib.cfd_get_one_launch_counters(self.h, C.byref(out)), "cfd_get_one_launch_counters")
-        return out.finished, out.handed_back
+        return out.finished, out.handed_back, out.waited
 
     def one_launch_bounds(self, arrive: int = 0, wait: int = 0, wait_first: int = 0):
         """Bounds of the one-kernel solves' waits in polls; 0: the default,

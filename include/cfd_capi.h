@@ -352,10 +352,11 @@ int cfd_get_solver_counters(cfd_ctx *ctx, cfd_solver_counters *out);
    workgroups hold a CU each and wait for each other's values; where that
    cannot be done -- the CUs are taken, a workgroup's halo does not fit -- the
    solve is handed back to launches of one kernel an operation, with the same
-   result bit for bit.  This context's tallies (a system too large for it is in
-   neither): */
+   result bit for bit.  After a try that was in vain the next 1, 2, 4 .. 64 solves
+   are handed back at once.  This context's tallies (waited: those handed back
+   after a try; a system too large for it is in none): */
 typedef struct cfd_one_launch_counters {
-  long long finished, handed_back;
+  long long finished, handed_back, waited;
 } cfd_one_launch_counters;
 int cfd_get_one_launch_counters(cfd_ctx *ctx, cfd_one_launch_counters *out);
 /* Bounds of the waits, in polls of the awaited memory, 0 for the default:

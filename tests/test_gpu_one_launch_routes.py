@@ -8,6 +8,7 @@ too large to be tried (neither); a halo that no workgroup holds (handed back).
 """
 from __future__ import annotations
 
+import threading
 import time
 
 import numpy as np
@@ -27,7 +28,7 @@ def make_sim(ncal):
 
 
 def delta(sim, before):
-    return tuple(a - b for a, b in zip(sim.one_launch_counters(), before))
+    return tuple(a - b for a, b in zip(sim.one_launch_counters(), before))[:2]
 
 
 def bicg(sim, K):
@@ -128,7 +129,7 @@ def test_bicgstab_whose_waits_run_out(require_gpu, ncal, bounds):
             for k in range(12):  # from the last x; the restart rule starts at the tenth solve
                 sim.upload(capi.RHS, (1.0 + 0.1 * k) * b)
                 it, rel = sim.bicgstab(tol=1e-6, maxit=40)
-            fin, back = sim.one_launch_counters()
+            fin, back, _ = sim.one_launch_counters()
             assert fin + back == 12
             assert "wait_first" in lim or fin == 0  # a first workgroup may find every value at its first look
             got.append((sim.download(capi.X), it, rel, sim.solver_counters()))
@@ -150,7 +151,7 @@ def test_one_bound_for_a_workgroup(require_gpu):
         t = time.perf_counter()
         sim.bicgstab(tol=0.0, maxit=10)
         t = time.perf_counter() - t
-        assert sim.one_launch_counters() == BACK
+        assert sim.one_launch_counters() == (0, 1, 1)
     assert t < 0.11
 
 
@@ -165,10 +166,71 @@ def test_timesteps_whose_sweeps_run_out(require_gpu, bounds):
             sim.setup(noise=1e-3, seed=1)
             sim.one_launch_bounds(**lim)
             steps = [sim.step().as_dict() for _ in range(3)]
-            fin, back = sim.one_launch_counters()
+            fin, back, _ = sim.one_launch_counters()
             assert fin + back == 8  # none in the first step, four in each that follows
             assert "wait_first" in lim or fin == 0
             got.append((steps, sim.download(capi.P), sim.download(capi.T0_U)))
     assert got[0][0] == got[1][0]
     assert np.isfinite(got[0][1]).all()
     assert np.array_equal(got[0][1], got[1][1]) and np.array_equal(got[0][2], got[1][2])
+
+
+def test_launches_that_are_given_up(require_gpu):
+    """An arrival bound of one poll: every try is given up, and tries get rarer."""
+    with make_sim((37, 25, 11)) as sim:
+        sim.init_state()
+        sim.createPressureMatrix()
+        b = np.random.default_rng(3).standard_normal(sim.N)
+        sim.upload(capi.RHS, b - b.mean())
+        sim.one_launch_bounds(arrive=-1)
+        want, way = bicg(sim, 8)
+        assert way == BACK
+        sim.one_launch_bounds(arrive=1)
+        before = sim.one_launch_counters()
+        for _ in range(64):
+            got, way = bicg(sim, 8)
+            assert way == BACK
+            assert np.array_equal(got, want)
+        # the 1st, 3rd, 6th, 11th, 20th and 37th
+        assert sim.one_launch_counters()[2] - before[2] == 6
+        sim.one_launch_bounds()
+        got, way = bicg(sim, 8)
+        assert way == RUNS
+        assert np.array_equal(got, want)
+
+
+def test_contexts_on_two_threads(require_gpu):
+    """Two systems of 256 workgroups each: one context's solves find the CUs
+    taken while the other's hold them."""
+    sims = [make_sim((64, 64, 128)) for _ in range(2)]
+    try:
+        want = []
+        for k, sim in enumerate(sims):
+            sim.init_state()
+            sim.createPressureMatrix()
+            b = np.random.default_rng(k).standard_normal(sim.N)
+            sim.upload(capi.RHS, b - b.mean())
+            sim.one_launch_bounds(arrive=-1)
+            want.append(bicg(sim, 60)[0])
+            sim.one_launch_bounds()
+        before = [sim.one_launch_counters() for sim in sims]
+        bad = []
+
+        def work(k):
+            for _ in range(20):
+                if not np.array_equal(bicg(sims[k], 60)[0], want[k]):
+                    bad.append(k)
+
+        threads = [threading.Thread(target=work, args=(k,)) for k in range(2)]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        assert not bad
+        for sim, b in zip(sims, before):
+            fin, back = delta(sim, b)
+            assert fin + back == 20
+        print("finished, handed back, waited:", [sim.one_launch_counters() for sim in sims], flush=True)
+    finally:
+        for sim in sims:
+            sim.close()
