@@ -47,8 +47,9 @@ constexpr int RES_FETCH = 6;            // halo entries a thread has in flight
 constexpr int RES_SLOTS = 1024;         // partial sums of the launch path at most (one per finalize thread)
 static_assert(RES_MAX_N / 512 <= RES_SLOTS, "one slot a finalize thread");
 static_assert(RES_OWN + RES_HALO < 65536, "16-bit LDS positions");
-// words of one exchanged sum: 5 entries a slot (resident_put), two words each
-constexpr int RES_RED_WORDS = RES_SLOTS * 5 * 2;
+// words of one exchanged sum: two entries a slot (resident_put), two words each
+constexpr int RES_SLOT_WORDS = 4;
+constexpr int RES_RED_WORDS = RES_SLOTS * RES_SLOT_WORDS;
 
 struct ResArgs {
   int64_t N, S;               // rows; rows between a thread's rows (256 nbx)
@@ -142,7 +143,7 @@ __device__ inline void resident_put(const ResArgs &a, ResLds &L, uint64_t *red, 
   if (a.nblk == 1) {
     L.one[q][slot][e] = v;
   } else {
-    uint64_t *dst = red + (size_t)q * RES_RED_WORDS + (size_t)slot * 4 + 2 * e;
+    uint64_t *dst = red + (size_t)q * RES_RED_WORDS + (size_t)slot * RES_SLOT_WORDS + 2 * e;
     ll_store(dst, dst + 1, v, epoch);
   }
 }
@@ -187,7 +188,7 @@ __device__ inline void resident_put_rows(const ResArgs &a, ResLds &L, uint64_t *
       s = ((wf[0] + wf[1]) + wf[2]) + wf[3];
     } else if (!ll_fetch<1>(
                    red, red + 1, epoch, res_spin<SET>(a.bounds), L.stuck,
-                   [&](int) { return (unsigned)(q * RES_RED_WORDS + slot * 4 + 2); },
+                   [&](int) { return (unsigned)(q * RES_RED_WORDS + slot * RES_SLOT_WORDS + 2); },
                    [&](int, bool, double x) { s = x; })) {
       L.stuck = 1;
     }
@@ -231,7 +232,7 @@ __device__ inline void resident_total(const ResArgs &a, ResLds &L, const uint64_
           red, red + 1, epoch, res_spin<SET>(a.bounds), L.stuck,
           [&](int u) {
             const int q = u % NV, slot = lane + u / NV * 64;
-            return slot < nslot ? (unsigned)(q * RES_RED_WORDS + slot * 4) : RES_NONE;
+            return slot < nslot ? (unsigned)(q * RES_RED_WORDS + slot * RES_SLOT_WORDS) : RES_NONE;
           },
           [&](int u, bool have, double x) { v[u / NV][u % NV] = have ? x : 0.0; });
       if (!ok) L.stuck = 1;
@@ -257,7 +258,7 @@ __device__ inline void resident_total(const ResArgs &a, ResLds &L, const uint64_
       const bool mine = slot < nslot;
       const bool ok = ll_fetch<NV>(
           red, red + 1, epoch, res_spin<SET>(a.bounds), L.stuck,
-          [&](int q) { return mine ? (unsigned)(q * RES_RED_WORDS + slot * 4) : RES_NONE; },
+          [&](int q) { return mine ? (unsigned)(q * RES_RED_WORDS + slot * RES_SLOT_WORDS) : RES_NONE; },
           [&](int q, bool have, double x) { v[q] = have ? x : 0.0; });
       if (!ok) L.stuck = 1;
       // combine_partials adds the slot to a zero
