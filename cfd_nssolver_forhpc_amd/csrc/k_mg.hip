@@ -470,10 +470,12 @@ struct FusedShape {
   int hz, R, TJ, njt, chunk, nci, halo;  // halo: rows beside a tile (0: one tile spans y)
 };
 
-// n / d as the compiler's division does it, split so that the reciprocal of
-// d is shared by the two divisions a cell of a pass makes: the same
-// operations on the same operands while neither needs rescaling (quotients
-// and divisors far from the exponent range's ends)
+// n / d, split so that the reciprocal of d is shared by the two divisions a cell
+// of a pass makes.  FP64: the compiler's own operations on the same operands
+// without its rescaling, so correctly rounded while d, 1 / d and n 2^-53 are
+// normal numbers.  (Past that a grid's cells are shorter than 2^-510 or longer
+// than 2^510, or n is below 2^-969, where the Krylov solver's dot products are
+// zero.)
 __device__ inline double div_recip(double d) {
   double y = __builtin_amdgcn_rcp(d);
   double e = fma(-d, y, 1.0);
@@ -486,18 +488,13 @@ __device__ inline double div_by(double n, double d, double y) {
   const double r = fma(-d, q, n);
   return __builtin_amdgcn_div_fixup(fma(r, y, q), d, n);
 }
-__device__ inline float div_recip(float d) {
-  const float y = __builtin_amdgcn_rcpf(d);
-  const float e = fmaf(-d, y, 1.0f);
-  return fmaf(e, y, y);
-}
-__device__ inline float div_by(float n, float d, float y) {
-  const float q = n * y;
-  const float r = fmaf(-d, q, n);
-  const float q1 = fmaf(r, y, q);
-  const float r1 = fmaf(-d, q1, n);
-  return __builtin_amdgcn_div_fixupf(fmaf(r1, y, q1), d, n);
-}
+// FP32: reciprocal and product in FP64 are off by 2^-51 at most, and a quotient
+// of two floats is at least 2^-49 away from the middle between two floats: the
+// correctly rounded quotient over the whole exponent range.  (Split in FP32 like
+// the other one it lost diagonals past 2^126 and below 2^-126; three timesteps
+// of 512x256x64 43.9 -> 44.2 ms, two of 1024x512x128 280.7 -> 281.7.)
+__device__ inline double div_recip(float d) { return __builtin_amdgcn_div_fixup(div_recip((double)d), (double)d, 1.0); }
+__device__ inline float div_by(float n, float, double y) { return (float)((double)n * y); }
 
 // the column a thread of mg_fused_kernel owns and what it carries
 // SCL: the pass forms the right-hand side r / jp itself (natural order, nz
@@ -513,7 +510,7 @@ template <typename T, int NS>
 struct FusedCol {
   T in[FUSED_RING], bA[FUSED_RING], bB[FUSED_RING];  // other colour before the pass; right-hand sides
   T st[NS][3];                                       // stage results of the last three planes
-  T yA[3], yB[3], dA[3], dB[3];                      // 1 / diagonal and diagonal of both colours
+  double yA[3], yB[3];                               // 1 / diagonal of both colours
   T cym, cyp, czm[2], czp[2];
   double dy, dz[2];
   int side[2];  // LDS position of the k neighbour beside k2, by plane parity
@@ -533,7 +530,6 @@ __global__ void __launch_bounds__(FUSED_THREADS) mg_fused_kernel(MGView L, MGVie
                                                                  const KrylovScalars *ks) {
   if (ks && ks->done) return;
   constexpr int PD = sizeof(T) == 8 || SCL ? 2 : 3;
-  constexpr bool KEEP_D = sizeof(T) == 4;  // FP64 adds the diagonal again instead of holding it
   __shared__ T half[2][NS][FUSED_THREADS];
   __shared__ CoefX<T> cxl[FUSED_CHUNK + 2 * NS];
   __shared__ double dxl[FUSED_CHUNK + 2 * NS];
@@ -630,7 +626,7 @@ __global__ void __launch_bounds__(FUSED_THREADS) mg_fused_kernel(MGView L, MGVie
   for (int m = PD + 2; m < FUSED_RING; ++m) c.in[m] = (T)0;
 #pragma unroll
   for (int q = 0; q < 3; ++q) {
-    c.yA[q] = c.yB[q] = c.dA[q] = c.dB[q] = (T)1;
+    c.yA[q] = c.yB[q] = 1.0;
 #pragma unroll
     for (int s = 0; s < NS; ++s) c.st[s][q] = (T)0;
   }
@@ -682,14 +678,12 @@ __global__ void __launch_bounds__(FUSED_THREADS) mg_fused_kernel(MGView L, MGVie
     if (!SCL) fetch(0);  // SCL: the first stage's neighbours are zero
     const double dx0 = dxl[min(n, ilast)], dx1 = dxl[min(max(n - 1, 0), ilast)];
     double dx2 = 0.0, dx3 = 0.0;
-    if (!KEEP_D) {
+    if (sizeof(T) == 8) {  // div_by's diagonal, added again instead of held
       dx2 = dxl[min(max(n - 2, 0), ilast)];
       if (NS > 3) dx3 = dxl[min(max(n - 3, 0), ilast)];
     }
-    c.dA[u % 3] = (T)(dx0 + c.dy + c.dz[q]);
-    c.yA[u % 3] = div_recip(c.dA[u % 3]);
-    c.dB[(u + 2) % 3] = (T)(dx1 + c.dy + c.dz[q]);
-    c.yB[(u + 2) % 3] = div_recip(c.dB[(u + 2) % 3]);
+    c.yA[u % 3] = div_recip((T)(dx0 + c.dy + c.dz[q]));
+    c.yB[(u + 2) % 3] = div_recip((T)(dx1 + c.dy + c.dz[q]));
 #pragma unroll
     for (int s = 0; s < NS; ++s) {
       if (s + 1 < NS) fetch(s + 1 < NS ? s + 1 : 0);
@@ -700,9 +694,8 @@ __global__ void __launch_bounds__(FUSED_THREADS) mg_fused_kernel(MGView L, MGVie
       const T x0 = s == 0 ? c.in[(u + 1) % 6] : c.st[s > 0 ? s - 1 : 0][r0];
       const T xp = s == 0 ? c.in[(u + 2) % 6] : c.st[s > 0 ? s - 1 : 0][rp];
       const T bv = (s & 1) ? c.bB[(u + 6 - s) % 6] : c.bA[(u + 6 - s) % 6];
-      const T d = KEEP_D ? ((s & 1) ? c.dB[r0] : c.dA[r0])
-                         : (T)((s == 0 ? dx0 : s == 1 ? dx1 : s == 2 ? dx2 : dx3) + c.dy + c.dz[q]);
-      const T y = (s & 1) ? c.yB[r0] : c.yA[r0];
+      const T d = (T)((s == 0 ? dx0 : s == 1 ? dx1 : s == 2 ? dx2 : dx3) + c.dy + c.dz[q]);
+      const double y = (s & 1) ? c.yB[r0] : c.yA[r0];
       T v = (T)0;
       if (!SCL || s > 0) {
         v = fma(cx[s].m, xm, (T)0);
@@ -922,7 +915,8 @@ struct BottomLevel {
 template <typename T>
 struct BottomCell {
   unsigned cn, x, y, z;  // own position | parent's; -x | +x; -y | +y; -z | +z
-  T a[6], d, r, b;       // coefficients, diagonal and its reciprocal, right-hand side
+  T a[6], d, b;          // coefficients, diagonal, right-hand side
+  double r;              // the diagonal's reciprocal
   bool on;
 
   __device__ T off(const T *xl) const {
