@@ -71,7 +71,7 @@ struct MGLevel {
   // by its last post-smoothing half-sweep for the prolongation above it
   double *xn64 = nullptr;
   float *xn32 = nullptr;
-  // a colour-split level's second x: mg_fused_kernel reads one and writes the other
+  // the second x of a level with fused passes: mg_fused_kernel reads one and writes the other
   double *xb64 = nullptr;
   float *xb32 = nullptr;
 };
@@ -1206,6 +1206,9 @@ FusedShape fused_shape(const MGView &v, int ns) {
   return s;
 }
 
+// whether the sweeps of a colour-split level run as fused passes
+bool fused_passes(const MGView &v, int nu) { return nu >= 2 && fused_shape(v, 4).R > 0; }
+
 template <typename T, typename V, int NS, int START, bool PRO, bool OUT>
 void launch_fused(const MGView &v, const MGView &C, const T *b, const T *xin, T *xout, const T *xc, V *out,
                   const KrylovScalars *ks, hipStream_t st) {
@@ -1295,7 +1298,7 @@ int mg_apply(Ctx &c, const V *r, V *out, const KrylovScalars *ks) {
   if (!b0 || !x0) return fail(CFD_ERR_STATE, "multigrid buffers of this precision are not allocated");
   auto X = [&](int l) { return l == 0 ? x0 : lx<T>(M.lv[l]); };
   const MGView &v0 = M.lv[0].v;
-  const bool scaled = split && M.nu >= 2 && v0.nz % 2 == 0 && fused_shape(v0, 4).R > 0 &&
+  const bool scaled = split && v0.nz % 2 == 0 && fused_passes(v0, M.nu) &&
                       reinterpret_cast<uintptr_t>(r) % (2 * sizeof(V)) == 0;
   if (scaled)
     launch_fused_scaled<T, V>(v0, r, c.f[CFD_JP], b0, x0, ks, c.stream);
@@ -1388,7 +1391,7 @@ int mg_apply(Ctx &c, const V *r, V *out, const KrylovScalars *ks) {
   };
   auto smooth = [&](int l, bool pre) {
     const MGView &v = M.lv[l].v;
-    if (l < M.split_levels && M.nu >= 2 && fused_shape(v, 4).R > 0) {
+    if (l < M.split_levels && fused_passes(v, M.nu)) {
       smooth_fused(l, pre);
       return;
     }
@@ -1647,17 +1650,18 @@ int mg_ensure(Ctx &c, bool fp32) {
     const bool sp = (int)l < M.split_levels;
     const size_t n = sp ? (size_t)L.v.nx * L.v.ny * (2 * ((L.v.nz + 1) / 2)) : (size_t)L.v.n;
     const bool nat = sp && l > 0;  // a split level below the finest keeps a natural copy of x
+    const bool second = sp && fused_passes(L.v, M.nu);
     int rc = CFD_OK;
     if (fp32) {
       if (!L.b32 && (rc = mg_alloc(&L.b32, n))) return rc;
       if (!L.x32 && (rc = mg_alloc(&L.x32, n))) return rc;
       if (nat && !L.xn32 && (rc = mg_alloc(&L.xn32, (size_t)L.v.n))) return rc;
-      if (sp && !L.xb32 && (rc = mg_alloc(&L.xb32, n))) return rc;
+      if (second && !L.xb32 && (rc = mg_alloc(&L.xb32, n))) return rc;
     } else {
       if (!L.b64 && (rc = mg_alloc(&L.b64, n))) return rc;
       if (!L.x64 && (rc = mg_alloc(&L.x64, n))) return rc;
       if (nat && !L.xn64 && (rc = mg_alloc(&L.xn64, (size_t)L.v.n))) return rc;
-      if (sp && !L.xb64 && (rc = mg_alloc(&L.xb64, n))) return rc;
+      if (second && !L.xb64 && (rc = mg_alloc(&L.xb64, n))) return rc;
     }
   }
   const size_t N = (size_t)c.g.N;
