@@ -1443,9 +1443,7 @@ int mg_apply(Ctx &c, const V *r, V *out, const KrylovScalars *ks) {
     S.b[l - ls] = lb<T>(M.lv[l]);
   }
   const size_t lds_bytes = bottom_layout(S);
-  if (lds_bytes) {
-    CFD_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(mg_bottom_kernel<T>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)BOTTOM_LDS));
+  if (lds_bytes) {  // at most BOTTOM_LDS, which mg_ensure has asked for
     mg_bottom_kernel<T><<<1, BOTTOM_THREADS, lds_bytes, c.stream>>>(S, ks);
   } else {
     mg_small_kernel<T><<<1, MG_SMALL_THREADS, 0, c.stream>>>(S, ks);
@@ -1502,6 +1500,9 @@ void mg_release(Ctx &c) {
 // builds the hierarchy (once) and the buffers of the requested precision
 int mg_ensure(Ctx &c, bool fp32) {
   if (!c.mg) {
+    for (const void *k : {reinterpret_cast<const void *>(mg_bottom_kernel<double>),
+                          reinterpret_cast<const void *>(mg_bottom_kernel<float>)})
+      CFD_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)BOTTOM_LDS));
     MGState *M = new MGState();
     c.mg = M;
     const int nc[3] = {c.g.nxc, c.g.nyc, c.g.nzc};
