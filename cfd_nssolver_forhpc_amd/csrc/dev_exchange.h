@@ -5,8 +5,11 @@
 // (ll_store / ll_load).  Each word is one relaxed agent-scope atomic, so a
 // reader that finds the number it waits for has the value, with no fence and
 // no flag to read first; an exchange costs one store and one load to the
-// level the XCDs share.  A buffer is rewritten only after a sum that every
-// workgroup contributed to after its reads of the buffer.
+// level the XCDs share.  A buffer is rewritten only when its readers are known
+// to be through: in the BiCGSTAB after a sum that every workgroup contributed to
+// after its reads; in SorPipeLine, whose sweeps end in no sum that is waited for,
+// a colour's values after the neighbours' next ones of the other colour, which
+// they leave after their reads, and a maximum after every workgroup's next one.
 #pragma once
 
 #include <atomic>

@@ -1,13 +1,13 @@
 // dev_resident.h -- BiCGSTAB iterations of a small ELL system in one launch.
 //
 // Below half a million rows an iteration of the launch path (launch_iters)
-// is eight dependent kernels whose work takes a microsecond or two each: at
-// 4096 and at 32768 rows it costs 35 us whatever the size, launch to drain.
-// Here the whole solve is one kernel.  Every thread owns RES_ROWS rows and
-// keeps their matrix entries and their entries of x, r, r0, p, A p, s and
-// A s in registers; a workgroup keeps the entries of the gathered vector it
-// needs (its own rows' and its halo's) in LDS.  What crosses workgroups per
-// iteration is two halos (p and s) and three sums.
+// is five dependent kernels (fold_of) whose work takes a microsecond or two
+// each: at 4096 and at 32768 rows it costs 24 us, launch to drain.  Here the
+// whole solve is one kernel.  Every thread owns RES_ROWS rows and keeps their
+// matrix entries and their entries of r, p, A p, s and A s in registers; a
+// workgroup keeps the entries of the gathered vector it needs (its own rows' and
+// its halo's) in LDS.  What crosses workgroups per iteration is two halos (p and
+// s) and three sums.
 //
 // Values cross workgroups as self-validating words (dev_exchange.h).
 //
@@ -20,10 +20,10 @@
 // waves, the blocks and the finalize kernel's tree in that order.
 //
 // What bounds it is the latency of the five exchanges, about 2 us each, and,
-// past 10^5 rows, the halo words.  Measured on one MI355X, us an iteration,
-// launch path -> here: 512 rows 15.4 -> 4.6 (one workgroup: sums through
-// LDS), 4096 19.2 -> 9.7, 32768 19.3 -> 10.9, 65536 21.0 -> 13.6, 303750
-// 30.6 -> 22.3, 524288 28.5 -> 19.7.  Of the 12 us that 32768 rows took before
+// past 10^5 rows, the halo words.  Measured on one MI355X over whole solves of
+// 2000 iterations, us an iteration, launches -> here: 512 rows 20.0 -> 4.6 (one
+// workgroup: sums through LDS), 4096 23.8 -> 9.7, 32768 24.1 -> 10.6, 65536
+// 25.1 -> 13.6, 303750 31.8 -> 22.8, 524288 29.9 -> 21.0.  Of the 12 us that 32768 rows took before
 // the wave sums were packed, every wave formed the total of up to 128 slots
 // itself and the next p left ahead of the stop test: halos 2.8, the sums'
 // way 5.5, products with their wave sums 1.9, the rest 1.6.

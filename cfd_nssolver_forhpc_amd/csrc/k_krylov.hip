@@ -768,7 +768,7 @@ hipError_t launch_iters(Ctx &c, const OpArgs &a, const Vecs<T> &v, KrylovScalars
 // wait reached its bound.
 // The limit is what the registers of 256 one-workgroup CUs hold (RES_MAX_N,
 // 524288 rows); it is the faster path over that whole range (at the limit
-// 19.7 us an iteration against 28.5, at one workgroup 4.6 against 15.4).
+// 21.0 us an iteration against 29.9, at one workgroup 4.6 against 20.0).
 int solve_resident(Ctx &c, const OpArgs &a, const Vecs<double> &v, KrylovScalars *ks, bool *solved, bool *lost) {
   *solved = *lost = false;
   if ((a.op != CFD_OP_ELL && a.op != OP_ELL_GRID) || a.N > RES_MAX_N) return CFD_OK;

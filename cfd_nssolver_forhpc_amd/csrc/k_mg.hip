@@ -20,9 +20,10 @@
 // so the red-black colouring stays consistent across the seam.  Restriction is the
 // volume-weighted sum of the children's residuals, prolongation adds the
 // parent's correction.  Smoother: red-black Gauss-Seidel, nu sweeps before
-// and after.  Levels of at most MG_SMALL cells run inside one 512-thread
-// workgroup (one launch for the whole bottom of the cycle); the coarsest is
-// solved by its dense inverse or smoothed MG_COARSE_SWEEPS times.
+// and after.  Levels of at most MG_SMALL cells run inside one workgroup (one
+// launch for the whole bottom of the cycle, mg_bottom_kernel; mg_small_kernel
+// where the coarsest level has more cells); the coarsest is solved by its dense
+// inverse or smoothed MG_COARSE_SWEEPS times.
 //
 // The finest level keeps x and b colour-split (ColourSplit), and so does every
 // next level while the level above halves every axis and it is not part of
@@ -30,8 +31,8 @@
 // half-sweeps in one pass over the level (mg_fused_kernel), the first pass
 // after the coarse correction with the prolongation folded in, the last one
 // writing the result; the restriction reads the children as colour pairs.
-// What a pass cannot take (one sweep, the odd sweep of an odd count, lines
-// too long for its tiles) runs as single colour sweeps whose threads walk
+// What a pass cannot take (one sweep, the odd sweep of an odd count, lines of
+// more than 128 cells, whose z its tiles do not split) runs as single colour sweeps whose threads walk
 // MG_PLANES planes and load each other-colour entry once for its three uses.
 // Each does the arithmetic of the generic per-cell functions term for term,
 // so the cycle's result is the same bit for bit in either layout.
@@ -445,14 +446,15 @@ __global__ void __launch_bounds__(256) mg_split_sweep_kernel(MGView L, MGView C,
 // What bounds a pass is latency on the small levels (8-14 us for 4
 // half-sweeps, 4 launches of 3.5-6 us before) and, on the finest, the stages'
 // chain of LDS reads and divisions: four half-sweeps of 512x256x64 take
-// 41-51 us FP64 and 28 us FP32 (4 x 21 and 4 x 15 as single sweeps), at 30 B
+// 40-51 us FP64 and 29-32 us FP32 (4 x 21 and 4 x 15 as single sweeps), at 30 B
 // a cell 6.1 TB/s of FP64 traffic.  With a branch per stage the compiler
 // drained every load before its use and an FP64 pass took 59-68 us.  One
 // workgroup a CU: tiles of 24 rows and 23 planes at that size, each computing
-// 1.5 times its cells, are what 256 CUs leave (two workgroups a CU, with twice
-// the overlap: a cycle of 490 us against 422).  Choosing tiles by waves and
-// steps (fused_shape) instead of the fewest tiles of rows: 396 -> 385 us a
-// cycle there, 159 -> 152 at 256x128x32, 151 -> 140 at 200x104x40.  Three timesteps
+// 32 x 29 instead, 1.7 times its cells (2.05 at 1024x512x128, 3.1 at
+// 256x128x32, 3.5 at 200x104x40, 6 at 128x64x16), are what 256 CUs leave (two
+// workgroups a CU, with twice the overlap: a cycle of 490 us against 422).
+// Choosing tiles by waves and steps (fused_shape) instead of the fewest tiles of rows: 396 -> 386 us a
+// cycle there, 159 -> 152 at 256x128x32, 151 -> 139 at 200x104x40.  Three timesteps
 // there went from 73.9 to 57.2 ms (FP64; mixed 65.5 to 50.8), the 256x128x32
 // adjoint from 110 to 83 ms.
 //
@@ -491,8 +493,8 @@ __device__ inline double div_by(double n, double d, double y) {
 // FP32: reciprocal and product in FP64 are off by 2^-51 at most, and a quotient
 // of two floats is at least 2^-49 away from the middle between two floats: the
 // correctly rounded quotient over the whole exponent range.  (Split in FP32 like
-// the other one it lost diagonals past 2^126 and below 2^-126; three timesteps
-// of 512x256x64 43.9 -> 44.2 ms, two of 1024x512x128 280.7 -> 281.7.)
+// the other one it lost diagonals past 2^126 and below 2^-126, with a cycle of
+// 270 us at 512x256x64 for 278 now; three timesteps there 43.3 -> 43.8 ms.)
 __device__ inline double div_recip(float d) { return __builtin_amdgcn_div_fixup(div_recip((double)d), (double)d, 1.0); }
 __device__ inline float div_by(float n, float, double y) { return (float)((double)n * y); }
 
