@@ -152,7 +152,7 @@ def test_one_bound_for_a_workgroup(require_gpu):
         sim.bicgstab(tol=0.0, maxit=10)
         t = time.perf_counter() - t
         assert sim.one_launch_counters() == (0, 1, 1)
-    assert t < 0.11
+    assert t < 0.15  # three bounds, one for each sum of the iteration, are 165 ms
 
 
 @pytest.mark.parametrize("bounds", [dict(wait=1), dict(wait=512, wait_first=1)])
